@@ -1,4 +1,4 @@
-// hipBLASLt plans for the layer's row-major GEMMs (see blas.hpp).
+// The layer's row-major GEMMs: split products and hipBLASLt plans (see blas.hpp).
 //
 // Row-major C = op(A) op(B) is column-major C^T = op(B)^T op(A)^T, so the
 // library's first operand is B's memory and its second is A's; a row-major
@@ -24,6 +24,22 @@ constexpr int kCandidates = 32;  // heuristic results timed per shape
 // that an algorithm that only wins on L2-resident weights is not picked.
 constexpr int64_t kColdTimingMaxM = 256;
 constexpr size_t kFlushBytes = size_t(64) << 20;
+
+// Whether a product gains more from the f16 matrix cores (about 400 against
+// hipBLASLt's 145 TFLOP/s of f32) than splitting its operands costs.  Measured,
+// splitting rows: 11 us up to 1024 x 2048, 26 us at 8192 x 2048, 107 us at
+// 32768 x 2048 (8 bytes an element, 5 TB/s); splitting columns (two reads of
+// the operand): 38 us at 8192 x 2048, 210 us at 8192 x 10496.  Both sides near
+// the line, f32 against split + product: 148 x 10496 x 2048 68 and 66 us,
+// 8192 x 2048 x 128 50 and 43 us; 148 x 2048 x 2048 23 and 39 us,
+// 8192 x 128 x 2048 41 and 61 us and 1024 x 1408 x 256 22 and 28 us stay.
+// Below 128 rows a product is bound by reading its weights, not by the cores.
+bool split_pays(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, bool b_kept) {
+    if (M < 128 || N < 128 || Kd < 64) return false;
+    const double gain = 2.0 * (double)M * (double)N * (double)Kd * (1 / 145e12 - 1 / 400e12);
+    const auto cost = [](double n, bool trans) { return trans ? 20e-6 + n * 12 / 4.5e12 : 14e-6 + n * 8 / 4.5e12; };
+    return gain > cost((double)M * (double)Kd, ta) + (b_kept ? 0.0 : cost((double)N * (double)Kd, !tb));
+}
 }
 
 gdn2_status Gemm::ensure_ws(size_t bytes) {
@@ -57,6 +73,9 @@ void Gemm::destroy() {
     if (ws_) (void)hipFree(ws_);
     ws_ = nullptr;
     ws_bytes_ = 0;
+    if (sws_) (void)hipFree(sws_);
+    sws_ = nullptr;
+    sws_bytes_ = 0;
     if (lt_) hipblasLtDestroy(lt_);
     lt_ = nullptr;
     if (rb_) rocblas_destroy_handle(rb_);
@@ -167,12 +186,80 @@ gdn2_status Gemm::plan(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const
     return GDN2_OK;
 }
 
+// Runs the product on the f16 matrix cores if that pays and its memory is
+// there; false: not run, take the library's product.  Memory grows only while
+// the stream is not being captured; a failed allocation is no error.
+bool Gemm::run_split(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const float *A, int64_t lda, const float *B,
+                     int64_t ldb, float *C, int64_t ldc, float beta, hipStream_t s, SplitWeight *w, gdn2_status *st) {
+    if (!split_pays(ta, tb, M, N, Kd, w != nullptr)) return false;
+    SplitGemmParams p{};
+    p.A = A; p.B = B; p.C = C; p.lda = lda; p.ldb = ldb; p.ldc = ldc; p.M = M; p.N = N; p.Kd = Kd;
+    p.beta = beta; p.ta = ta; p.tb = tb;
+    p.vec_c = reinterpret_cast<uintptr_t>(C) % 16 == 0 && ldc % 4 == 0;
+    const size_t part = (plan_split_gemm(&p) + 255) & ~(size_t)255;
+    const size_t fa = split_frag_bytes(M, Kd), sa = split_stat_bytes(M);
+    const size_t fb = split_frag_bytes(N, Kd), sb = split_stat_bytes(N);
+    const size_t need = part + fa + sa + (w ? 0 : fb + sb);
+    const auto capturing = [&] {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+    };
+    const auto grow = [](void **ptr, size_t bytes) {
+        if (hipMalloc(ptr, bytes) == hipSuccess) return true;
+        *ptr = nullptr;
+        (void)hipGetLastError();
+        return false;
+    };
+    if (need > sws_bytes_) {
+        if (capturing()) return false;
+        void *bigger = nullptr;
+        if (!grow(&bigger, need)) return false;
+        if (sws_ && (hipDeviceSynchronize() != hipSuccess || hipFree(sws_) != hipSuccess)) (void)hipGetLastError();
+        sws_ = bigger;
+        sws_bytes_ = need;
+    }
+    const auto check = [&](hipError_t e) {
+        if (e != hipSuccess) *st = fail(GDN2_EHIP, std::string("split product: ") + hipGetErrorString(e));
+        return e == hipSuccess;
+    };
+    *st = GDN2_OK;
+    if (w && !w->frags) {
+        if (capturing()) return false;
+        void *buf = nullptr;
+        if (!grow(&buf, fb + sb)) return false;
+        w->frags = buf;
+        w->stat = reinterpret_cast<SplitStat *>(static_cast<char *>(buf) + fb);
+        if (!check(w->refresh(s))) return true;
+    }
+    char *base = static_cast<char *>(sws_);
+    p.part = reinterpret_cast<float *>(base);
+    void *fra = base + part;
+    SplitStat *sta = reinterpret_cast<SplitStat *>(base + part + fa);
+    if (!check(launch_split(A, lda, ta, M, Kd, fra, sta, s))) return true;
+    p.fa = fra;
+    p.sa = sta;
+    if (w) {
+        p.fb = w->frags;
+        p.sb = w->stat;
+    } else {
+        void *frb = base + part + fa + sa;
+        SplitStat *stb = reinterpret_cast<SplitStat *>(base + part + fa + sa + fb);
+        if (!check(launch_split(B, ldb, !tb, N, Kd, frb, stb, s))) return true;
+        p.fb = frb;
+        p.sb = stb;
+    }
+    (void)check(launch_split_gemm(p, s));
+    return true;
+}
+
 gdn2_status Gemm::run(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const float *A, int64_t lda, const float *B,
-                      int64_t ldb, float *C, int64_t ldc, float beta, hipStream_t s) {
+                      int64_t ldb, float *C, int64_t ldc, float beta, hipStream_t s, SplitWeight *w) {
     if (M == 0 || N == 0) return GDN2_OK;
+    gdn2_status st = GDN2_OK;
+    if (run_split(ta, tb, M, N, Kd, A, lda, B, ldb, C, ldc, beta, s, w, &st)) return st;
     const float alpha = 1.0f;
     const Plan *p = nullptr;
-    gdn2_status st = plan(ta, tb, M, N, Kd, A, lda, B, ldb, ldc, s, &p);
+    st = plan(ta, tb, M, N, Kd, A, lda, B, ldb, ldc, s, &p);
     if (st != GDN2_OK) return st;
     if (p->ok) {
         if ((st = ensure_ws(p->ws)) != GDN2_OK) return st;

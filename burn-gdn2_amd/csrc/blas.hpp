@@ -1,10 +1,12 @@
-// Row-major f32 GEMMs of the layer: C[M, N] = op(A) op(B) (+ beta C) through
-// hipBLASLt, with one plan (descriptors + algorithm) cached per shape.  The
-// algorithm is the fastest of the heuristic's first 32 candidates, timed on
-// the first call's operands into a scratch output (when the stream is not
-// being captured; otherwise the heuristic's first), with L2 flushed before
-// each timed run for shapes of at most 256 rows.  rocBLAS runs the shapes
-// hipBLASLt has no algorithm for.
+// Row-major f32 GEMMs of the layer: C[M, N] = op(A) op(B) (+ beta C).
+// Products large enough to pay for splitting their operands run on the f16
+// matrix cores (split_gemm.hpp); the others run through hipBLASLt, with one
+// plan (descriptors + algorithm) cached per shape.  The algorithm is the
+// fastest of the heuristic's first 32 candidates, timed on the first call's
+// operands into a scratch output (when the stream is not being captured;
+// otherwise the heuristic's first), with L2 flushed before each timed run for
+// shapes of at most 256 rows.  rocBLAS runs the shapes hipBLASLt has no
+// algorithm for.
 #pragma once
 
 #include <hipblaslt/hipblaslt.h>
@@ -14,8 +16,28 @@
 #include <vector>
 
 #include "common.hpp"
+#include "split_gemm.hpp"
 
 namespace gdn2 {
+
+// A weight matrix as the second operand of split products, split once: the
+// owner calls refresh() whenever the weight's values change, so that captured
+// graphs, which read the split copy, keep seeing the current values.
+struct SplitWeight {
+    const float *src = nullptr; // [rows of the stored matrix, cols], row stride ld
+    int64_t ld = 0, rows = 0, Kd = 0; // rows of the operand (N of the product) and its contraction
+    bool trans = false;         // the operand's rows are src's columns
+    void *frags = nullptr;      // allocated by the first product that uses it
+    SplitStat *stat = nullptr;
+    hipError_t refresh(hipStream_t s) const {
+        return frags ? launch_split(src, ld, trans, rows, Kd, frags, stat, s) : hipSuccess;
+    }
+    void destroy() {
+        if (frags) (void)hipFree(frags);
+        frags = nullptr;
+        stat = nullptr;
+    }
+};
 
 class Gemm {
   public:
@@ -23,10 +45,13 @@ class Gemm {
     void destroy();
     // op(A) [M, Kd]: A stored [M, Kd] (ta = false) or [Kd, M] (ta = true), row stride lda;
     // op(B) [Kd, N]: B stored [Kd, N] (tb = false) or [N, Kd] (tb = true), row stride ldb.
+    // w: op(B) as a weight that may keep its split copy (its src and ld are B and ldb).
     gdn2_status run(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const float *A, int64_t lda, const float *B,
-                    int64_t ldb, float *C, int64_t ldc, float beta, hipStream_t s);
+                    int64_t ldb, float *C, int64_t ldc, float beta, hipStream_t s, SplitWeight *w = nullptr);
 
   private:
+    bool run_split(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const float *A, int64_t lda, const float *B,
+                   int64_t ldb, float *C, int64_t ldc, float beta, hipStream_t s, SplitWeight *w, gdn2_status *st);
     struct Plan {
         bool ta, tb;
         int64_t M, N, Kd, lda, ldb, ldc;
@@ -44,6 +69,8 @@ class Gemm {
     std::vector<Plan> plans_;
     void *ws_ = nullptr;
     size_t ws_bytes_ = 0;
+    void *sws_ = nullptr; // split operands and partial sums of one product
+    size_t sws_bytes_ = 0;
 };
 
 }  // namespace gdn2

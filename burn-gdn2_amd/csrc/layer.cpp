@@ -171,6 +171,9 @@ struct gdn2_layer {
     int64_t ld_in = 0, off_q = 0, off_k = 0, off_b = 0, off_v = 0, off_w = 0, off_f0 = 0, off_g0 = 0;
     float *w_in = nullptr;
     float *p[P_COUNT] = {};  // standalone parameters (null for those inside w_in)
+    // Split copies of the Linear weights (blas.hpp), allocated by the first
+    // product large enough to use them: W of y = x W, and W^T of dx = dy W^T.
+    SplitWeight sw_in, sw_in_t, sw_o, sw_o_t, sw_f1, sw_g1;
     void *ws = nullptr;
     size_t ws_bytes = 0;
     void *bws = nullptr;  // backward workspace, grown on demand
@@ -297,7 +300,7 @@ gdn2_status input_gemms(gdn2_layer &L, const float *x, int64_t M, const Work &wk
                         bool with_bias = false) {
     const Dims &d = L.d;
     gdn2_status st;
-    if ((st = L.mm.run(false, false, M, L.ld_in, d.D, x, d.D, L.w_in, L.ld_in, wk.Y, L.ld_in, 0.0f, s)) != GDN2_OK)
+    if ((st = L.mm.run(false, false, M, L.ld_in, d.D, x, d.D, L.w_in, L.ld_in, wk.Y, L.ld_in, 0.0f, s, &L.sw_in)) != GDN2_OK)
         return st;
     if (lowrank_up_supported((int)d.V, M, wk.Y, L.ld_in, L.off_f0, L.off_g0)) { // a few rows (decode): one small launch for both
         LowRankParams lp{};
@@ -308,12 +311,12 @@ gdn2_status input_gemms(gdn2_layer &L, const float *x, int64_t M, const Work &wk
         GDN2_HIP_CHECK(launch_lowrank_up(lp, s));
         return GDN2_OK;
     }
-    if ((st = L.mm.run(false, false, M, d.kd, d.V, wk.Y + L.off_f0, L.ld_in, L.p[P_F1], d.kd, wk.F, d.kd, 0.0f, s)) !=
-        GDN2_OK)
+    if ((st = L.mm.run(false, false, M, d.kd, d.V, wk.Y + L.off_f0, L.ld_in, L.p[P_F1], d.kd, wk.F, d.kd, 0.0f, s,
+                       &L.sw_f1)) != GDN2_OK)
         return st;
     if (with_bias) GDN2_HIP_CHECK(launch_fill_rows(wk.G, d.vd, L.p[P_G1_BIAS], M, d.vd, s));
     return L.mm.run(false, false, M, d.vd, d.V, wk.Y + L.off_g0, L.ld_in, L.p[P_G1], d.vd, wk.G, d.vd,
-                    with_bias ? 1.0f : 0.0f, s);
+                    with_bias ? 1.0f : 0.0f, s, &L.sw_g1);
 }
 
 gdn2_status project_epilogue(gdn2_layer &L, int64_t B, int64_t T, const float *const conv_in[3], const Work &wk,
@@ -377,7 +380,7 @@ gdn2_status output_side(gdn2_layer &L, int64_t M, bool norm, const Work &wk, flo
         GDN2_HIP_CHECK(launch_rmsnorm_gate(y, d.vd, wk.O, d.vd, wk.G, d.vd, L.p[P_G1_BIAS], L.p[P_O_NORM], M, (int)d.HV,
                                            (int)d.V,
                                            (float)L.cfg.norm_eps, s));
-    return L.mm.run(false, false, M, d.D, d.vd, y, d.vd, L.p[P_O], d.D, out, d.D, 0.0f, s);
+    return L.mm.run(false, false, M, d.D, d.vd, y, d.vd, L.p[P_O], d.D, out, d.D, 0.0f, s, &L.sw_o);
 }
 
 gdn2_status check_layer_call(const gdn2_layer *L, const float *x, int64_t B, int64_t T, const void *out,
@@ -496,6 +499,7 @@ extern "C" void gdn2_layer_destroy(gdn2_layer *L) {
     (void)hipSetDevice(L->device);
     (void)hipDeviceSynchronize();
     L->mm.destroy();
+    for (SplitWeight *w : {&L->sw_in, &L->sw_in_t, &L->sw_o, &L->sw_o_t, &L->sw_f1, &L->sw_g1}) w->destroy();
     (void)hipFree(L->w_in);
     for (float *p : L->p) (void)hipFree(p);
     (void)hipFree(L->ws);
@@ -520,6 +524,15 @@ extern "C" gdn2_status gdn2_layer_set_param(gdn2_layer *L, const char *name, con
                                    sizeof(float) * cols, rows, hipMemcpyHostToDevice));
     else
         GDN2_HIP_CHECK(hipMemcpy(L->p[id], host, sizeof(float) * n, hipMemcpyHostToDevice));
+    // the split copies that products (and captured graphs) already read
+    const float *changed = off >= 0 ? L->w_in : L->p[id];
+    bool any = false;
+    for (SplitWeight *w : {&L->sw_in, &L->sw_in_t, &L->sw_o, &L->sw_o_t, &L->sw_f1, &L->sw_g1})
+        if (w->frags && w->src == changed) {
+            GDN2_HIP_CHECK(w->refresh(nullptr));
+            any = true;
+        }
+    if (any) GDN2_HIP_CHECK(hipStreamSynchronize(nullptr));
     return GDN2_OK;
 }
 
@@ -587,6 +600,15 @@ extern "C" gdn2_status gdn2_layer_create(const gdn2_config *c, uint64_t seed, gd
         delete[] host;
         if (st != GDN2_OK) return cleanup(st);
     }
+    auto weight = [](SplitWeight *w, const float *src, int64_t ld, int64_t rows, int64_t Kd, bool trans) {
+        w->src = src; w->ld = ld; w->rows = rows; w->Kd = Kd; w->trans = trans;
+    };
+    weight(&L->sw_in, L->w_in, L->ld_in, L->ld_in, d.D, true);
+    weight(&L->sw_in_t, L->w_in, L->ld_in, d.D, L->ld_in, false);
+    weight(&L->sw_o, L->p[P_O], d.D, d.D, d.vd, true);
+    weight(&L->sw_o_t, L->p[P_O], d.D, d.vd, d.D, false);
+    weight(&L->sw_f1, L->p[P_F1], d.kd, d.kd, d.V, true);
+    weight(&L->sw_g1, L->p[P_G1], d.vd, d.vd, d.V, true);
     *out = L;
     return GDN2_OK;
 }
@@ -1373,7 +1395,7 @@ extern "C" gdn2_status gdn2_layer_backward_f32(gdn2_layer *L, const float *x, in
     }
 
     // o_proj and the gated RMSNorm
-    if ((st = L->mm.run(false, true, M, d.vd, d.D, d_out, d.D, L->p[P_O], d.D, bw.dy, d.vd, 0.0f, s)) != GDN2_OK)
+    if ((st = L->mm.run(false, true, M, d.vd, d.D, d_out, d.D, L->p[P_O], d.D, bw.dy, d.vd, 0.0f, s, &L->sw_o_t)) != GDN2_OK)
         return st;
     NormBwdParams np{};
     np.O = fw.O; np.G = fw.G; np.weight = L->p[P_O_NORM]; np.gate_bias = L->p[P_G1_BIAS]; np.HV = (int)d.HV;
@@ -1497,7 +1519,7 @@ extern "C" gdn2_status gdn2_layer_backward_f32(gdn2_layer *L, const float *x, in
         GDN2_OK)
         return st;
     if (dx && (st = L->mm.run(false, true, M, d.D, L->ld_in, bw.dY, L->ld_in, L->w_in, L->ld_in, dx, d.D,
-                           0.0f, s)) != GDN2_OK)
+                           0.0f, s, &L->sw_in_t)) != GDN2_OK)
         return st;
     if (d_state_in) d_state_in->some = true;
     return GDN2_OK;

@@ -1,0 +1,41 @@
+// f32 matrix products on the f16 matrix cores (split_gemm.hip).
+#pragma once
+
+#include <algorithm>
+
+#include "common.hpp"
+
+namespace gdn2 {
+
+struct SplitStat {
+    unsigned amax, small, nonzero;
+};
+
+struct SplitGemmParams {
+    // C [M, N] (+)= op(A) [M, Kd] op(B) [Kd, N], row-major; ta: A is stored [Kd, M], tb: B is stored [N, Kd]
+    const float *A, *B;
+    float *C;
+    int64_t lda, ldb, ldc, M, N, Kd;
+    float beta;
+    bool ta, tb, vec_c;    // vec_c: rows of C are 16-byte aligned
+    const void *fa, *fb;   // the split operands: rows of op(A), columns of op(B)
+    const SplitStat *sa, *sb;
+    float *part;           // partial sums of the tiles cut along the contraction
+    // plan_split_gemm:
+    int tile, KT;
+    unsigned ntm, ntn, split, whole;
+    int64_t rta, rtb;
+};
+
+// Bytes of a split operand of `rows` rows of Kd elements, and of its row records.
+size_t split_frag_bytes(int64_t rows, int64_t Kd);
+size_t split_stat_bytes(int64_t rows);
+// Splits an operand: rows of src when !trans (its contiguous dimension is the
+// contraction), columns of src when trans.
+hipError_t launch_split(const float *src, int64_t ld, bool trans, int64_t rows, int64_t Kd, void *frags, SplitStat *stat,
+                        hipStream_t s);
+// Fills the plan of p from M, N, Kd; returns the bytes of `part`.
+size_t plan_split_gemm(SplitGemmParams *p);
+hipError_t launch_split_gemm(const SplitGemmParams &p, hipStream_t s);
+
+}  // namespace gdn2
