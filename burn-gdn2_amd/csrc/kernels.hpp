@@ -182,6 +182,8 @@ hipError_t launch_conv_cache(const ConvCacheParams &p, hipStream_t s);
 hipError_t launch_rmsnorm_gate(float *out, int64_t ld_out, const float *x, int64_t ld_x, const float *gate,
                                int64_t ld_gate, const float *gate_bias, const float *weight, int64_t M, int HV, int V,
                                float eps, hipStream_t s);
+hipError_t launch_copy_rows(float *dst, int64_t ldd, const float *src, int64_t lds, int64_t rows, int64_t cols,
+                            hipStream_t s);
 hipError_t launch_fill_rows(float *y, int64_t ld, const float *row, int64_t M, int64_t N, hipStream_t s);
 
 // The reference's GVA layout of the key-side operands (src/module.rs:456-468:

@@ -18,6 +18,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -161,6 +162,91 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 }  // namespace
 
+namespace {
+
+// Synchronous copies between a strided device matrix and contiguous host
+// memory, through two pinned buffers: a kernel moves a block of rows over the
+// bus while the host copies the block before it.  (hipMemcpy2D moves a strided
+// matrix row by row, 7 us each: 15 ms for a 2048 x 2048 block of W_in, whose
+// rows are ld_in apart, against 0.4 ms; hipMemcpy of 16 MB took 0.93 ms.)
+// Bounded by its two buffers, allocated by the first copy and freed with the
+// layer; locked, since several threads may read gradients of one layer.
+struct HostStage {
+    static constexpr size_t kBytes = size_t(4) << 20;
+    std::mutex lock;
+    float *buf[2] = {};
+    hipEvent_t ev[2] = {};
+
+    void destroy() {
+        for (int i = 0; i < 2; ++i) {
+            if (ev[i]) (void)hipEventDestroy(ev[i]);
+            if (buf[i]) (void)hipHostFree(buf[i]);
+            ev[i] = nullptr;
+            buf[i] = nullptr;
+        }
+    }
+    bool ensure() {
+        if (buf[1] && ev[1]) return true;
+        bool ok = true;
+        for (int i = 0; i < 2 && ok; ++i)
+            ok = hipHostMalloc(reinterpret_cast<void **>(&buf[i]), kBytes, hipHostMallocDefault) == hipSuccess &&
+                 hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) == hipSuccess;
+        if (!ok) {
+            destroy();
+            (void)hipGetLastError();
+        }
+        return ok;
+    }
+
+    // rows x cols of dev (row stride ld), on the current device
+    hipError_t copy(float *dev, int64_t ld, float *host, int64_t rows, int64_t cols, bool to_host) {
+        std::lock_guard<std::mutex> g(lock);
+        const size_t row = sizeof(float) * (size_t)cols;
+        if (rows == 0 || cols == 0) return hipSuccess;
+        if (row > kBytes || !ensure())
+            return to_host ? hipMemcpy2D(host, row, dev, sizeof(float) * ld, row, rows, hipMemcpyDeviceToHost)
+                           : hipMemcpy2D(dev, sizeof(float) * ld, host, row, row, rows, hipMemcpyHostToDevice);
+        const int64_t per = (int64_t)(kBytes / row), n = (rows + per - 1) / per;
+        const auto count = [&](int64_t i) { return std::min(per, rows - i * per); };
+        const auto move = [&](int64_t i) { // block i between its buffer and the device
+            float *d = dev + i * per * ld, *b = buf[i & 1];
+            hipError_t e = to_host ? launch_copy_rows(b, cols, d, ld, count(i), cols, nullptr)
+                                   : launch_copy_rows(d, ld, b, cols, count(i), cols, nullptr);
+            return e != hipSuccess ? e : hipEventRecord(ev[i & 1], nullptr);
+        };
+        hipError_t e = hipSuccess;
+        if (to_host) {
+            for (int64_t i = 0; i < std::min<int64_t>(2, n) && e == hipSuccess; ++i) e = move(i);
+            for (int64_t i = 0; i < n && e == hipSuccess; ++i) {
+                if ((e = hipEventSynchronize(ev[i & 1])) != hipSuccess) break;
+                std::memcpy(host + i * per * cols, buf[i & 1], row * (size_t)count(i));
+                if (i + 2 < n) e = move(i + 2);
+            }
+        } else {
+            for (int64_t i = 0; i < n && e == hipSuccess; ++i) {
+                if (i >= 2 && (e = hipEventSynchronize(ev[i & 1])) != hipSuccess) break;
+                std::memcpy(buf[i & 1], host + i * per * cols, row * (size_t)count(i));
+                e = move(i);
+            }
+        }
+        const hipError_t f = hipStreamSynchronize(nullptr); // nothing reads or writes the buffers after the call
+        return e != hipSuccess ? e : f;
+    }
+};
+
+// Makes a device current for a scope.
+struct OnDevice {
+    int prev = -1;
+    explicit OnDevice(int device) {
+        if (hipGetDevice(&prev) != hipSuccess || prev == device || hipSetDevice(device) != hipSuccess) prev = -1;
+    }
+    ~OnDevice() {
+        if (prev >= 0) (void)hipSetDevice(prev);
+    }
+};
+
+}  // namespace
+
 struct gdn2_layer {
     gdn2_config cfg;
     Dims d;
@@ -178,6 +264,7 @@ struct gdn2_layer {
     size_t ws_bytes = 0;
     void *bws = nullptr;  // backward workspace, grown on demand
     size_t bws_bytes = 0;
+    mutable HostStage stage; // pinned buffers of the parameter and gradient copies
 
     int64_t col_offset(int id) const {
         switch (id) {
@@ -504,6 +591,7 @@ extern "C" void gdn2_layer_destroy(gdn2_layer *L) {
     for (float *p : L->p) (void)hipFree(p);
     (void)hipFree(L->ws);
     (void)hipFree(L->bws);
+    L->stage.destroy();
     if (prev >= 0) (void)hipSetDevice(prev);
     delete L;
 }
@@ -519,11 +607,9 @@ extern "C" gdn2_status gdn2_layer_set_param(gdn2_layer *L, const char *name, con
         return fail(GDN2_EINVAL, std::string("gdn2_layer_set_param: ") + name + " has " + std::to_string(n) +
                                      " elements, got " + std::to_string(numel));
     const int64_t off = L->col_offset(id);
-    if (off >= 0)
-        GDN2_HIP_CHECK(hipMemcpy2D(L->w_in + off, sizeof(float) * L->ld_in, host, sizeof(float) * cols,
-                                   sizeof(float) * cols, rows, hipMemcpyHostToDevice));
-    else
-        GDN2_HIP_CHECK(hipMemcpy(L->p[id], host, sizeof(float) * n, hipMemcpyHostToDevice));
+    const OnDevice on(L->device);
+    GDN2_HIP_CHECK(off >= 0 ? L->stage.copy(L->w_in + off, L->ld_in, const_cast<float *>(host), rows, cols, false)
+                            : L->stage.copy(L->p[id], cols, const_cast<float *>(host), rows, cols, false));
     // the split copies that products (and captured graphs) already read
     const float *changed = off >= 0 ? L->w_in : L->p[id];
     bool any = false;
@@ -547,11 +633,9 @@ extern "C" gdn2_status gdn2_layer_get_param(const gdn2_layer *L, const char *nam
         return fail(GDN2_EINVAL, std::string("gdn2_layer_get_param: ") + name + " has " + std::to_string(n) +
                                      " elements, got " + std::to_string(numel));
     const int64_t off = L->col_offset(id);
-    if (off >= 0)
-        GDN2_HIP_CHECK(hipMemcpy2D(host, sizeof(float) * cols, L->w_in + off, sizeof(float) * L->ld_in,
-                                   sizeof(float) * cols, rows, hipMemcpyDeviceToHost));
-    else
-        GDN2_HIP_CHECK(hipMemcpy(host, L->p[id], sizeof(float) * n, hipMemcpyDeviceToHost));
+    const OnDevice on(L->device);
+    GDN2_HIP_CHECK(off >= 0 ? L->stage.copy(L->w_in + off, L->ld_in, host, rows, cols, true)
+                            : L->stage.copy(L->p[id], cols, host, rows, cols, true));
     return GDN2_OK;
 }
 
@@ -1303,11 +1387,9 @@ extern "C" gdn2_status gdn2_layer_grads_get(const gdn2_layer_grads *G, const cha
                                      " elements, got " + std::to_string(numel));
     GDN2_HIP_CHECK(hipDeviceSynchronize());
     const int64_t off = L->col_offset(id);
-    if (off >= 0)
-        GDN2_HIP_CHECK(hipMemcpy2D(host, sizeof(float) * cols, G->g_in + off, sizeof(float) * L->ld_in,
-                                   sizeof(float) * cols, rows, hipMemcpyDeviceToHost));
-    else
-        GDN2_HIP_CHECK(hipMemcpy(host, G->p[id], sizeof(float) * n, hipMemcpyDeviceToHost));
+    const OnDevice on(L->device);
+    GDN2_HIP_CHECK(off >= 0 ? L->stage.copy(G->g_in + off, L->ld_in, host, rows, cols, true)
+                            : L->stage.copy(G->p[id], cols, host, rows, cols, true));
     return GDN2_OK;
 }
 

@@ -3,6 +3,8 @@
 // project() returns them, so that each chunk of a head is one contiguous
 // block), the conv-cache update, the gated RMSNorm and a row fill for Linear
 // biases.
+#include <algorithm>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -368,6 +370,20 @@ __global__ __launch_bounds__(256) void fill_rows_kernel(float *y, int64_t ld, co
     }
 }
 
+// Rows of one strided matrix into another; one of the two is pinned host
+// memory, which the kernel reads or writes over the bus.  vec: columns in
+// groups of four, both sides 16-byte aligned.
+__global__ __launch_bounds__(256) void copy_rows_kernel(float *__restrict__ dst, int64_t ldd, const float *__restrict__ src,
+                                                        int64_t lds, int64_t rows, int64_t cols, bool vec) {
+    const int64_t n = vec ? cols / 4 : cols, step = (int64_t)gridDim.x * 256;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < rows * n; i += step) {
+        const int64_t r = i / n, c = i % n;
+        if (vec)
+            *reinterpret_cast<floatx4 *>(dst + r * ldd + 4 * c) = *reinterpret_cast<const floatx4 *>(src + r * lds + 4 * c);
+        else
+            dst[r * ldd + c] = src[r * lds + c];
+    }
+}
 
 // ---------------------------------------------------------------------------
 // Backward (the adjoints of the kernels above)
@@ -705,6 +721,16 @@ hipError_t launch_lowrank_up(const LowRankParams &p, hipStream_t s) {
 hipError_t launch_cache_sweep(const float *buf, int64_t n, float *sink, hipStream_t s) {
     if (n < 4) return hipSuccess;
     hipLaunchKernelGGL(cache_sweep_kernel, dim3(2048), dim3(256), 0, s, buf, n / 4, sink);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_rows(float *dst, int64_t ldd, const float *src, int64_t lds, int64_t rows, int64_t cols,
+                            hipStream_t s) {
+    if (rows * cols == 0) return hipSuccess;
+    const auto aligned = [](const float *p, int64_t ld) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0; };
+    const bool vec = cols % 4 == 0 && aligned(dst, ldd) && aligned(src, lds);
+    hipLaunchKernelGGL(copy_rows_kernel, dim3(std::min(1024, grid_for(vec ? rows * cols / 4 : rows * cols))), dim3(256), 0,
+                       s, dst, ldd, src, lds, rows, cols, vec);
     return hipGetLastError();
 }
 
