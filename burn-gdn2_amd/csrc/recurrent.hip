@@ -5,11 +5,9 @@
 // src/kernel/fused_recurrent_cube.rs:14-57 (decode step); the fused decode
 // adds src/short_conv.rs:22-65, src/module.rs:417-472 and :501-517 around it.
 //
-// Memory plan.  One workgroup (256 lanes) owns the state slice
-// S[b, hv, :, v0 : v0 + VS].  Lane t holds the 4 contiguous columns
-// 4 * (t % (VS/4)) of rows r = t / (VS/4) + i * RPP in registers (float4),
-// so S is read from HBM exactly once and written exactly once per launch,
-// with 16-byte coalesced accesses, however many tokens the launch covers.
+// Memory plan.  S stays in registers for the whole launch, so that it is read
+// from HBM exactly once and written exactly once however many tokens the
+// launch covers.
 // Both K-reductions of a token (the erase term (b*k)^T S' and the read-out
 // q^T S') come from the same register pass, using
 //   o = scale * (S'^T q + v_new * (k . q)),   S' = diag(exp g) S,
@@ -37,101 +35,170 @@ __device__ __forceinline__ float block_sum256(float v, float *red) {
 }
 
 // ---------------------------------------------------------------------------
-// Register-resident scan.  K rows x VS columns per workgroup of 256 lanes.
+// Register-resident scan: each wave owns all K rows of 16 value columns for
+// the whole launch, so that a token needs no exchange between waves.  Lane
+// (rg = l % 8, cg = l / 8) holds columns 2 cg, 2 cg + 1 of the rows
+// 32 j + 4 rg + i; a K-reduction is a chain in the lane and three DPP steps
+// over rg.  The workgroup's NW waves share what does not depend on the
+// column: e^g, e^g b k, e^g q and k of eight tokens at a time, formed once into
+// LDS (and k . q), while the next eight tokens' operands are on their way to
+// registers; one barrier per eight tokens.  A token is bound by the four
+// multiply-adds per state element (150 instructions a wave at K = 128); two
+// columns a lane halve the LDS reads per multiply-add, which bound it with
+// one.  Measured at K = V = 128 and 16 heads (before: three barriers a token
+// and K-reductions across the workgroup's waves): 4 sequences of 37 tokens 25
+// us (54), 32 of 48 tokens 75 (116), 1 of 2048 tokens 1066 (3344).
 // ---------------------------------------------------------------------------
-template <int K, int VS>
-__global__ __launch_bounds__(256) void scan_kernel(ScanParams p) {
-    constexpr int TPR = VS / 4;    // lanes per state row
-    constexpr int RPP = 256 / TPR; // rows covered by one pass of the workgroup
-    constexpr int NP = K / RPP;    // float4 registers of S per lane
-    static_assert(VS % 4 == 0 && TPR <= 64 && 64 % TPR == 0, "VS");
-    static_assert(K % RPP == 0, "K");
+template <int CTRL> __device__ __forceinline__ float dpp_add(float v) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+// Sum over the eight lanes of l / 8, in all of them: partners i ^ 1, i ^ 2
+// (quad_perm), then 7 - i of the eight (row_half_mirror).
+__device__ __forceinline__ float sum8(float v) { return dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(v))); }
 
-    const int nvs = p.V / VS;
+template <int K, int NW, bool AHEAD>
+__global__ __launch_bounds__(64 * NW) void scan_kernel(ScanParams p) {
+    constexpr int TB = 8, TPW = TB / NW;  // tokens of a block; tokens a wave prepares
+    constexpr int RI = K / 64, NJ = K / 32, VC = 16 * NW;
+    static_assert(K % 64 == 0 && TB % NW == 0, "K, NW");
+    const int nvs = p.V / VC;
     const int bh = blockIdx.x / nvs, vsl = blockIdx.x % nvs;
     const int bi = bh / p.HV, hv = bh % p.HV, hk = hv / p.rep;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int cg = tid % TPR, r0 = tid / TPR;
+    const int rg = lane & 7, cg = lane >> 3;
 
-    __shared__ float s_eg[2][K], s_a1[2][K], s_a2[2][K], s_k[2][K];
-    __shared__ float s_red[2][4][VS];
-    __shared__ float s_vn[VS];
-    __shared__ float s_kq[4];
-
-    const size_t sbase = (size_t)bh * K * p.V + (size_t)vsl * VS + cg * 4;
-    float4 S[NP];
-#pragma unroll
-    for (int i = 0; i < NP; ++i)
-        S[i] = *reinterpret_cast<const float4 *>(p.state_in + sbase + (size_t)(r0 + i * RPP) * p.V);
+    __shared__ __align__(16) float s_row[2][TB][4][K]; // e^g, e^g b k, e^g q, k
+    __shared__ __align__(8) float s_wv[2][TB][VC];
+    __shared__ float s_kq[2][TB];
 
     const int64_t koff = (int64_t)bi * p.sqb + (int64_t)hk * p.sqh;
-    const int64_t voff = (int64_t)bi * p.svb + (int64_t)hv * p.svh;
-    const int64_t ooff = (int64_t)bi * p.sob + (int64_t)hv * p.soh;
+    const int64_t voff = (int64_t)bi * p.svb + (int64_t)hv * p.svh + vsl * VC;
+    const int64_t ooff = (int64_t)bi * p.sob + (int64_t)hv * p.soh + vsl * VC;
 
-    for (int t = 0; t < p.T; ++t) {
-        const int buf = t & 1;
-        float kq = 0.0f;
-        for (int r = tid; r < K; r += 256) {
-            const int64_t o = koff + (int64_t)t * p.sqt + r;
-            const float qq = p.q[o], kk = p.k[o], gg = p.g[o], bb = p.b[o];
-            const float eg = expf(gg);
-            s_eg[buf][r] = eg;
-            s_a1[buf][r] = eg * (bb * kk);
-            s_a2[buf][r] = eg * qq;
-            s_k[buf][r] = kk;
-            kq += kk * qq;
+    // operands of a block (tokens past the end repeat the last one)
+    float x[TPW][4][RI], xv[2], xw[2];
+    auto load = [&](int t0) {
+#pragma unroll
+        for (int u = 0; u < TPW; ++u) {
+            const int64_t o = koff + (int64_t)min(t0 + wave * TPW + u, p.T - 1) * p.sqt + lane;
+#pragma unroll
+            for (int r = 0; r < RI; ++r) {
+                x[u][0][r] = p.q[o + 64 * r];
+                x[u][1][r] = p.k[o + 64 * r];
+                x[u][2][r] = p.g[o + 64 * r];
+                x[u][3][r] = p.b[o + 64 * r];
+            }
         }
-        kq = wave_sum(kq);
-        if (lane == 0) s_kq[wave] = kq;
-        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int64_t o = voff + (int64_t)min(t0 + 4 * u + tid / VC, p.T - 1) * p.svt + tid % VC;
+            xv[u] = p.v[o];
+            xw[u] = p.w[o];
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < TPW; ++u) {
+            const int t = wave * TPW + u;
+            float kq = 0.f;
+#pragma unroll
+            for (int r = 0; r < RI; ++r) {
+                const float qq = x[u][0][r], kk = x[u][1][r], eg = expf(x[u][2][r]);
+                s_row[buf][t][0][64 * r + lane] = eg;
+                s_row[buf][t][1][64 * r + lane] = eg * (x[u][3][r] * kk);
+                s_row[buf][t][2][64 * r + lane] = eg * qq;
+                s_row[buf][t][3][64 * r + lane] = kk;
+                kq += kk * qq;
+            }
+            kq = wave_sum(kq);
+            if (lane == 0) s_kq[buf][t] = kq;
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) s_wv[buf][4 * u + tid / VC][tid % VC] = xw[u] * xv[u];
+    };
 
-        float e1[4] = {0.f, 0.f, 0.f, 0.f}, e2[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p.T > 0) load(0);
+    const int col = wave * 16 + 2 * cg;
+    const size_t sbase = (size_t)bh * K * p.V + (size_t)vsl * VC + col;
+    float S[NJ][4][2];
 #pragma unroll
-        for (int i = 0; i < NP; ++i) {
-            const int r = r0 + i * RPP;
-            const float a1 = s_a1[buf][r], a2 = s_a2[buf][r];
-            e1[0] += S[i].x * a1; e1[1] += S[i].y * a1; e1[2] += S[i].z * a1; e1[3] += S[i].w * a1;
-            e2[0] += S[i].x * a2; e2[1] += S[i].y * a2; e2[2] += S[i].z * a2; e2[3] += S[i].w * a2;
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float2 v = *reinterpret_cast<const float2 *>(p.state_in + sbase + (size_t)(32 * j + 4 * rg + i) * p.V);
+            S[j][i][0] = v.x;
+            S[j][i][1] = v.y;
         }
+    if (p.T > 0) store(0);
+    __syncthreads();
+    float *out = p.out + ooff + col + (rg & 1); // lanes rg = 0, 1 store the two columns
+    for (int t0 = 0; t0 < p.T; t0 += TB) {
+        const int buf = (t0 / TB) & 1, tn = min(TB, p.T - t0);
+        if (t0 + TB < p.T) load(t0 + TB);
+        // AHEAD: e^g b k and e^g q of token t are read during the token before it
+        float4 a1[NJ], a2[NJ], eg[NJ], kk[NJ];
+        auto fetch = [&](int t) {
+            const float4 *row = reinterpret_cast<const float4 *>(&s_row[buf][t][0][0]) + rg;
 #pragma unroll
-        for (int off = TPR; off < 64; off <<= 1)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                e1[j] += __shfl_xor(e1[j], off, 64);
-                e2[j] += __shfl_xor(e2[j], off, 64);
+            for (int j = 0; j < NJ; ++j) {
+                a1[j] = row[K / 4 + 8 * j];
+                a2[j] = row[2 * (K / 4) + 8 * j];
             }
-        if (lane < TPR)
+        };
+        if (AHEAD) fetch(0);
+        for (int t = 0; t < tn; ++t) {
+            const float4 *row = reinterpret_cast<const float4 *>(&s_row[buf][t][0][0]) + rg;
+            if (AHEAD) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                s_red[0][wave][cg * 4 + j] = e1[j];
-                s_red[1][wave][cg * 4 + j] = e2[j];
+                for (int j = 0; j < NJ; ++j) {
+                    eg[j] = row[8 * j];
+                    kk[j] = row[3 * (K / 4) + 8 * j];
+                }
             }
-        __syncthreads();
-        if (tid < VS) {
-            const float E1 = s_red[0][0][tid] + s_red[0][1][tid] + s_red[0][2][tid] + s_red[0][3][tid];
-            const float E2 = s_red[1][0][tid] + s_red[1][1][tid] + s_red[1][2][tid] + s_red[1][3][tid];
-            const float kqs = s_kq[0] + s_kq[1] + s_kq[2] + s_kq[3];
-            const int col = vsl * VS + tid;
-            const int64_t vo = voff + (int64_t)t * p.svt + col;
-            const float vn = p.w[vo] * p.v[vo] - E1;
-            p.out[ooff + (int64_t)t * p.sot + col] = p.scale * (E2 + vn * kqs);
-            s_vn[tid] = vn;
+            const float2 wv = *reinterpret_cast<const float2 *>(&s_wv[buf][t][col]);
+            const float kq = s_kq[buf][t];
+            if (AHEAD) __builtin_amdgcn_sched_barrier(0); // these reads ahead of the sums that hide them
+            float e1[2] = {0.f, 0.f}, e2[2] = {0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const float4 x1 = AHEAD ? a1[j] : row[K / 4 + 8 * j], x2 = AHEAD ? a2[j] : row[2 * (K / 4) + 8 * j];
+                const float a1v[4] = {x1.x, x1.y, x1.z, x1.w}, a2v[4] = {x2.x, x2.y, x2.z, x2.w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        e1[c] += S[j][i][c] * a1v[i];
+                        e2[c] += S[j][i][c] * a2v[i];
+                    }
+            }
+            if (AHEAD) {
+                fetch(min(t + 1, TB - 1));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const float vn[2] = {wv.x - sum8(e1[0]), wv.y - sum8(e1[1])};
+            const float o0 = p.scale * (sum8(e2[0]) + vn[0] * kq), o1 = p.scale * (sum8(e2[1]) + vn[1] * kq);
+            if (rg < 2) out[(int64_t)(t0 + t) * p.sot] = rg ? o1 : o0;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const float4 x1 = AHEAD ? eg[j] : row[8 * j], x2 = AHEAD ? kk[j] : row[3 * (K / 4) + 8 * j];
+                const float egv[4] = {x1.x, x1.y, x1.z, x1.w}, kkv[4] = {x2.x, x2.y, x2.z, x2.w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) S[j][i][c] = S[j][i][c] * egv[i] + kkv[i] * vn[c];
+            }
         }
-        __syncthreads();
-        const float4 vn = *reinterpret_cast<const float4 *>(&s_vn[cg * 4]);
-#pragma unroll
-        for (int i = 0; i < NP; ++i) {
-            const int r = r0 + i * RPP;
-            const float eg = s_eg[buf][r], kk = s_k[buf][r];
-            S[i].x = S[i].x * eg + kk * vn.x;
-            S[i].y = S[i].y * eg + kk * vn.y;
-            S[i].z = S[i].z * eg + kk * vn.z;
-            S[i].w = S[i].w * eg + kk * vn.w;
+        if (t0 + TB < p.T) {
+            store(buf ^ 1);
+            __syncthreads(); // the next block's rows are there; every wave is done with this block's
         }
     }
 #pragma unroll
-    for (int i = 0; i < NP; ++i)
-        *reinterpret_cast<float4 *>(p.state_out + sbase + (size_t)(r0 + i * RPP) * p.V) = S[i];
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<float2 *>(p.state_out + sbase + (size_t)(32 * j + 4 * rg + i) * p.V) =
+                make_float2(S[j][i][0], S[j][i][1]);
 }
 
 // Any K, V (<= 1024): one workgroup per (b, hv), the state is updated in
@@ -635,10 +702,17 @@ __global__ __launch_bounds__(256) void decode_fused_generic_kernel(DecodeParams 
     }
 }
 
-template <int K, int VS>
+// Up to two workgroups a unit a token is a chain of LDS reads, sums and
+// exchanges, and reading ahead (178 registers at K = 128) shortens it: 4
+// sequences of 37 tokens at 16 heads 25 against 34 us.  Beyond, four waves a
+// SIMD (127 registers) hide it better: 32 sequences of 48 tokens 75 against 82.
+template <int K, int NW>
 hipError_t launch_scan_t(const ScanParams &p, hipStream_t s) {
-    const int grid = p.B * p.HV * (p.V / VS);
-    hipLaunchKernelGGL((scan_kernel<K, VS>), dim3(grid), dim3(256), 0, s, p);
+    const int grid = p.B * p.HV * (p.V / (16 * NW));
+    if (grid <= 512)
+        hipLaunchKernelGGL((scan_kernel<K, NW, true>), dim3(grid), dim3(64 * NW), 0, s, p);
+    else
+        hipLaunchKernelGGL((scan_kernel<K, NW, false>), dim3(grid), dim3(64 * NW), 0, s, p);
     return hipGetLastError();
 }
 
@@ -664,14 +738,17 @@ hipError_t launch_scan(const ScanParams &p, hipStream_t s) {
         if (p.K == 64 && p.V == 64) return launch_step_t<64, 64>(p, s);
         if (p.K == 64 && p.V == 128) return launch_step_t<64, 128>(p, s);
     }
-    // Register kernels: VS columns per workgroup.  VS = 64 splits each head's
-    // V = 128 columns over two workgroups, which doubles the number of
-    // workgroups for small batch x head counts.
-    if (p.K == 128 && p.V % 64 == 0) return launch_scan_t<128, 64>(p, s);
-    if (p.K == 64 && p.V % 64 == 0) return launch_scan_t<64, 64>(p, s);
-    if (p.K == 256 && p.V % 64 == 0) return launch_scan_t<256, 64>(p, s);
-    if (p.K == 64 && p.V % 32 == 0) return launch_scan_t<64, 32>(p, s);
-    if (p.K == 128 && p.V % 32 == 0) return launch_scan_t<128, 32>(p, s);
+    // Register kernels: four waves (64 columns) a workgroup, or two where V is
+    // no multiple of 64.
+    if (p.V % 64 == 0) {
+        if (p.K == 64) return launch_scan_t<64, 4>(p, s);
+        if (p.K == 128) return launch_scan_t<128, 4>(p, s);
+        if (p.K == 256) return launch_scan_t<256, 4>(p, s);
+    } else if (p.V % 32 == 0) {
+        if (p.K == 64) return launch_scan_t<64, 2>(p, s);
+        if (p.K == 128) return launch_scan_t<128, 2>(p, s);
+        if (p.K == 256) return launch_scan_t<256, 2>(p, s);
+    }
     const size_t lds = sizeof(float) * 4 * (size_t)p.K;
     hipLaunchKernelGGL(scan_generic_kernel, dim3(p.B * p.HV), dim3(256), lds, s, p);
     return hipGetLastError();
