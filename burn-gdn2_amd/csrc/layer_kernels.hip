@@ -43,18 +43,23 @@ __device__ __forceinline__ float conv4(const float *x, int64_t ldx, int t, const
     return acc;
 }
 
-// One workgroup per (batch row, block of kProjTB tokens, head), so that every
+// One workgroup per (batch row, block of TB tokens, head), so that every
 // raw projection element is read once (plus three tokens of conv history per
 // thread's run of tokens) and every output is a contiguous head-major block.
 // Key heads (blockIdx.y < H) produce q, k, g, b of their head; the L2 norms
 // over K need the whole head, so q and k pass through LDS (heads up to 256
 // channels; wider heads keep them in the output rows instead).  Value heads
-// produce v and w.  A thread owns one channel and a run of kProjRun tokens,
+// produce v and w.  A thread owns one channel and a run of RUN tokens,
 // sliding the four-tap window along it.  Blocks of 32 tokens give a head of
 // 128 channels exactly one (channel, run) per thread, so that every load of a
 // thread is requested at once (64-token blocks took two rounds: 876 against
-// 717 us at B = 8, T = 4096).
-constexpr int kProjTB = 32, kProjRun = 16, kProjLdsMaxK = 256;
+// 717 us at B = 8, T = 4096).  The launch takes shorter runs where those
+// would leave threads without work (64 channels), and blocks of 8 tokens
+// where the grid does not fill the chip: a run is a serial chain of gates.
+// Measured against blocks of 32 with runs of 16 everywhere: 4 x 37 tokens of
+// 16 heads of 128 9.4 against 19.7 us, 1 x 1024 of 4 heads of 64 7.3 against
+// 18.0, 8 x 4096 of 16 heads of 64 440 against 463.
+constexpr int kProjLdsMaxK = 256;
 
 // xpad row of token tt (tt < 0: the cache, or token 0 replicated) in column c
 __device__ __forceinline__ float conv_row(const float *col, int64_t ld, int tt, const float *cache, int64_t n_ch) {
@@ -62,27 +67,28 @@ __device__ __forceinline__ float conv_row(const float *col, int64_t ld, int tt, 
     return cache ? cache[(int64_t)(3 + tt) * n_ch] : col[0];
 }
 
+template <int TB, int RUN>
 __global__ __launch_bounds__(256) void project_kernel(ProjectParams p) {
     extern __shared__ float sm[];
-    const int nb = (p.T + kProjTB - 1) / kProjTB;
-    const int bi = blockIdx.x / nb, t0 = (blockIdx.x % nb) * kProjTB;
+    const int nb = (p.T + TB - 1) / TB;
+    const int bi = blockIdx.x / nb, t0 = (blockIdx.x % nb) * TB;
     const int head = blockIdx.y;
-    const int tn = min(kProjTB, p.T - t0);
+    const int tn = min(TB, p.T - t0);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const bool sc = p.use_short_conv != 0;
     const int kd = p.H * p.K, vd = p.HV * p.V;
     const float *Y0 = p.Y + (int64_t)bi * p.T * p.ldY;  // token 0 of this sequence
-    constexpr int NRUN = kProjTB / kProjRun;
+    constexpr int NRUN = TB / RUN;
     if (head < p.H) {
         const int h = head, K = p.K, K1 = K + 1;
         const int64_t ob = ((int64_t)bi * p.H + h) * p.T * K;  // [B, H, T, K] row of token 0
         // staging of the activated q, k of token t0 + tl, channel c
         const bool lds = K <= kProjLdsMaxK;
-        float *sq = lds ? sm : p.q + ob + (int64_t)t0 * K, *sk = lds ? sm + kProjTB * K1 : p.k + ob + (int64_t)t0 * K;
+        float *sq = lds ? sm : p.q + ob + (int64_t)t0 * K, *sk = lds ? sm + TB * K1 : p.k + ob + (int64_t)t0 * K;
         const int ld = lds ? K1 : K;
         for (int e = tid; e < K * NRUN; e += 256) {
             const int c = e % K, run = e / K, gc = h * K + c;
-            const int ta = t0 + run * kProjRun, tb = min(t0 + tn, ta + kProjRun);
+            const int ta = t0 + run * RUN, tb = min(t0 + tn, ta + RUN);
             if (ta >= tb) continue;
             const float *qc = Y0 + p.off_q + gc, *kc = Y0 + p.off_k + gc;
             float wq[4] = {0.f, 0.f, 0.f, 0.f}, wk[4] = {0.f, 0.f, 0.f, 0.f};
@@ -104,9 +110,9 @@ __global__ __launch_bounds__(256) void project_kernel(ProjectParams p) {
             const float dtb = p.dt_bias[gc], A = expf(p.a_log[h]);
             const float dfs = p.decay_factors ? sigmoid_(p.decay_factors[gc]) * p.one_minus_min_decay : 0.f;
             // the run's loads first, all in flight together (rows past the end read row ta)
-            float xqs[kProjRun], xks[kProjRun], fs[kProjRun], bs[kProjRun];
+            float xqs[RUN], xks[RUN], fs[RUN], bs[RUN];
 #pragma unroll
-            for (int j = 0; j < kProjRun; ++j) {
+            for (int j = 0; j < RUN; ++j) {
                 const int t = ta + j < tb ? ta + j : ta;
                 const int64_t row = (int64_t)t * p.ldY;
                 xqs[j] = qc[row];
@@ -115,7 +121,7 @@ __global__ __launch_bounds__(256) void project_kernel(ProjectParams p) {
                 bs[j] = Y0[row + p.off_b + gc];
             }
 #pragma unroll
-            for (int j = 0; j < kProjRun; ++j) {
+            for (int j = 0; j < RUN; ++j) {
                 const int t = ta + j;
                 if (t >= tb) continue;  // (only the tail of the last block)
                 const float xq = xqs[j], xk = xks[j];
@@ -161,7 +167,7 @@ __global__ __launch_bounds__(256) void project_kernel(ProjectParams p) {
         const int64_t ob = ((int64_t)bi * p.HV + hv) * p.T * V;  // [B, HV, T, V] row of token 0
         for (int e = tid; e < V * NRUN; e += 256) {
             const int c = e % V, run = e / V, gc = hv * V + c;
-            const int ta = t0 + run * kProjRun, tb = min(t0 + tn, ta + kProjRun);
+            const int ta = t0 + run * RUN, tb = min(t0 + tn, ta + RUN);
             if (ta >= tb) continue;
             const float *vc = Y0 + p.off_v + gc;
             float wv[4] = {0.f, 0.f, 0.f, 0.f}, v1 = 0.f, v2 = 0.f, v3 = 0.f;
@@ -172,16 +178,16 @@ __global__ __launch_bounds__(256) void project_kernel(ProjectParams p) {
                 v1 = conv_row(vc, p.ldY, ta - 3, cv, vd); v2 = conv_row(vc, p.ldY, ta - 2, cv, vd);
                 v3 = conv_row(vc, p.ldY, ta - 1, cv, vd);
             }
-            float xvs[kProjRun], xws[kProjRun];
+            float xvs[RUN], xws[RUN];
 #pragma unroll
-            for (int j = 0; j < kProjRun; ++j) {
+            for (int j = 0; j < RUN; ++j) {
                 const int t = ta + j < tb ? ta + j : ta;
                 const int64_t row = (int64_t)t * p.ldY;
                 xvs[j] = vc[row];
                 xws[j] = Y0[row + p.off_w + gc];
             }
 #pragma unroll
-            for (int j = 0; j < kProjRun; ++j) {
+            for (int j = 0; j < RUN; ++j) {
                 const int t = ta + j;
                 if (t >= tb) continue;
                 const float xv = xvs[j];
@@ -654,20 +660,25 @@ int grid_for(int64_t n) {
 
 size_t project_lds_bytes(int kd) { return sizeof(float) * 2 * (size_t)kd; }
 
-size_t project_tile_lds_bytes(int K) { return K <= kProjLdsMaxK ? sizeof(float) * 2 * (size_t)kProjTB * (K + 1) : 0; }
-
-hipError_t launch_project(const ProjectParams &p, hipStream_t s) {
-    const int64_t M = (int64_t)p.B * p.T;
-    if (M == 0) return hipSuccess;
-    const size_t lds = project_tile_lds_bytes(p.K);
+namespace {
+template <int TB, int RUN> hipError_t launch_project_t(const ProjectParams &p, hipStream_t s) {
+    const size_t lds = p.K <= kProjLdsMaxK ? sizeof(float) * 2 * TB * (size_t)(p.K + 1) : 0;
     if (lds > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&project_kernel),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&project_kernel<TB, RUN>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    const int nb = (p.T + kProjTB - 1) / kProjTB;
-    hipLaunchKernelGGL(project_kernel, dim3((unsigned)(p.B * nb), (unsigned)(p.H + p.HV)), dim3(256), lds, s, p);
+    const int nb = (p.T + TB - 1) / TB;
+    hipLaunchKernelGGL((project_kernel<TB, RUN>), dim3((unsigned)(p.B * nb), (unsigned)(p.H + p.HV)), dim3(256), lds, s, p);
     return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_project(const ProjectParams &p, hipStream_t s) {
+    if (p.B == 0 || p.T == 0) return hipSuccess;
+    const bool few = (int64_t)p.B * ((p.T + 31) / 32) * (p.H + p.HV) < 1024; // four workgroups a unit
+    if (p.K <= 64) return few ? launch_project_t<8, 2>(p, s) : launch_project_t<32, 8>(p, s);
+    return few ? launch_project_t<8, 4>(p, s) : launch_project_t<32, 16>(p, s);
 }
 
 hipError_t launch_gva_expand(const GvaParams &p, hipStream_t s) {
