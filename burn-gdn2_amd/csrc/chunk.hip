@@ -684,20 +684,31 @@ __global__ __launch_bounds__(512, K > 128 ? 2 : 4) void chunk_intra_kernel(Chunk
 }
 
 // ---------------------------------------------------------------------------
-// chunk-inter: one workgroup per (b, hv, 64 value columns); wave w owns 16
-// columns.  S[:, cols] stays in MFMA accumulators for the whole sequence.
+// chunk-inter: one workgroup per (b, hv, 64 value columns); a wave owns 16
+// columns.  S[:, cols] stays in f32 accumulators for the whole sequence.
 // Per chunk n:
 //   A: X1 = W S, X2 = scale (q exp(G)) S      (reads sW, sQ)
 //   B: v_new = U - X1
 //   C: S = exp(G_last) S + Kd^T v_new         (reads sKd)
 //   D: out = X2 + A_qk v_new                  (reads sA; independent of C)
-// D(n) runs at the top of iteration n + 1, before the wait for chunk n + 1's
-// copies, whose latency its MFMAs cover.
-// LDS holds one chunk of W, q exp(G) (2 C K floats), Kd^T (K C) and A_qk
-// (C C).  Each buffer is refilled while another phase runs: Kd^T(n) and
-// A_qk(n) are fetched during A(n) and stored after it; W, q exp(G)(n+1) are
-// fetched during B-D(n) and stored after them.  HBM latency is therefore off
-// the sequential path without a second copy of the buffers.
+// The products run on the f16 matrix cores, two f16 terms per f32 operand
+// (chunk_common.hpp): as f32 products they took 13.6k of a chunk's 17.2k
+// cycles (K = 128, one wave a SIMD).  Each wave loads its share of W, q exp(G),
+// Kd^T and A_qk as f32 row tiles, half a chunk ahead of their use, finds the
+// rows' scales in registers and writes the terms into LDS, where a chunk of
+// every operand has one buffer: W, q exp(G)(n + 1) while C(n), D(n) run,
+// Kd^T, A_qk(n) while A(n) runs.  S and v_new are split in registers, with a
+// scale per column.
+// What bounds it now: at one wave a SIMD a chunk's 5k cycles of vector
+// instructions (half of them splitting), 2.6k of matrix instructions and 5k of
+// LDS reads ran one after the other, 15k in all; with a state and an output
+// wave per column tile (inter_roles) they overlap, 12k, of which LDS is busy
+// half.  Measured, before -> now: B = 8, T = 4096, 16 heads, K = V = 128 478
+// -> 429 us under the profiler, with chunk-intra 1007 -> 887 us a pass; B = 1,
+// T = 32768 pass 1 (two waves a SIMD) 562 -> 279 us beside the walk, pass 3
+// 529 -> 339 us.
+// Error against f64 (2-norm, outputs and state): unchanged to two digits
+// (2.6e-7).
 //
 // Segmented form (NSEG > 1, few long sequences).  Over one segment the
 // recurrence is affine in its entering state:
@@ -739,31 +750,49 @@ __device__ __forceinline__ size_t seg_slot(const ChunkParams &p, int bh, int j) 
     return (size_t)bh * p.NSLOT + (j - p.SLOT0);
 }
 
+// Waves of a workgroup.  With the output (and K <= 128) each column tile has
+// two: a state wave (A's X1, B, C) and an output wave (A's X2, D, the stores),
+// so that one's matrix instructions, LDS reads and splitting cover the
+// other's waits; the state wave hands S and v_new over in LDS, already as f16
+// terms.  K = 256 has no LDS left for that.
+constexpr bool inter_roles(int K, int MODE) {
+    return (MODE == kInterOut || MODE == kInterOutStates || MODE == kInterOutTrain) && K <= 128;
+}
+constexpr int inter_threads(int K, int MODE, int NWV) { return 64 * NWV * (inter_roles(K, MODE) ? 2 : 1); }
+
 template <int K, int MODE, int NWV>
-__global__ __launch_bounds__(64 * NWV, 1) void chunk_inter_kernel(ChunkParams p, int nseg_launch, int seg_base) {
+__global__ __launch_bounds__(inter_threads(K, MODE, NWV), 1) void chunk_inter_kernel(ChunkParams p, int nseg_launch,
+                                                                                     int seg_base) {
     constexpr bool OUT = MODE == kInterOut || MODE == kInterOutStates || MODE == kInterOutTrain;
     constexpr bool LOCAL = MODE == kInterLocal;
     constexpr bool STATES = MODE == kInterStates || MODE == kInterOutStates || MODE == kInterOutTrain;
     constexpr bool FRAG = MODE == kInterStates || MODE == kInterOutTrain; // the backward's layouts
-    constexpr int NTH = 64 * NWV;  // threads per workgroup
-    constexpr int VSW = 16 * NWV;  // value columns per workgroup
+    constexpr bool ROLES = inter_roles(K, MODE);
+    constexpr int VSW = 16 * NWV; // value columns per workgroup
     constexpr int NKT = K / 16;
     constexpr int FR = NKT * NT;   // 16x16 fragments per operand per chunk
     constexpr int OPF4 = FR * 64;  // float4 per operand per chunk
-    constexpr int PFO = OPF4 / NTH; // float4 per lane per operand
-    static_assert(OPF4 % NTH == 0 && K % VSW == 0, "K");
+    static_assert(K % VSW == 0, "K");
     constexpr int AF4 = NT * NT * 64; // float4 of A_qk per chunk
-    constexpr int APF = AF4 / NTH;
-    __shared__ floatx4 sW[OPF4], sKd[OPF4];
     // K = 256: W and Kd^T take 64 KiB each, so scale q exp(G), which feeds only
     // the output (off the sequential chain), is read from L2 into registers in
-    // phase A instead of through a third LDS buffer (145 KiB in all).
-    constexpr bool QLDS = OUT && K <= 128;
-    __shared__ floatx4 sQ[QLDS ? OPF4 : 1], sA[OUT ? AF4 : 1];
-    __shared__ float sPf[NTH]; // destination of the L2 touches, never read
-    // exp(G_last) of the chunk, copied with Kd^T: read just before phase C, so
-    // that it holds no registers through phases A and D
-    __shared__ floatx4 sGam[K / 4];
+    // phase A instead of through a third LDS buffer, and its product is an f32
+    // one.
+    constexpr bool QLDS = ROLES;
+    // A_qk by pairs of tiles on or below the diagonal: row tiles 0 and 1 hold one, 2 and 3 two
+    constexpr int AFR = 12;
+    __shared__ floatx4 sW[OPF4], sKd[OPF4];
+    __shared__ floatx4 sQ[QLDS ? OPF4 : 1], sA[OUT ? AFR * 64 : 1];
+    __shared__ floatx4 sS[ROLES ? NWV * NKT * 64 : 1], sV[ROLES ? NWV * NT * 64 : 1]; // S, v_new of the column tiles
+    __shared__ float eS[ROLES ? NWV * 16 : 1], eV[ROLES ? NWV * 16 : 1];              // and their columns' inverse scales
+    __shared__ floatx4 sGam[K / 4]; // exp(G_last) of the chunk
+    // inverse scales of the rows of W, q exp(G), Kd^T and A_qk (split_row_tile)
+    __shared__ __align__(16) float eW[C], eQ[QLDS ? C : 4], eK[K], eA[OUT ? C : 4];
+    // A chunk's operands are loaded and split by row tiles: CW row tiles of W,
+    // q exp(G) and A_qk a wave (with eight waves the first four take one each),
+    // CK of Kd^T.
+    constexpr int CW = NWV <= NT ? NT / NWV : 1, CK = NKT / NWV;
+    static_assert(NKT % NWV == 0, "row tiles of Kd^T per wave");
 
     const int V = p.V;
     const int nvv = V / VSW;                    // value slices
@@ -773,30 +802,15 @@ __global__ __launch_bounds__(64 * NWV, 1) void chunk_inter_kernel(ChunkParams p,
     const int bh = sq / nseg_launch, seg = seg_base + sq % nseg_launch;
     const int bi = bh / p.HV, hv = bh % p.HV;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6); // wave-uniform (scalar)
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6); // wave-uniform (scalar)
+    const int wave = wid % NWV;                               // this wave's column tile
+    const bool out_role = ROLES && wid >= NWV;
     const int lr = lane & 15, lg = lane >> 4;
     const bool pcol = LOCAL && vs >= nvv;          // a slice of P (wave-uniform)
     const int vt = (pcol ? vs - nvv : vs) * NWV + wave; // this wave's 16-column tile
     const int col = 16 * vt + lr;
     int n0, n1;
     seg_range(p, seg, &n0, &n1);
-
-    // entering state: S0 (one segment, or the split's segment 0), the chained
-    // state (pass 3; in uniform runs slot 0 is a copy of S0, so that no
-    // workgroup reads the state that the last segment overwrites), 0 (pass 1
-    // value columns) or the identity (pass 1, P columns)
-    const float *Sin = nullptr;
-    if (!LOCAL)
-        Sin = p.NSEG == 1 || (p.SLOT0 && seg == 0) ? p.state + (size_t)bh * K * V
-                                                   : p.ws_qseg + seg_slot(p, bh, seg) * K * V;
-    floatx4 S[NKT];
-#pragma unroll
-    for (int kb = 0; kb < NKT; ++kb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = 16 * kb + 4 * lg + i;
-            S[kb][i] = !LOCAL ? Sin[(size_t)row * V + col] : (pcol && row == col ? 1.f : 0.f);
-        }
 
     const floatx4 *__restrict__ W4 = reinterpret_cast<const floatx4 *>(p.ws_w);
     const floatx4 *__restrict__ Q4 = reinterpret_cast<const floatx4 *>(p.ws_qg);
@@ -807,44 +821,82 @@ __global__ __launch_bounds__(64 * NWV, 1) void chunk_inter_kernel(ChunkParams p,
     const size_t cid0 = (size_t)bh * p.NC;
     const size_t uvf4 = (size_t)C * V / 4;
 
-    // the operands go from global memory straight into LDS (lds_copy4):
-    // thread tid's float4 i lands at index i * NTH + tid, as a wave's 64 lanes.
-    // (The buffer-resource form of these copies, buffer_load_dwordx4 ... lds
-    // with 32-bit offsets, needs fewer registers but measured 1.8 % slower.)
-    const int wv = 64 * wave;
-    // Each chunk's operands are also pulled toward L2 one phase before their
-    // LDS copy (l2_touch, one 128-byte line per thread): W, q exp(G) of chunk
-    // n + 1 during A(n), Kd^T, A_qk, U of chunk n + 1 during B-D(n).  Every
-    // wave issues the same count (2, then 3) last before the vmcnt waits, which
-    // leave them in flight; past the last chunk the current one is touched.
-    float *pf_slot = &sPf[wv];
-    constexpr int LOP = OPF4 / 8, LA = AF4 / 8, LU = NWV * NT * 64 / 8; // lines per operand block
-    const int vsu = pcol ? 0 : vs; // the P slices of pass 1 read no U
-    auto touch_wq = [&](size_t c) { // 2 per wave
-        l2_touch(reinterpret_cast<const char *>(W4 + c * OPF4) + 128 * (tid % LOP), pf_slot);
-        l2_touch(reinterpret_cast<const char *>((OUT ? Q4 : K4) + c * OPF4) + 128 * (tid % LOP), pf_slot);
-    };
-    auto touch_kau = [&](size_t c) { // 3 per wave
-        l2_touch(reinterpret_cast<const char *>(K4 + c * OPF4) + 128 * (tid % LOP), pf_slot);
-        if (OUT)
-            l2_touch(reinterpret_cast<const char *>(A4 + c * AF4) + 128 * (tid % LA), pf_slot);
-        else
-            l2_touch(reinterpret_cast<const char *>(W4 + c * OPF4) + 128 * (tid % LOP), pf_slot);
-        l2_touch(reinterpret_cast<const char *>(U4 + c * uvf4 + (size_t)vsu * NWV * NT * 64) + 128 * (tid % LU), pf_slot);
-    };
-    if (n1 > n0) {
+    // This wave's row tiles of the operands, on their way from HBM to LDS: W and
+    // q exp(G) of chunk n + 1 are requested at the start of A(n) (K = 256: of
+    // C(n), for registers) and split into sW, sQ during C(n); Kd^T, A_qk,
+    // exp(G_last) and U of chunk n + 1 at the start of C(n) (K = 256: Kd^T of
+    // chunk n at the start of A(n)), and split into sKd, sA during A(n + 1).
+    // Past the last chunk the current one is taken again.
+    constexpr bool LATE = K > 128;
+    const bool owns_w = NWV <= NT || wave < NT; // (wave-uniform)
+    auto load_rows = [&](const floatx4 *src, floatx4 *r, size_t c) { // W or q exp(G)
 #pragma unroll
-        for (int i = 0; i < PFO; ++i) {
-            lds_copy4(&W4[(cid0 + n0) * OPF4 + i * NTH + tid], &sW[i * NTH + wv]);
-            if (QLDS) lds_copy4(&Q4[(cid0 + n0) * OPF4 + i * NTH + tid], &sQ[i * NTH + wv]);
+        for (int i = 0; i < CW * NKT; ++i) r[i] = ld_uni(src + c * OPF4 + (owns_w ? wave : 0) * CW * NKT * 64, i * 64 + lane);
+    };
+    auto split_rows = [&](const floatx4 *r, floatx4 *s, float *e) {
+        if (!owns_w) return;
+#pragma unroll
+        for (int i = 0; i < CW; ++i) {
+            const int mt = wave * CW + i;
+            split_row_tile<NKT>(&r[i * NKT], &s[mt * NKT * 64], lane, &e[16 * mt]);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        touch_kau(cid0 + n0);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    // S and the first copies have landed: nothing from before the loop is
-    // left in flight for the compiler's own vmcnt waits inside it
-    vm_wait0();
+    };
+    auto load_a = [&](floatx4 *r, size_t c) { // A_qk is lower block-triangular: tiles (mt, qt <= mt) only
+#pragma unroll
+        for (int i = 0; i < CW * NT; ++i) {
+            const int mt = wave * CW + i / NT, qt = i % NT;
+            r[i] = qt <= mt ? ld_uni(A4 + c * AF4 + mt * NT * 64, qt * 64 + lane) : floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    const auto a_first = [](int mt) { return mt < 2 ? 2 * mt : 4 * (mt - 1); }; // row tile mt's first fragment in sA
+    auto split_a = [&](const floatx4 *r) {
+#pragma unroll
+        for (int i = 0; i < CW; ++i) {
+            const int mt = wave * CW + i;
+            floatx4 *d = &sA[a_first(mt) * 64];
+            if (mt < 2)
+                split_row_tile<2>(&r[i * NT], d, lane, &eA[16 * mt]);
+            else
+                split_row_tile<4>(&r[i * NT], d, lane, &eA[16 * mt]);
+        }
+    };
+    auto rows_of = [&](const float *e, int tile) { return *reinterpret_cast<const floatx4 *>(&e[16 * tile + 4 * lg]); };
+    auto half8 = [&](const floatx4 *s, int f) { return __builtin_bit_cast(halfx8, s[f * 64 + lane]); };
+    // X (+)= T S' for the NT row tiles of a chunk operand in LDS (W or q exp(G))
+    auto times_s = [&](const floatx4 *s, const halfx8 *hi, const halfx8 *lo, floatx4 *X) {
+#pragma unroll
+        for (int mt = 0; mt < NT; ++mt) X[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        halfx8 w[2][NT][2]; // a step's operands are read during the step before it
+        auto fetch = [&](int kp) {
+#pragma unroll
+            for (int mt = 0; mt < NT; ++mt)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) w[kp & 1][mt][h] = half8(s, mt * NKT + 2 * kp + h);
+        };
+        fetch(0);
+#pragma unroll
+        for (int kp = 0; kp < NKT / 2; ++kp) {
+            if (kp + 1 < NKT / 2) fetch(kp + 1);
+#pragma unroll
+            for (int t = 0; t < 3; ++t) // hi hi, lo hi, hi lo: four independent chains
+#pragma unroll
+                for (int mt = 0; mt < NT; ++mt)
+                    X[mt] = mfma32h(w[kp & 1][mt][t == 1], t == 2 ? lo[kp] : hi[kp], X[mt]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // y = A_qk v_new
+    auto times_v = [&](const halfx8 *vh, const halfx8 *vl, floatx4 *y) {
+#pragma unroll
+        for (int mt = 0; mt < NT; ++mt) y[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int tp = 0; tp < NT / 2; ++tp)
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+#pragma unroll
+                for (int mt = 2 * tp; mt < NT; ++mt)
+                    y[mt] = mfma32h(half8(sA, a_first(mt) + 2 * tp + (t == 1)), t == 2 ? vl[tp] : vh[tp], y[mt]);
+    };
 
     // chunk nn's output rows from X2 through a buffer resource over its valid
     // rows: rows past T fall outside its range and the hardware drops those
@@ -864,51 +916,126 @@ __global__ __launch_bounds__(64 * NWV, 1) void chunk_inter_kernel(ChunkParams p,
                 __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, val), R, olane, 4 * (16 * mt + i) * sot, 0);
             }
     };
-    floatx4 X1[NT], X2[NT]; // chunk n's v_new and output, both read again in iteration n + 1
-    // D: out = X2 + A_qk v_new (A_qk is lower block-triangular; the chains of
-    // the four time tiles interleave).  D(n) runs at the top of iteration
-    // n + 1, where its MFMAs cover this wave's wait for the next copies.  Its
-    // A_qk tiles are read from sA during the last time tile of C(n), so that
-    // D waits on no LDS read.
-    floatx4 aq[NT][NT]; // A_qk tiles (mt, qt), mt >= qt
-    auto load_aq = [&]() {
+
+    if (ROLES && out_role) { // the output wave of a column tile (every barrier below has its twin in the state wave)
+        if (n1 <= n0) return;
+        floatx4 rq[QLDS ? CW * NKT : 1], ra[CW * NT], X2[NT];
+        load_rows(Q4, rq, cid0 + n0);
+        load_a(ra, cid0 + n0);
+        split_rows(rq, sQ, eQ);
+        for (int n = n0; n < n1; ++n) {
+            const size_t cnext = cid0 + (n + 1 < n1 ? n + 1 : n);
+            lds_barrier(); // sQ and S's terms of chunk n are there; the state wave is done with sKd (n-1)
+            load_rows(Q4, rq, cnext);
+            if (n > n0) store_out(X2, n - 1);
+            __builtin_amdgcn_sched_barrier(0); // keep these loads here, a phase ahead of their use
+            halfx8 hi[NKT / 2], lo[NKT / 2];
 #pragma unroll
-        for (int qt = 0; qt < NT; ++qt)
+            for (int kp = 0; kp < NKT / 2; ++kp) {
+                hi[kp] = half8(sS, wave * NKT + 2 * kp);
+                lo[kp] = half8(sS, wave * NKT + 2 * kp + 1);
+            }
+            times_s(sQ, hi, lo, X2); // X2 = scale (q exp(G)) S
+            const float es = eS[wave * 16 + lr];
 #pragma unroll
-            for (int mt = qt; mt < NT; ++mt) aq[mt][qt] = sA[(mt * NT + qt) * 64 + lane];
+            for (int mt = 0; mt < NT; ++mt) X2[mt] = X2[mt] * (rows_of(eQ, mt) * es);
+            split_a(ra);
+            lds_barrier(); // sQ free; sA and v_new's terms of chunk n are there
+            load_a(ra, cnext);
+            __builtin_amdgcn_sched_barrier(0);
+            halfx8 vh[NT / 2], vl[NT / 2];
+#pragma unroll
+            for (int tp = 0; tp < NT / 2; ++tp) {
+                vh[tp] = half8(sV, wave * NT + 2 * tp);
+                vl[tp] = half8(sV, wave * NT + 2 * tp + 1);
+            }
+            floatx4 y[NT];
+            times_v(vh, vl, y); // D: out = X2 + A_qk v_new
+            const float ev = eV[wave * 16 + lr];
+#pragma unroll
+            for (int mt = 0; mt < NT; ++mt) X2[mt] += y[mt] * (rows_of(eA, mt) * ev);
+            split_rows(rq, sQ, eQ);
+        }
+        store_out(X2, n1 - 1);
+        return;
+    }
+
+    // entering state: S0 (one segment, or the split's segment 0), the chained
+    // state (pass 3; in uniform runs slot 0 is a copy of S0, so that no
+    // workgroup reads the state that the last segment overwrites), 0 (pass 1
+    // value columns) or the identity (pass 1, P columns)
+    const float *Sin = nullptr;
+    if (!LOCAL)
+        Sin = p.NSEG == 1 || (p.SLOT0 && seg == 0) ? p.state + (size_t)bh * K * V
+                                                   : p.ws_qseg + seg_slot(p, bh, seg) * K * V;
+    // S and the leaving state through buffer resources: 32-bit offsets, a lane
+    // term and a wave-uniform row term, that hold no registers across the loop
+    auto state_rsrc = [&](const float *base, int ld) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), (short)0, K * ld * 4, 0x00020000);
     };
-    auto phase_d = [&]() {
+    floatx4 S[NKT];
+    const __amdgpu_buffer_rsrc_t Rin = state_rsrc(LOCAL ? p.state : Sin, V);
 #pragma unroll
-        for (int qt = 0; qt < NT; ++qt)
+    for (int kb = 0; kb < NKT; ++kb)
 #pragma unroll
-            for (int st = 0; st < 4; ++st)
+        for (int i = 0; i < 4; ++i) {
+            const int row = 16 * kb + 4 * lg + i;
+            S[kb][i] = LOCAL ? (pcol && row == col ? 1.f : 0.f)
+                             : __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                             Rin, 4 * (4 * lg * V + col), 4 * (16 * kb + i) * V, 0));
+        }
+
+    floatx4 rw[CW * NKT], rk[CK * NT], ra[OUT && !ROLES ? CW * NT : 1], rg, u_cur[NT];
+    auto load_k = [&](size_t c) {
 #pragma unroll
-                for (int mt = qt; mt < NT; ++mt) X2[mt] = mfma16(aq[mt][qt][st], X1[qt][st], X2[mt]);
+        for (int i = 0; i < CK * NT; ++i) rk[i] = ld_uni(K4 + c * OPF4 + wave * CK * NT * 64, i * 64 + lane);
     };
+    auto load_gu = [&](size_t c) {
+        if (OUT && !ROLES) load_a(ra, c);
+        rg = ld_uni(G4 + c * (K / 4), lane % (K / 4));
+#pragma unroll
+        for (int mt = 0; mt < NT; ++mt) // (the P slices of pass 1 have no U)
+            u_cur[mt] = pcol ? floatx4{0.f, 0.f, 0.f, 0.f} : ld_uni(U4 + c * uvf4 + (size_t)vt * NT * 64, mt * 64 + lane);
+    };
+    auto split_k = [&]() {
+#pragma unroll
+        for (int i = 0; i < CK; ++i) {
+            const int kb = wave * CK + i;
+            split_row_tile<NT>(&rk[i * NT], &sKd[kb * NT * 64], lane, &eK[16 * kb]);
+        }
+        if (OUT && !ROLES) split_a(ra);
+        if (wave == 0 && lane < K / 4) sGam[lane] = rg;
+    };
+    halfx8 sh[NKT / 2], sl[NKT / 2]; // S as the second operand of phase A, and its columns' inverse scales
+    float es = 0.f;
+    auto split_s = [&]() {
+        es = split_columns<NKT>(S, sh, sl);
+        if (ROLES) {
+#pragma unroll
+            for (int kp = 0; kp < NKT / 2; ++kp) {
+                sS[(wave * NKT + 2 * kp) * 64 + lane] = __builtin_bit_cast(floatx4, sh[kp]);
+                sS[(wave * NKT + 2 * kp + 1) * 64 + lane] = __builtin_bit_cast(floatx4, sl[kp]);
+            }
+            if (lane < 16) eS[wave * 16 + lane] = es;
+        }
+    };
+    if (n1 > n0) {
+        load_rows(W4, rw, cid0 + n0);
+        if (!LATE) load_k(cid0 + n0);
+        load_gu(cid0 + n0);
+        split_rows(rw, sW, eW);
+        split_s();
+    }
+    floatx4 X1[NT], X2[NT]; // chunk n's v_new; its output (K = 256), stored in iteration n + 1
     for (int n = n0; n < n1; ++n) {
         const size_t cid = cid0 + n;
         const size_t cnext = n + 1 < n1 ? cid + 1 : cid;
-        if (OUT && n > n0) phase_d(); // D(n - 1)
-        vm_wait<3>();  // this wave's copies of chunk n's W, q exp(G) have landed (not the 3 touches after them)
-        lds_barrier(); // sW, sQ hold chunk n; every wave is done with sKd, sA (n-1)
-#pragma unroll
-        for (int i = 0; i < PFO; ++i) lds_copy4(&K4[cid * OPF4 + i * NTH + tid], &sKd[i * NTH + wv]);
-        if (OUT) {
-            // A_qk is lower block-triangular: copy i of wave w brings tile
-            // f = NWV i + w = (f / NT, f % NT), copied only on or below the
-            // diagonal (10 of the 16 tiles)
-#pragma unroll
-            for (int i = 0; i < APF; ++i) {
-                const int f = NWV * i + wave;
-                if (f % NT <= f / NT) lds_copy4(&A4[cid * AF4 + i * NTH + tid], &sA[i * NTH + wv]);
-            }
-            if (n > n0) store_out(X2, n - 1);
-        }
-        if (wave == 0 && lane < K / 4) lds_copy4(&G4[cid * (K / 4) + lane], sGam);
-        floatx4 u_cur[NT];
-#pragma unroll
-        for (int mt = 0; mt < NT; ++mt)
-            u_cur[mt] = pcol ? floatx4{0.f, 0.f, 0.f, 0.f} : U4[cid * uvf4 + (size_t)(vt * NT + mt) * 64 + lane];
+        lds_barrier(); // sW holds chunk n's terms; every wave is done with sKd, sA (n-1)
+        if (LATE)
+            load_k(cid);
+        else
+            load_rows(W4, rw, cnext);
+        if (OUT && !ROLES && n > n0) store_out(X2, n - 1);
         if (STATES) { // the state entering chunk n
             size_t slot = cid;
             bool keep = true;
@@ -934,62 +1061,44 @@ __global__ __launch_bounds__(64 * NWV, 1) void chunk_inter_kernel(ChunkParams p,
                         }
             }
         }
-        // keep these loads here, a whole phase ahead of their use and of the
-        // vmcnt wait before the next barrier, and the touches last
-        __builtin_amdgcn_sched_barrier(0);
-        touch_wq(cnext);
-        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_sched_barrier(0); // keep these loads here, a phase ahead of their use
 
-        // A: X1 = W S, X2 = scale (q exp(G)) S
+        // A: X1 = W S (K = 256: and X2 = scale (q exp(G)) S, in f32 from L2)
+        times_s(sW, sh, sl, X1);
+        if (OUT && !ROLES) {
+            floatx4 ma[2][NT];
+            auto load_m = [&](int kb, int bf) {
 #pragma unroll
-        for (int mt = 0; mt < NT; ++mt) X1[mt] = X2[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-        floatx4 wa[2][NT], ma[2][NT];
-        auto load_a = [&](int kb, int bf) {
+                for (int mt = 0; mt < NT; ++mt) ma[bf][mt] = ld_uni(Q4 + cid * OPF4, (mt * NKT + kb) * 64 + lane);
+            };
+            load_m(0, 0);
 #pragma unroll
-            for (int mt = 0; mt < NT; ++mt) {
-                wa[bf][mt] = sW[(mt * NKT + kb) * 64 + lane];
-                if (OUT)
-                    ma[bf][mt] = QLDS ? sQ[(mt * NKT + kb) * 64 + lane] : Q4[cid * OPF4 + (mt * NKT + kb) * 64 + lane];
+            for (int mt = 0; mt < NT; ++mt) X2[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kb = 0; kb < NKT; ++kb) {
+                if (kb + 1 < NKT) load_m(kb + 1, (kb & 1) ^ 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int st = 0; st < 4; ++st)
+#pragma unroll
+                    for (int mt = 0; mt < NT; ++mt) X2[mt] = mfma16(ma[kb & 1][mt][st], S[kb][st], X2[mt]);
             }
-        };
-        load_a(0, 0);
-#pragma unroll
-        for (int kb = 0; kb < NKT; ++kb) {
-            const int cb = kb & 1;
-            // eight (pass 1: four) independent accumulator chains per k-step;
-            // the next step's operands are requested after the first quarter
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-#pragma unroll
-                for (int mt = 0; mt < NT; ++mt) {
-                    X1[mt] = mfma16(wa[cb][mt][st], S[kb][st], X1[mt]);
-                    if (OUT) X2[mt] = mfma16(ma[cb][mt][st], S[kb][st], X2[mt]);
-                }
-                if (st == 0) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (kb + 1 < NKT) load_a(kb + 1, cb ^ 1);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
         }
-        vm_wait<2>();  // this wave's copies of chunk n's Kd, A_qk, exp(G_last) and its U have landed (not the 2 touches)
-        lds_barrier(); // A done everywhere (sW, sQ free); sKd(n), sA(n) visible
-        // exp(G_last) and phase C's first Kd^T tile, requested before the
-        // copies below so that their latency is spent on the copies' issue
-        floatx4 gk[NKT], ka[2][NKT];
-        auto load_c = [&](int tt, int bf) {
-#pragma unroll
-            for (int kb = 0; kb < NKT; ++kb) ka[bf][kb] = sKd[(kb * NT + tt) * 64 + lane];
-        };
-#pragma unroll
-        for (int kb = 0; kb < NKT; ++kb) gk[kb] = sGam[4 * kb + lg]; // rows 16 kb + 4 lg .. + 3
-        load_c(0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-
+        split_k();
         // B: v_new = U - X1 (kept in X1)
 #pragma unroll
-        for (int mt = 0; mt < NT; ++mt) X1[mt] = u_cur[mt] - X1[mt];
+        for (int mt = 0; mt < NT; ++mt) X1[mt] = u_cur[mt] - X1[mt] * (rows_of(eW, mt) * es);
+        halfx8 vh[NT / 2], vl[NT / 2];
+        const float ev = split_columns<NT>(X1, vh, vl);
+        if (ROLES) {
+#pragma unroll
+            for (int tp = 0; tp < NT / 2; ++tp) {
+                sV[(wave * NT + 2 * tp) * 64 + lane] = __builtin_bit_cast(floatx4, vh[tp]);
+                sV[(wave * NT + 2 * tp + 1) * 64 + lane] = __builtin_bit_cast(floatx4, vl[tp]);
+            }
+            if (lane < 16) eV[wave * 16 + lane] = ev;
+        }
+        lds_barrier(); // A done everywhere (sW, sQ free); sKd(n), sA(n) hold their terms
         if (STATES) {
             // row-major rows through a buffer resource over the chunk's rows:
             // token rows [B * HV, T, V] (the resource ends at row T, so rows past T
@@ -1011,53 +1120,48 @@ __global__ __launch_bounds__(64 * NWV, 1) void chunk_inter_kernel(ChunkParams p,
                 for (int mt = 0; mt < NT; ++mt) reinterpret_cast<floatx4 *>(Vn)[(vt * NT + mt) * 64 + lane] = X1[mt];
             }
         }
-
-        // W, q exp(G) of chunk n+1, then the touches of its Kd^T, A_qk, U
-        __builtin_amdgcn_sched_barrier(0);
-        if (n + 1 < n1) {
-#pragma unroll
-            for (int i = 0; i < PFO; ++i) {
-                lds_copy4(&W4[(cid + 1) * OPF4 + i * NTH + tid], &sW[i * NTH + wv]);
-                if (QLDS) lds_copy4(&Q4[(cid + 1) * OPF4 + i * NTH + tid], &sQ[i * NTH + wv]);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        touch_kau(cnext);
+        if (LATE)
+            load_rows(W4, rw, cnext);
+        else
+            load_k(cnext);
+        load_gu(cnext);
         __builtin_amdgcn_sched_barrier(0);
 
-        // C: S = exp(G_last) S + Kd^T v_new
+        // C: S = exp(G_last) S + Kd^T v_new, four chains at a time
 #pragma unroll
-        for (int kb = 0; kb < NKT; ++kb) {
-            S[kb][0] *= gk[kb][0];
-            S[kb][1] *= gk[kb][1];
-            S[kb][2] *= gk[kb][2];
-            S[kb][3] *= gk[kb][3];
-        }
-        __builtin_amdgcn_sched_barrier(0);
+        for (int k4 = 0; k4 < NKT; k4 += 4) {
+            constexpr int KC = NKT < 4 ? NKT : 4;
+            floatx4 d[KC];
+            halfx8 k[KC][NT / 2][2];
 #pragma unroll
-        for (int tt = 0; tt < NT; ++tt) {
-            const int cb = tt & 1;
-            // NKT independent accumulator chains per k-step; the next time
-            // tile's operands are requested after the first quarter
+            for (int i = 0; i < KC; ++i) {
+                d[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int st = 0; st < 4; ++st) {
-#pragma unroll
-                for (int kb = 0; kb < NKT; ++kb) S[kb] = mfma16(ka[cb][kb][st], X1[tt][st], S[kb]);
-                if (st == 0) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (tt + 1 < NT) load_c(tt + 1, cb ^ 1);
-                    else if (OUT) load_aq(); // for D(n), at the top of iteration n + 1
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+                for (int f = 0; f < NT; ++f) k[i][f / 2][f & 1] = half8(sKd, (k4 + i) * NT + f);
             }
-            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int tp = 0; tp < NT / 2; ++tp)
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+#pragma unroll
+                    for (int i = 0; i < KC; ++i) d[i] = mfma32h(k[i][tp][t == 1], t == 2 ? vl[tp] : vh[tp], d[i]);
+#pragma unroll
+            for (int i = 0; i < KC; ++i) {
+                const floatx4 g = sGam[4 * (k4 + i) + lg]; // rows 16 kb + 4 lg .. + 3
+                S[k4 + i] = g * S[k4 + i] + d[i] * (rows_of(eK, k4 + i) * ev);
+            }
+            __builtin_amdgcn_sched_barrier(0); // one group's fragments at a time in registers
         }
+        if (OUT && !ROLES) { // D: out = X2 + A_qk v_new
+            floatx4 y[NT];
+            times_v(vh, vl, y);
+#pragma unroll
+            for (int mt = 0; mt < NT; ++mt) X2[mt] += y[mt] * (rows_of(eA, mt) * ev);
+        }
+        split_rows(rw, sW, eW);
+        split_s();
     }
-    vm_wait0(); // the last touches have landed in sPf
-    if (OUT && n1 > n0) {
-        phase_d();
-        store_out(X2, n1 - 1);
-    }
+    if (OUT && !ROLES && n1 > n0) store_out(X2, n1 - 1);
 
     // leaving state: the final state (last segment), the state entering
     // segment 1 (the split's segment 0), Q_j or P_j (pass 1)
@@ -1075,10 +1179,15 @@ __global__ __launch_bounds__(64 * NWV, 1) void chunk_inter_kernel(ChunkParams p,
         Sout = p.ws_qseg + seg_slot(p, bh, seg + 1) * K * V;
     }
     if (Sout) {
+        const __amdgpu_buffer_rsrc_t R = state_rsrc(Sout, ld);
 #pragma unroll
         for (int kb = 0; kb < NKT; ++kb)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) Sout[(size_t)(16 * kb + 4 * lg + i) * ld + col] = S[kb][i];
+            for (int i = 0; i < 4; ++i) {
+                const float val = S[kb][i]; // (through a scalar, see store_out)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, val), R, 4 * (4 * lg * ld + col),
+                                                      4 * (16 * kb + i) * ld, 0);
+            }
     }
 }
 
@@ -1241,18 +1350,17 @@ __global__ __launch_bounds__(256) void chunk_states_kernel(ChunkParams p) {
 // segments in all, pass 3's workgroups stay those of the uniform run's n, and
 // segment 0's walk takes one value slice per sequence beside pass 1's.
 // Segment 0 gets L0 = r NC / (n + r) chunks and the others L = ceil((NC - L0)
-// / n), so that its walk and pass 1 end together: r = 1.1 where pass 1 runs
-// eight waves over 128 columns, two per SIMD (the fastest of r = 0.5 .. 1.8
-// at B = 1, T = 65536, 16 heads, K = V = 128), else 0.8 (pass 1 cheaper per
-// chunk than the walk; the fastest of 0.6 .. 1.6 at B = 8, T = 4096, 4
-// heads, K = 64, V = 96).  Only where every segment keeps at least
+// / n), so that its walk and pass 1 end together: r = 0.7 (B = 1, T = 32768, 16
+// heads, K = V = 128: 1209 us in all, 1228 at 0.85, 1253 at 1.0, 1291 at 1.2;
+// B = 8, T = 4096, 4 heads, K = 64, V = 96: 242, 244, 247, 249).  Only where
+// every segment keeps at least
 // kMinSplitChunks chunks; else the uniform run.
 constexpr int kMinSplitChunks = 16;
 
-bool split_segments(const ChunkParams &p, bool wide_pass1, ChunkParams *q) {
+bool split_segments(const ChunkParams &p, ChunkParams *q) {
     if (p.NSEG < 2) return false;
     const int n = p.NSEG, NC = p.NC;
-    const double r = wide_pass1 ? 1.1 : 0.8;
+    const double r = 0.7;
     const int L0 = (int)(r * NC / (n + r));
     const int L = (NC - L0 + n - 1) / n;
     const int last = NC - L0 - (n - 1) * L;
@@ -1352,8 +1460,8 @@ size_t half_cu_pad() {
 template <int K, int V, int MODE>
 void launch_inter(const ChunkParams &p, hipStream_t s, int nseg, int seg_base, size_t lds = 0) {
     constexpr int NWV = inter_nwv(K, V), VSW = 16 * NWV;
-    hipLaunchKernelGGL((chunk_inter_kernel<K, MODE, NWV>), dim3(p.B * p.HV * nseg * (V / VSW)), dim3(64 * NWV), lds,
-                       s, p, nseg, seg_base);
+    hipLaunchKernelGGL((chunk_inter_kernel<K, MODE, NWV>), dim3(p.B * p.HV * nseg * (V / VSW)),
+                       dim3(inter_threads(K, MODE, NWV)), lds, s, p, nseg, seg_base);
 }
 
 // phases: 1 intra; 2 inter with the output, 4 training (every segment's P and
@@ -1369,14 +1477,14 @@ hipError_t launch_chunk_t(const ChunkParams &p0, hipStream_t s, int phases) {
     constexpr int NWV = inter_nwv(K, V), VSW = 16 * NWV; // waves and value columns per sequential workgroup
     // Pass 1 (segment summaries: no output, so no q exp(G) or A_qk in LDS) at
     // K = 128 takes 128 columns (V or P) per workgroup of eight waves: the
-    // chunk's W and Kd^T are copied once for twice the columns, and two waves
-    // per SIMD still fit its registers.
+    // chunk's W and Kd^T are loaded and split once for twice the columns, and
+    // two waves per SIMD still fit its registers.
     constexpr int NWL = (K == 128 && V % 128 == 0) ? 8 : NWV, VSWL = 16 * NWL;
     const dim3 blk(64 * NWV), blkl(64 * NWL);
     const int seqs = p0.B * p0.HV;
     const bool infer = (phases & 112) || (phases & 14) == 2;
     ChunkParams ps;
-    const bool split = infer && split_segments(p0, NWL == 8, &ps);
+    const bool split = infer && split_segments(p0, &ps);
     const ChunkParams &p = split ? ps : p0;
     auto summaries = [&](int nl) -> hipError_t { // pass 1 over segments 0 .. nl - 1 (uniform)
         hipLaunchKernelGGL((chunk_inter_kernel<K, kInterLocal, NWL>), dim3(seqs * nl * ((V + K) / VSWL)), blkl, 0, s,

@@ -126,6 +126,105 @@ __device__ __forceinline__ void quad_swap_pairs(floatx4 &x, bool odd) { // odd =
     }
 }
 
+// ---------------------------------------------------------------------------
+// f32 products on the f16 matrix cores, for the sequential kernels: an operand
+// x is taken as two f16 terms of x 2^s,
+//   hi = f16(x 2^s),  lo = f16(x 2^s - hi),
+// and hi hi + hi lo + lo hi accumulated in f32 (the remaining lo lo is below
+// 2^-22 of a product).  s is one exponent per row of the first operand and per
+// column of the second, chosen so that their largest magnitude lies in
+// [2^14, 2^15): 23 bits of every element down to 2^-17 of the largest, and an
+// absolute error of 2^-40 of it below.  A 16x16x32 step takes the fragments
+// of two neighbouring 16x16 tiles of the contraction, k = 4 group + step in
+// each, so that two f32 accumulator tiles are one f16 second operand.  Three
+// such steps (16 cycles each) stand for the eight 16x16x4 f32 steps (32 cycles
+// each) of the same contraction.
+// ---------------------------------------------------------------------------
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef int intx4v __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ floatx4 mfma32h(halfx8 a, halfx8 b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+// The scale 2^s for a largest magnitude mx (1 where it is 0 or not finite;
+// s at most 100, so that the inverse and its product with another stay normal).
+__device__ __forceinline__ float f16_scale(float mx) {
+    const bool ok = mx > 0.f && mx < __builtin_inff();
+    return __builtin_ldexpf(1.f, ok ? min(100, 15 - __builtin_amdgcn_frexp_expf(mx)) : 0);
+}
+// 1 / scale, exactly
+__device__ __forceinline__ float inv_scale(float scale) {
+    return __builtin_bit_cast(float, 0x7F000000u - __builtin_bit_cast(unsigned, scale));
+}
+__device__ __forceinline__ float max4(float m, floatx4 x) {
+    m = fmaxf(fmaxf(m, fabsf(x[0])), fabsf(x[1]));
+    return fmaxf(fmaxf(m, fabsf(x[2])), fabsf(x[3]));
+}
+// Largest over the four lanes l % 16, in all of them.  (The swaps' results go
+// through scalars: a bit_cast of a vector's element reads element 0.)
+__device__ __forceinline__ float max_groups(float m) {
+    const unsigned u = __builtin_bit_cast(unsigned, m);
+    const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const unsigned a0 = a[0], a1 = a[1];
+    m = fmaxf(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
+    const unsigned v = __builtin_bit_cast(unsigned, m);
+    const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    const unsigned b0 = b[0], b1 = b[1];
+    return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
+}
+// Two tiles' four elements each as the two terms of one 32-deep operand: the
+// scaled values rounded in pairs, then their exact remainders rounded by one
+// mixed-precision multiply-add each (v_fma_mixlo/hi_f16).
+__device__ __forceinline__ void split_pair(floatx4 a, floatx4 b, float scale, halfx8 *hi, halfx8 *lo) {
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+        const float x = j < 4 ? a[j & 3] : b[j & 3], y = j < 4 ? a[(j & 3) + 1] : b[(j & 3) + 1];
+        const halfx2 h = __builtin_convertvector(floatx2{x * scale, y * scale}, halfx2);
+        (*hi)[j] = h[0];
+        (*hi)[j + 1] = h[1];
+        (*lo)[j] = (_Float16)__builtin_fmaf(x, scale, -(float)h[0]);
+        (*lo)[j + 1] = (_Float16)__builtin_fmaf(y, scale, -(float)h[1]);
+    }
+}
+// One row tile of a first operand, NF fragments v along the contraction, into
+// LDS as its two terms: of fragments 2 p and 2 p + 1 (64 float4 each from s),
+// the first becomes hi and the second lo of the pair.  Every lane of the wave
+// takes part; ex[l % 16] receives the rows' 2^-s.
+template <int NF> __device__ __forceinline__ void split_row_tile(const floatx4 *v, floatx4 *s, int lane, float *ex) {
+    static_assert(NF % 2 == 0, "pairs of tiles");
+    float mx = 0.f;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) mx = max4(mx, v[f]);
+    const float scale = f16_scale(max_groups(mx));
+#pragma unroll
+    for (int f = 0; f < NF; f += 2) {
+        halfx8 hi, lo;
+        split_pair(v[f], v[f + 1], scale, &hi, &lo);
+        s[f * 64 + lane] = __builtin_bit_cast(floatx4, hi);
+        s[(f + 1) * 64 + lane] = __builtin_bit_cast(floatx4, lo);
+    }
+    if (lane < 16) ex[lane] = inv_scale(scale);
+}
+// An accumulator column block as the second operand: T tiles of 16 rows.
+// Returns the column's 2^-s.
+template <int T> __device__ __forceinline__ float split_columns(const floatx4 *x, halfx8 *hi, halfx8 *lo) {
+    float mx = 0.f;
+#pragma unroll
+    for (int t = 0; t < T; ++t) mx = max4(mx, x[t]);
+    const float scale = f16_scale(max_groups(mx));
+#pragma unroll
+    for (int t = 0; t < T; t += 2) split_pair(x[t], x[t + 1], scale, &hi[t / 2], &lo[t / 2]);
+    return inv_scale(scale);
+}
+
+// Element idx of a wave-uniform array: one scalar base and a 32-bit offset per
+// lane, where 64-bit lane addresses of many loads would take registers.
+__device__ __forceinline__ floatx4 ld_uni(const floatx4 *base, unsigned idx) {
+    return *reinterpret_cast<const floatx4 *>(reinterpret_cast<const char *>(base) + idx * 16u);
+}
+
 // Direct global -> LDS copy of one float4 per lane (global_load_lds_dwordx4):
 // lane l of the calling wave writes wave_base[l]; wave_base is wave-uniform.
 // The copy counts in vmcnt: wait with vm_wait0() before the barrier that
