@@ -1353,9 +1353,10 @@ __global__ __launch_bounds__(256) void chunk_states_kernel(ChunkParams p) {
 // / n), so that its walk and pass 1 end together: r = 0.7 (B = 1, T = 32768, 16
 // heads, K = V = 128: 1209 us in all, 1228 at 0.85, 1253 at 1.0, 1291 at 1.2;
 // B = 8, T = 4096, 4 heads, K = 64, V = 96: 242, 244, 247, 249).  Only where
-// every segment keeps at least
-// kMinSplitChunks chunks; else the uniform run.
-constexpr int kMinSplitChunks = 16;
+// every segment keeps at least kMinSplitChunks chunks; else the uniform run
+// (16 against 6 chunks: B = 4, T = 2048, 16 heads, K = V = 128 334 against 307
+// us in all, B = 2, T = 3001 with 16 value heads of 256 370 against 329).
+constexpr int kMinSplitChunks = 6;
 
 bool split_segments(const ChunkParams &p, ChunkParams *q) {
     if (p.NSEG < 2) return false;
