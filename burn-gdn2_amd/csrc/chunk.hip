@@ -1195,80 +1195,34 @@ __global__ __launch_bounds__(inter_threads(K, MODE, NWV), 1) void chunk_inter_ke
 // (Q_j from pass 1) <- S_in(j + 1) = P_j S_in(j) + Q_j for j = j0 .. NSEG - 2:
 // in uniform runs j0 = 0 and slot 0 <- S0 first; in the split j0 = 1 and
 // S_in(1) is already in its slot (segment 0's walk left it there).  One
-// workgroup per (b, hv, 64 value columns); S in MFMA accumulators, P_j read
-// as A-operand fragments (lane (g, r): row r of a 16-row tile, columns 4g ..
-// 4g + 3) from L2.
-template <int K, int NWV>
-__global__ __launch_bounds__(64 * NWV, 1) void chunk_chain_kernel(ChunkParams p) {
-    constexpr int NKT = K / 16;
-    const int V = p.V, nvv = V / (16 * NWV);
+// workgroup per (b, hv, 16 value columns), P_j read as A-operand fragments
+// (lane (g, r): row r of a 16-row tile, columns 4g .. 4g + 3).
+template <int K>
+__global__ __launch_bounds__(4 * K) void chunk_chain_kernel(ChunkParams p) {
+    const int V = p.V;
     int bh, vs;
-    inter_block(blockIdx.x, p.B * p.HV, nvv, &bh, &vs);
+    inter_block(blockIdx.x, p.B * p.HV, V / 16, &bh, &vs);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lr = lane & 15, lg = lane >> 4;
-    const int col = 16 * (vs * NWV + wave) + lr;
+    const int col = 16 * vs + lr;
 
     const int j0 = p.SLOT0;
     const float *S0 = j0 ? p.ws_qseg + seg_slot(p, bh, 1) * K * V : p.state + (size_t)bh * K * V;
     float *slot0 = p.ws_qseg + seg_slot(p, bh, j0) * K * V; // the slot of segment j0
-    floatx4 S[NKT];
+    floatx4 S;
 #pragma unroll
-    for (int kb = 0; kb < NKT; ++kb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const size_t o = (size_t)(16 * kb + 4 * lg + i) * V + col;
-            S[kb][i] = S0[o];
-            if (!j0) slot0[o] = S[kb][i];
-        }
-    // Every operand is requested one step ahead of its products: the next
-    // k-block of P_j (two register buffers), the first k-block of P_{j+1} during
-    // the last one of P_j, and Q_{j+1} during the products of step j, so that
-    // a step waits on no memory round trip but its own first one.
-    const int nsteps = p.NSEG - 1 - j0; // step i chains segment j0 + i
-    auto P_of = [&](int i) { return p.ws_pseg + seg_slot(p, bh, j0 + i) * K * K; };
-    auto load_pa = [&](floatx4 *pa, const float *P, int kb) {
-#pragma unroll
-        for (int it = 0; it < NKT; ++it)
-            pa[it] = *reinterpret_cast<const floatx4 *>(P + (size_t)(16 * it + lr) * K + 16 * kb + 4 * lg);
-    };
-    auto load_q = [&](floatx4 *q, int j) { // slot j + 1 (from segment j0's) holds Q_{j0 + j} from pass 1
-        const float *Q = slot0 + (size_t)(j + 1) * K * V;
-#pragma unroll
-        for (int it = 0; it < NKT; ++it)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) q[it][i] = Q[(size_t)(16 * it + 4 * lg + i) * V + col];
-    };
-    floatx4 pa[2][NKT], Nq[NKT];
-    if (nsteps > 0) {
-        load_q(Nq, 0);
-        load_pa(pa[0], P_of(0), 0);
+    for (int i = 0; i < 4; ++i) {
+        const size_t o = (size_t)(16 * wave + 4 * lg + i) * V + col;
+        const float v = S0[o];
+        S[i] = v;
+        if (!j0) slot0[o] = v;
     }
-    for (int j = 0; j < nsteps; ++j) {
-        float *Q = slot0 + (size_t)(j + 1) * K * V;
-        floatx4 N[NKT];
-#pragma unroll
-        for (int it = 0; it < NKT; ++it) N[it] = Nq[it];
-#pragma unroll
-        for (int kb = 0; kb < NKT; ++kb) {
-            const int cb = kb & 1;
-            if (kb + 1 < NKT)
-                load_pa(pa[cb ^ 1], P_of(j), kb + 1);
-            else if (j + 1 < nsteps)
-                load_pa(pa[cb ^ 1], P_of(j + 1), 0);
-            if (kb == 0 && j + 1 < nsteps) load_q(Nq, j + 1);
-#pragma unroll
-            for (int st = 0; st < 4; ++st)
-#pragma unroll
-                for (int it = 0; it < NKT; ++it) N[it] = mfma16(pa[cb][it][st], S[kb][st], N[it]);
-        }
-#pragma unroll
-        for (int it = 0; it < NKT; ++it) {
-            S[it] = N[it];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) Q[(size_t)(16 * it + 4 * lg + i) * V + col] = N[it][i];
-        }
-    }
+    const float *P0 = p.ws_pseg + seg_slot(p, bh, j0) * K * K + (size_t)(16 * wave + lr) * K + 4 * lg;
+    chain_walk<K>( // step i chains segment j0 + i
+        S, p.NSEG - 1 - j0, V, col,
+        [&](int i, int kb) { return *reinterpret_cast<const floatx4 *>(P0 + (size_t)i * K * K + 16 * kb); },
+        [&](int i) { return slot0 + (size_t)(i + 1) * K * V; });
 }
 
 // The states at the boundaries of caller chunks of Cc = p.st_cc tokens (Cc <
@@ -1503,7 +1457,7 @@ hipError_t launch_chunk_t(const ChunkParams &p0, hipStream_t s, int phases) {
             });
     };
     auto chain = [&]() -> hipError_t {
-        hipLaunchKernelGGL((chunk_chain_kernel<K, NWV>), dim3(seqs * (V / VSW)), blk, 0, s, p);
+        hipLaunchKernelGGL((chunk_chain_kernel<K>), dim3(seqs * (V / 16)), dim3(4 * K), 0, s, p);
         return hipGetLastError();
     };
     auto output_pass = [&]() -> hipError_t { // pass 3 (split: segments 1 .. NSEG - 1)

@@ -373,57 +373,36 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd_inter_kernel(BwdParams bp, int
 // Pass 2 of the segmented reverse recurrence.  ws_rseg holds NSEG slots of
 // K x V per (b, hv): slot NSEG-1 <- d_state_out (or 0), then slot j - 1 (R_j
 // from pass 1) <- P_j^T slot j + R_j for j = NSEG-1 .. 1: the gradient leaving
-// every segment.  Same MFMA layout as the forward's chunk_chain_kernel, with
-// P_j^T's A fragments gathered from the forward's row-major P_j.
-template <int K, int NW>
-__global__ __launch_bounds__(64 * NW, 1) void bwd_chain_kernel(BwdParams bp) {
+// every segment.  The forward's chain with P_j^T's A fragments gathered from
+// its row-major P_j.
+template <int K>
+__global__ __launch_bounds__(4 * K) void bwd_chain_kernel(BwdParams bp) {
     const ChunkParams &p = bp.f;
-    constexpr int NKT = K / 16;
-    const int V = p.V, nvv = V / (16 * NW);
+    const int V = p.V, nlast = p.NSEG - 1;
     int bh, vs;
-    inter_block(blockIdx.x, p.B * p.HV, nvv, &bh, &vs);
+    inter_block(blockIdx.x, p.B * p.HV, V / 16, &bh, &vs);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lr = lane & 15, lg = lane >> 4;
-    const int col = 16 * (vs * NW + wave) + lr;
+    const int col = 16 * vs + lr;
     float *slot0 = bp.ws_rseg + (size_t)bh * p.NSEG * K * V;
-    float *last = slot0 + (size_t)(p.NSEG - 1) * K * V;
-    floatx4 S[NKT];
+    float *last = slot0 + (size_t)nlast * K * V;
+    floatx4 S;
 #pragma unroll
-    for (int kb = 0; kb < NKT; ++kb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const size_t o = (size_t)(16 * kb + 4 * lg + i) * V + col;
-            S[kb][i] = bp.d_state_out ? bp.d_state_out[(size_t)bh * K * V + o] : 0.f;
-            last[o] = S[kb][i];
-        }
-    for (int j = p.NSEG - 1; j >= 1; --j) {
-        const float *P = p.ws_pseg + ((size_t)bh * p.NSEG + j) * K * K; // P_j, row-major
-        float *Q = slot0 + (size_t)(j - 1) * K * V;
-        floatx4 N[NKT];
-#pragma unroll
-        for (int it = 0; it < NKT; ++it)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) N[it][i] = Q[(size_t)(16 * it + 4 * lg + i) * V + col];
-#pragma unroll
-        for (int kb = 0; kb < NKT; ++kb) {
-            floatx4 pa[NKT];
-#pragma unroll
-            for (int it = 0; it < NKT; ++it) // P_j^T[16 it + lr][16 kb + 4 lg + st] = P_j[16 kb + 4 lg + st][16 it + lr]
-#pragma unroll
-                for (int st = 0; st < 4; ++st) pa[it][st] = P[(size_t)(16 * kb + 4 * lg + st) * K + 16 * it + lr];
-#pragma unroll
-            for (int st = 0; st < 4; ++st)
-#pragma unroll
-                for (int it = 0; it < NKT; ++it) N[it] = mfma16(pa[it][st], S[kb][st], N[it]);
-        }
-#pragma unroll
-        for (int it = 0; it < NKT; ++it) {
-            S[it] = N[it];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) Q[(size_t)(16 * it + 4 * lg + i) * V + col] = N[it][i];
-        }
+    for (int i = 0; i < 4; ++i) {
+        const size_t o = (size_t)(16 * wave + 4 * lg + i) * V + col;
+        const float v = bp.d_state_out ? bp.d_state_out[(size_t)bh * K * V + o] : 0.f;
+        S[i] = v;
+        last[o] = v;
     }
+    const float *P0 = p.ws_pseg + (size_t)bh * p.NSEG * K * K + 16 * wave + lr;
+    chain_walk<K>( // step i applies P_j^T, j = NSEG - 1 - i: element (16 w + lr, 16 kb + 4 lg + st) = P_j[16 kb + 4 lg + st][16 w + lr]
+        S, nlast, V, col,
+        [&](int i, int kb) {
+            const float *P = P0 + (size_t)(nlast - i) * K * K + (size_t)(16 * kb + 4 * lg) * K;
+            return floatx4{P[0], P[K], P[2 * K], P[3 * K]};
+        },
+        [&](int i) { return slot0 + (size_t)(nlast - 1 - i) * K * V; });
 }
 
 // ---------------------------------------------------------------------------
@@ -1073,7 +1052,7 @@ hipError_t launch_bwd_t(const BwdParams &bp, hipStream_t s) {
         hipLaunchKernelGGL((bwd_inter_kernel<K, kRevLocal, NW>), dim3(seqs * (p.NSEG - 1) * (V / VSW)), dim3(64 * NW),
                            0, s, bp, 1, p.NSEG - 1);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        hipLaunchKernelGGL((bwd_chain_kernel<K, NW>), dim3(seqs * (V / VSW)), dim3(64 * NW), 0, s, bp);
+        hipLaunchKernelGGL((bwd_chain_kernel<K>), dim3(seqs * (V / 16)), dim3(4 * K), 0, s, bp);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     hipLaunchKernelGGL((bwd_inter_kernel<K, kRevOut, NW>), dim3(seqs * p.NSEG * (V / VSW)), dim3(64 * NW), 0, s, bp,

@@ -279,6 +279,57 @@ __device__ __forceinline__ void inter_block(int blk, int nseq, int nvs, int *bh,
     }
 }
 
+// The chain of the segmented passes, X <- P_i X + Q_i for i = 0 .. nsteps - 1,
+// on a workgroup of K / 16 waves that owns 16 value columns of one sequence:
+// wave w holds rows 16 w .. of X, and the waves exchange X through LDS between
+// steps.  The steps are a serial chain, so what counts is one step: K / 4
+// dependent products a wave and one barrier.  A wave's rows of P_{i+1} and Q_{i+1} are
+// requested as those of step i are used, and land during it.  Against a wave
+// that walks all rows of its columns ((K / 16)^2 x 4 products a step): the
+// forward's chain at T = 32768, 16 heads, K = V = 128 (12 segments) 76 -> 26
+// us, at T = 1024, 4 heads of 64 13.4 -> 6.7; B = 4, T = 2048, 16 heads of
+// 128 (one step) 27 -> 15 forward, 32 -> 12 backward.
+// load(i, kb): this lane's A fragment of P_i, row tile w, columns 16 kb ..;
+// slot(i): where Q_i lies and X of step i goes, row-major with row length V.
+template <int K, class Load, class Slot>
+__device__ __forceinline__ void chain_walk(floatx4 x, int nsteps, int V, int col, Load load, Slot slot) {
+    constexpr int NKT = K / 16;
+    __shared__ floatx4 sX[2][NKT * 64];
+    const int lane = threadIdx.x & 63, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const size_t o = (size_t)(16 * wave + 4 * lg) * V + col;
+    floatx4 pa[NKT], q = {};
+    auto load_q = [&](int i) {
+        const float *Q = slot(i) + o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) q[r] = Q[(size_t)r * V];
+    };
+    if (nsteps > 0) {
+#pragma unroll
+        for (int kb = 0; kb < NKT; ++kb) pa[kb] = load(0, kb);
+        load_q(0);
+    }
+    sX[0][wave * 64 + lane] = x;
+    for (int i = 0; i < nsteps; ++i) {
+        lds_barrier(); // X of step i - 1 is whole; the buffer that step i - 2 was read from is free
+        const floatx4 *X = sX[i & 1];
+        const int nx = min(i + 1, nsteps - 1); // (the last step's requests are not used)
+        x = q;
+        load_q(nx);
+#pragma unroll
+        for (int kb = 0; kb < NKT; ++kb) {
+            const floatx4 b = X[kb * 64 + lane];
+#pragma unroll
+            for (int st = 0; st < 4; ++st) x = mfma16(pa[kb][st], b[st], x);
+            pa[kb] = load(nx, kb);
+        }
+        sX[(i & 1) ^ 1][wave * 64 + lane] = x;
+        float *Q = slot(i) + o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Q[(size_t)r * V] = x[r];
+    }
+}
+
 // Host side of the chunked forward, shared with the backward (chunk.hip).
 gdn2_status chunk_setup(const gdn2_chunk_args *a, const char *who, bool need_out, ChunkParams *p);
 size_t chunk_fwd_ws_bytes(const gdn2_chunk_args *a);
