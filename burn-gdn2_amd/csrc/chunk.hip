@@ -38,6 +38,7 @@
 // state S and v_new therefore never leave registers.
 #include "chunk_common.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 namespace gdn2 {
@@ -1571,18 +1572,23 @@ struct WsLayout {
 // segment's transition, the chain) costs little beside the shorter walk: at
 // 4 value heads x 16 chunks (hidden 256, K = V = 64) chunk-inter takes 57 us
 // in 4 segments against 79 us in one.
+// For K <= 128 a segment keeps 2 chunks where that makes at most 8 segments: a
+// step of a short chain costs less than the chunks it saves.  In all,
+// forward / training pair, 4 against 2 chunks: T = 1024, 4 heads of 64 50.5
+// against 45.0 / 139 against 117 us, T = 512 47.4 against 42.5 / 128 against
+// 103, B = 4, T = 512, 4 heads of 128 76 against 65 / 225 against 187; with
+// more segments B = 2, T = 2048, 2 heads, V = 96 (16) 56.0 against 58.0, T =
+// 4096, 4 heads of 128 (32) 112 against 138; K = 256 (T = 1024, 8 heads) 166
+// against 184; below 8 chunks (T = 300) one segment, 36.8 against 42.4.  Not where the workspace would then outgrow the no-allocation entry's
+// scratch, so that that entry's range does not depend on this rule.
 constexpr int64_t kInterWorkgroups = 256;
-constexpr int64_t kMinSegmentChunks = 4;
+constexpr int64_t kMinSegmentChunks = 4, kMinShortSegmentChunks = 2, kMaxShortSegments = 8;
 
 struct Segments {
     int nseg, segl;
 };
 
-Segments inter_segments(int64_t B, int64_t HV, int64_t K, int64_t V, int64_t NC) {
-    const int64_t w = (K > 0 && V > 0) ? B * HV * (V / (16 * inter_nwv((int)K, (int)V))) : 0;
-    if (w <= 0 || NC <= 0) return {1, (int)NC}; // (K, V) outside the chunk kernels, or no tokens
-    int64_t n = kInterWorkgroups / w;
-    if (n > NC / kMinSegmentChunks) n = NC / kMinSegmentChunks;
+Segments segments_of(int64_t n, int64_t NC) { // n segments of equal length, the last one shorter
     if (n < 2) return {1, (int)NC};
     const int64_t L = (NC + n - 1) / n;
     return {(int)((NC + L - 1) / L), (int)L};
@@ -1590,9 +1596,8 @@ Segments inter_segments(int64_t B, int64_t HV, int64_t K, int64_t V, int64_t NC)
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
-WsLayout ws_layout(int64_t seqs, int64_t NC, int64_t K, int64_t V) {
+WsLayout ws_layout(int64_t seqs, int64_t NC, int64_t K, int64_t V, int64_t nseg) {
     const int64_t nchunks = seqs * NC;
-    const int64_t nseg = inter_segments(seqs, 1, K, V, NC).nseg;
     const int64_t np = nseg > 1 ? seqs * nseg : 0, nq = np;
     WsLayout L;
     size_t off = 0;
@@ -1608,8 +1613,23 @@ WsLayout ws_layout(int64_t seqs, int64_t NC, int64_t K, int64_t V) {
     return L;
 }
 
+Segments inter_segments(int64_t B, int64_t HV, int64_t K, int64_t V, int64_t NC) {
+    const int64_t w = (K > 0 && V > 0) ? B * HV * (V / (16 * inter_nwv((int)K, (int)V))) : 0;
+    if (w <= 0 || NC <= 0) return {1, (int)NC}; // (K, V) outside the chunk kernels, or no tokens
+    const int64_t fill = kInterWorkgroups / w;
+    const int64_t n = std::min(fill, NC / kMinSegmentChunks);
+    const int64_t ns = std::min({fill, NC / kMinShortSegmentChunks, kMaxShortSegments});
+    if (K <= 128 && NC >= 2 * kMinSegmentChunks && ns > n) {
+        const Segments sg = segments_of(ns, NC);
+        if (ws_layout(B * HV, NC, K, V, sg.nseg).total <= kNoallocScratchBytes) return sg;
+    }
+    return segments_of(n, NC);
+}
+
 WsLayout ws_layout(const gdn2_chunk_args *a) {
-    return ws_layout(a->batch * a->num_v_heads, (a->seq_len + kChunk - 1) / kChunk, a->head_dim, a->head_v_dim);
+    const int64_t seqs = a->batch * a->num_v_heads, NC = (a->seq_len + kChunk - 1) / kChunk;
+    return ws_layout(seqs, NC, a->head_dim, a->head_v_dim,
+                     inter_segments(seqs, 1, a->head_dim, a->head_v_dim, NC).nseg);
 }
 
 bool aligned16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }

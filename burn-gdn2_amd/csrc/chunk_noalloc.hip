@@ -21,9 +21,10 @@
 #include <string>
 
 #include "common.hpp"
+#include "kernels.hpp"
 
 namespace {
-constexpr size_t kScratchBytes = size_t(64) << 20; // 64 MiB per GPU
+constexpr size_t kScratchBytes = gdn2::kNoallocScratchBytes;
 constexpr int kMaxDevices = 64;
 }  // namespace
 

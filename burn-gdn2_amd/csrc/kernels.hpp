@@ -174,6 +174,7 @@ struct ConvBwdParams {
 };
 
 constexpr int kChunk = 64; // chunk length of the kernels (four 16-row tiles)
+constexpr size_t kNoallocScratchBytes = size_t(64) << 20; // the no-allocation forward's array, per GPU
 
 size_t project_lds_bytes(int kd);
 hipError_t launch_project(const ProjectParams &p, hipStream_t s);
