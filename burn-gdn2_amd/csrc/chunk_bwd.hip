@@ -63,18 +63,25 @@ __device__ __forceinline__ floatx4 mfma4x(floatx4 a, floatx4 b, floatx4 c) {
 }
 
 // ---------------------------------------------------------------------------
-// Reverse recurrence.  One workgroup per (b, hv, 16 NW value columns), wave w
-// owns 16 columns; dS' stays in MFMA accumulators (key rows x 16 columns).
-// NW = 4, or 2 where V is not a multiple of 64 (V = 32, 96) and for K = 32,
-// as in the forward's chunk-inter.
+// Reverse recurrence.  One workgroup per (b, hv, 16 NW value columns); dS'
+// stays in accumulators (key rows x 16 columns).  NW = 4, or 2 where V is not
+// a multiple of 64 (V = 32, 96) and for K = 32, as in the forward's chunk-inter.
 // Per chunk n, last to first:
-//   1: dv_new = A_qk^T dO + Kd dS'         (reads sAT, sKd)
+//   1: dv_new = A_qk^T dO + Kd dS'
 //      dS' and dv_new go to the workspace for the per-chunk kernels
-//   2: dS' <- e^{G_last} dS' + QG^T dO - W^T dv_new   (reads sQT, sWT)
-// The operands are A-operand fragments written by the training forward, so
-// every product has the shape of the forward's chunk-inter products.  As
-// there, each LDS buffer is refilled by direct copies while the other phase
-// runs, behind fence-free barriers that wait only for those copies.
+//   2: dS' <- e^{G_last} dS' + QG^T dO - W^T dv_new
+// The products run on the f16 matrix cores, every operand as two f16 terms per
+// row or column scale.  What bounds the walk is one chunk's serial work: loads,
+// splitting, LDS reads and products of a wave one after the other.  So each
+// column tile has two waves: a state wave takes what hangs on dS' (Kd dS',
+// W^T dv_new, the update), and an output-gradient wave computes A_qk^T dO of
+// chunk n - 1 and QG^T dO of chunk n beside it and hands them over in LDS.
+// An operand is split once, by row tiles shared out over the waves of its
+// role, during the phase before its use; its loads are issued a phase earlier
+// still.  B = 4, T = 2048, 16 heads, K = V = 128: 174 us with f32 products in
+// one wave a column tile, 140 now (0.48 GB, 92 us at the card's copy rate);
+// the half of it that pass 1 walks 137 -> 104; K = 64, V = 96, T = 1999 79 -> 48
+// and 70 -> 44.
 //
 // Segmented form (NSEG > 1), the mirror of the forward's: over a segment the
 // map from the gradient leaving it to the gradient entering it is affine,
@@ -87,32 +94,25 @@ __device__ __forceinline__ floatx4 mfma4x(floatx4 a, floatx4 b, floatx4 c) {
 // ---------------------------------------------------------------------------
 constexpr int kRevOut = 0, kRevLocal = 1;
 
+// K = 256: no LDS left for a third operand, the terms handed over and a second
+// wave per column tile.  f32 products, one wave per column tile; QG^T, whose
+// product feeds only dS (not the dS -> dv_new chain), is read from L2.  The
+// operands are A-operand fragments written by the training forward; each LDS
+// buffer is refilled by direct copies while the other phase runs, behind
+// fence-free barriers that wait only for those copies.
 template <int K, int MODE, int NW>
-__global__ __launch_bounds__(64 * NW, 1) void bwd_inter_kernel(BwdParams bp, int seg0, int nseg_launch) {
+__global__ __launch_bounds__(64 * NW, 1) void bwd_inter_wide_kernel(BwdParams bp, int seg0, int nseg_launch) {
     const ChunkParams &p = bp.f;
     constexpr bool LOCAL = MODE == kRevLocal;
     constexpr int NTH = 64 * NW, NKT = K / 16;
     constexpr int OPF4 = NKT * NT * 64, PFO = OPF4 / NTH;
     constexpr int AF4 = NT * NT * 64, APF = AF4 / NTH;
     static_assert(OPF4 % NTH == 0 && AF4 % NTH == 0, "K");
-    // K = 256: Kd and W^T take 64 KiB of LDS each, so (scale q e^G)^T, whose
-    // product QG^T dO feeds only dS (not the dS -> dv_new chain), is read from
-    // L2 into registers in phase 2 instead of through a third LDS buffer.
-    constexpr bool QLDS = K <= 128;
-    __shared__ floatx4 sKd[OPF4], sAT[AF4], sQT[QLDS ? OPF4 : 1], sWT[OPF4];
+    __shared__ floatx4 sKd[OPF4], sAT[AF4], sWT[OPF4];
     __shared__ float sPf[256]; // destination of the L2 touches, never read
-    // e^{G_last} of the chunk, copied with the Q^T / W^T operands and read
-    // in phase 2: one copy for the workgroup instead of every wave's loads
+    // e^{G_last} of the chunk, copied with the W^T operand and read in phase
+    // 2: one copy for the workgroup instead of every wave's loads
     __shared__ floatx4 sGam[K / 4];
-    // K = 128: the chunk's d_out rows of the workgroup's 16 NW columns,
-    // double-buffered, copied with Kd and A_qk^T (16-byte copies, a quarter of
-    // the vector memory instructions of per-lane row loads), in the LDS left
-    // beside its one workgroup per CU.  K = 256 has none left, and at K <= 64
-    // they would cost a second workgroup per CU: those load them into registers.
-    constexpr bool DOLDS = K == 128;
-    constexpr int VSW = 16 * NW, DOF4 = C * VSW / 4, DOPF = DOF4 / NTH;
-    static_assert(DOF4 % NTH == 0, "d_out block");
-    __shared__ floatx4 sDO[DOLDS ? 2 : 1][DOLDS ? DOF4 : 1];
 
     const int V = p.V, nvv = V / (16 * NW);
     int sq, vs;
@@ -173,9 +173,8 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd_inter_kernel(BwdParams bp, int
         }
     };
     // chunk n's rows of d_out through a buffer resource over its valid rows
-    // (rows past T read 0).  Registers: row 4 lg of each 16-row tile, the rest
-    // of the row offset wave-uniform.  LDS: the block [C][VSW] row-major in
-    // buffer n & 1, thread tid's float4 i at index i * NTH + tid.
+    // (rows past T read 0): row 4 lg of each 16-row tile, the rest of the row
+    // offset wave-uniform
     const float *dob = bp.d_out + (int64_t)bi * p.sob + (int64_t)hv * p.soh;
     const int ro = (int)p.sot, dol = 4 * lg * ro + col;
     auto load_dO = [&](floatx4 *dO, int n) {
@@ -185,30 +184,11 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd_inter_kernel(BwdParams bp, int
 #pragma unroll
             for (int i = 0; i < 4; ++i) dO[mt][i] = bld1(R, dol + (16 * mt + i) * ro);
     };
-    const int col0 = 16 * vs * NW; // the workgroup's first column
-    auto copy_dO = [&](int n) {
-        const __amdgpu_buffer_rsrc_t R = rows_rsrc(dob + (int64_t)n * C * p.sot, ro, min(C, p.T - n * C), V);
-#pragma unroll
-        for (int i = 0; i < DOPF; ++i) {
-            const int f = i * NTH + tid, row = f / (VSW / 4), c4 = f % (VSW / 4);
-            lds_copy4_rsrc(R, 4 * (row * ro + col0 + 4 * c4), &sDO[n & 1][i * NTH + wv]);
-        }
-    };
-    auto read_dO = [&](floatx4 *dO, int n) { // this lane's B-fragment values from the block
-        const float *blk = reinterpret_cast<const float *>(sDO[n & 1]);
-#pragma unroll
-        for (int mt = 0; mt < NT; ++mt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) dO[mt][i] = blk[(16 * mt + 4 * lg + i) * VSW + 16 * wave + lr];
-    };
 
     floatx4 dO[NT]; // rows of d_out of the current chunk, loaded a phase ahead
     if (n1 > n0) {
         copy_ka(cid0 + n1 - 1);
-        if constexpr (DOLDS)
-            copy_dO(n1 - 1);
-        else
-            load_dO(dO, n1 - 1);
+        load_dO(dO, n1 - 1);
         __builtin_amdgcn_sched_barrier(0);
         touch_qw(cid0 + n1 - 1);
         __builtin_amdgcn_sched_barrier(0);
@@ -219,14 +199,10 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd_inter_kernel(BwdParams bp, int
 
     for (int n = n1 - 1; n >= n0; --n) {
         const size_t cid = cid0 + n;
-        vm_wait<2>();  // this wave's copies of Kd, A_qk^T (n) and its dO rows have landed (not the last 2 touches)
-        lds_barrier(); // sKd, sAT hold chunk n; every wave is done with sQT, sWT (n+1)
-        if constexpr (DOLDS) read_dO(dO, n); // used from the end of phase 1 on
+        vm_wait<2>();  // this wave's copies of Kd, A_qk^T (n) have landed (not the last 2 touches)
+        lds_barrier(); // sKd, sAT hold chunk n; every wave is done with sWT (n+1)
 #pragma unroll
-        for (int i = 0; i < PFO; ++i) {
-            if (QLDS) lds_copy4(&QT4[cid * OPF4 + i * NTH + tid], &sQT[i * NTH + wv]);
-            lds_copy4(&WT4[cid * OPF4 + i * NTH + tid], &sWT[i * NTH + wv]);
-        }
+        for (int i = 0; i < PFO; ++i) lds_copy4(&WT4[cid * OPF4 + i * NTH + tid], &sWT[i * NTH + wv]);
         if (!LOCAL) { // dL/d(state leaving chunk n)
             float *Dsn = bp.ws_dsn + cid * K * V;
 #pragma unroll
@@ -276,18 +252,15 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd_inter_kernel(BwdParams bp, int
 #pragma unroll
                     for (int st = 0; st <= rt; ++st) dvn[st] = mfma16(at[st][rt][j], dO[rt][j], dvn[st]);
         }
-        vm_wait0();    // this wave's copies of QT, WT (n) and its e^{G_last} have landed
-        lds_barrier(); // phase 1 done everywhere (sKd, sAT free); sQT, sWT (n) visible
+        vm_wait0();    // this wave's copies of WT (n) and its e^{G_last} have landed
+        lds_barrier(); // phase 1 done everywhere (sKd, sAT free); sWT (n) visible
 
         // Kd, A_qk^T and the dO rows of chunk n - 1; dv_new to the workspace
         floatx4 dO_next[NT];
         __builtin_amdgcn_sched_barrier(0);
         if (n > n0) {
             copy_ka(cid - 1);
-            if constexpr (DOLDS)
-                copy_dO(n - 1); // into the other buffer: every wave read this one after the last barrier
-            else
-                load_dO(dO_next, n - 1);
+            load_dO(dO_next, n - 1);
         }
         if (!LOCAL) {
             float *Dvn = bp.ws_dvn + cid * C * V;
@@ -325,7 +298,7 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd_inter_kernel(BwdParams bp, int
             auto load_qw = [&](int tt, int bf) {
 #pragma unroll
                 for (int kb = 0; kb < NKT; ++kb) {
-                    qa[bf][kb] = QLDS ? sQT[(kb * NT + tt) * 64 + lane] : QT4[cid * OPF4 + (kb * NT + tt) * 64 + lane];
+                    qa[bf][kb] = QT4[cid * OPF4 + (kb * NT + tt) * 64 + lane];
                     wa[bf][kb] = sWT[(kb * NT + tt) * 64 + lane];
                 }
             };
@@ -349,7 +322,7 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd_inter_kernel(BwdParams bp, int
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (!DOLDS && n > n0) {
+        if (n > n0) {
 #pragma unroll
             for (int mt = 0; mt < NT; ++mt) dO[mt] = dO_next[mt];
         }
@@ -367,6 +340,280 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd_inter_kernel(BwdParams bp, int
         for (int kb = 0; kb < NKT; ++kb)
 #pragma unroll
             for (int i = 0; i < 4; ++i) out[(size_t)(16 * kb + 4 * lg + i) * V + col] = dS[kb][i];
+    }
+}
+
+// K <= 128 (see above): the terms of all operands in LDS, two waves per column
+// tile.
+template <int K, int MODE, int NW>
+__global__ __launch_bounds__(128 * NW, 1) void bwd_inter_kernel(BwdParams bp, int seg0, int nseg_launch) {
+    const ChunkParams &p = bp.f;
+    constexpr bool LOCAL = MODE == kRevLocal;
+    constexpr int NKT = K / 16, OPF4 = NKT * NT * 64, AF4 = NT * NT * 64;
+    static_assert(NT % NW == 0 && NKT % NW == 0, "row tiles per wave");
+    constexpr int CW = NT / NW, CK = NKT / NW; // row tiles a wave loads and splits: of Kd, A_qk^T; of W^T, QG^T
+    __shared__ floatx4 sKd[OPF4], sWT[OPF4], sQT[OPF4];
+    __shared__ floatx4 sAT[12 * 64]; // A_qk^T by pairs of tiles on or above the diagonal
+    __shared__ floatx4 sZ[NW * NT * 64], sY[NW * NKT * 64]; // A_qk^T dO, QG^T dO of the column tiles
+    __shared__ floatx4 sGam[K / 4];                         // e^{G_last} of the chunk
+    __shared__ __align__(16) float eKd[C], eAT[C], eQT[K], eWT[K]; // inverse scales of the rows (split_row_tile)
+
+    const int V = p.V, nvv = V / (16 * NW);
+    int sq, vs;
+    inter_block(blockIdx.x, p.B * p.HV * nseg_launch, nvv, &sq, &vs);
+    const int bh = sq / nseg_launch, seg = seg0 + sq % nseg_launch;
+    const int bi = bh / p.HV, hv = bh % p.HV;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = wid % NW; // this wave's column tile
+    const int lr = lane & 15, lg = lane >> 4;
+    const int vt = vs * NW + wave, col = 16 * vt + lr;
+    const int n0 = seg * p.SEGL, n1 = min(p.NC, n0 + p.SEGL);
+
+    const floatx4 *__restrict__ KD4 = reinterpret_cast<const floatx4 *>(p.ws_kd);
+    const floatx4 *__restrict__ AT4 = reinterpret_cast<const floatx4 *>(p.ws_aqkt);
+    const floatx4 *__restrict__ QT4 = reinterpret_cast<const floatx4 *>(p.ws_qgt);
+    const floatx4 *__restrict__ WT4 = reinterpret_cast<const floatx4 *>(p.ws_wt);
+    const floatx4 *__restrict__ G4 = reinterpret_cast<const floatx4 *>(p.ws_gam);
+    const size_t cid0 = (size_t)bh * p.NC;
+    auto rows_of = [&](const float *e, int tile) { return *reinterpret_cast<const floatx4 *>(&e[16 * tile + 4 * lg]); };
+    auto half8 = [&](const floatx4 *s, int f) { return __builtin_bit_cast(halfx8, s[f * 64 + lane]); };
+    // row tiles of a key-row operand (QG^T, W^T) through registers into its terms in LDS
+    auto load_key = [&](const floatx4 *src, floatx4 *r, size_t c) {
+#pragma unroll
+        for (int i = 0; i < CK * NT; ++i) r[i] = ld_uni(src + c * OPF4 + wave * CK * NT * 64, i * 64 + lane);
+    };
+    auto split_key = [&](const floatx4 *r, floatx4 *s, float *e) {
+#pragma unroll
+        for (int i = 0; i < CK; ++i) {
+            const int kb = wave * CK + i;
+            split_row_tile<NT>(&r[i * NT], &s[kb * NT * 64], lane, &e[16 * kb]);
+        }
+    };
+    // rows of a key-row operand times C x 16 terms, four row tiles (chains) at a time; f(kb, product before scales)
+    auto times_t = [&](const floatx4 *s, const halfx8 *hi, const halfx8 *lo, auto f) {
+        constexpr int KC = NKT < 4 ? NKT : 4;
+#pragma unroll
+        for (int k4 = 0; k4 < NKT; k4 += 4) {
+            floatx4 d[KC];
+            halfx8 k[KC][NT / 2][2];
+#pragma unroll
+            for (int i = 0; i < KC; ++i) {
+                d[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int t = 0; t < NT; ++t) k[i][t / 2][t & 1] = half8(s, (k4 + i) * NT + t);
+            }
+#pragma unroll
+            for (int tp = 0; tp < NT / 2; ++tp)
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+#pragma unroll
+                    for (int i = 0; i < KC; ++i) d[i] = mfma32h(k[i][tp][t == 1], t == 2 ? lo[tp] : hi[tp], d[i]);
+#pragma unroll
+            for (int i = 0; i < KC; ++i) f(k4 + i, d[i]);
+            __builtin_amdgcn_sched_barrier(0); // one group's fragments at a time in registers
+        }
+    };
+
+    if (wid >= NW) { // the output-gradient wave of a column tile (every barrier has its twin below)
+        if (n1 <= n0) return;
+        // this lane's column of chunk n's rows of d_out, through a buffer
+        // resource over its valid rows (rows past T read 0)
+        const float *dob = bp.d_out + (int64_t)bi * p.sob + (int64_t)hv * p.soh;
+        const int ro = (int)p.sot, dol = 4 * lg * ro + col;
+        auto load_dO = [&](floatx4 *dO, int n) {
+            const __amdgpu_buffer_rsrc_t R = rows_rsrc(dob + (int64_t)n * C * p.sot, ro, min(C, p.T - n * C), V);
+#pragma unroll
+            for (int mt = 0; mt < NT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) dO[mt][i] = bld1(R, dol + (16 * mt + i) * ro);
+        };
+        const auto at_first = [](int st) { return st < 2 ? 4 * st : 4 + 2 * st; }; // row tile st's first fragment in sAT
+        auto load_at = [&](floatx4 *r, size_t c) { // upper block-triangular: tiles (st, rt >= st) only
+#pragma unroll
+            for (int i = 0; i < CW * NT; ++i) {
+                const int st = wave * CW + i / NT, rt = i % NT;
+                r[i] = rt >= st ? ld_uni(AT4 + c * AF4 + st * NT * 64, rt * 64 + lane) : floatx4{0.f, 0.f, 0.f, 0.f};
+            }
+        };
+        auto split_at = [&](const floatx4 *r) {
+#pragma unroll
+            for (int i = 0; i < CW; ++i) {
+                const int st = wave * CW + i;
+                floatx4 *d = &sAT[at_first(st) * 64];
+                if (st < 2)
+                    split_row_tile<4>(&r[i * NT], d, lane, &eAT[16 * st]);
+                else
+                    split_row_tile<2>(&r[i * NT + 2], d, lane, &eAT[16 * st]);
+            }
+        };
+        halfx8 oh[NT / 2], ol[NT / 2]; // dO of a chunk and its columns' inverse scale
+        float eo = 0.f;
+        auto products_z = [&]() {
+            floatx4 z[NT];
+#pragma unroll
+            for (int st = 0; st < NT; ++st) z[st] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int tp = 0; tp < NT / 2; ++tp)
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+#pragma unroll
+                    for (int st = 0; st < 2 * tp + 2; ++st) // (row tiles 2, 3 hold the second pair only)
+                        z[st] = mfma32h(half8(sAT, at_first(st) + (st < 2 ? 2 * tp : 0) + (t == 1)), t == 2 ? ol[tp] : oh[tp],
+                                        z[st]);
+#pragma unroll
+            for (int st = 0; st < NT; ++st) sZ[(wave * NT + st) * 64 + lane] = z[st] * (rows_of(eAT, st) * eo);
+        };
+        floatx4 rq[CK * NT], ra[CW * NT], dO[NT];
+        auto at_or_first = [&](int n) { return max(n, n0); };
+        load_at(ra, cid0 + n1 - 1);
+        load_key(QT4, rq, cid0 + n1 - 1);
+        load_dO(dO, n1 - 1);
+        split_at(ra);
+        load_at(ra, cid0 + at_or_first(n1 - 2));
+        split_key(rq, sQT, eQT);
+        eo = split_columns<NT>(dO, oh, ol);
+        load_dO(dO, at_or_first(n1 - 2));
+        lds_barrier(); // sAT holds the last chunk's terms
+        products_z();
+        for (int n = n1 - 1; n >= n0; --n) {
+            lds_barrier(); // sQT and sZ of chunk n are there
+            load_key(QT4, rq, cid0 + at_or_first(n - 1));
+            __builtin_amdgcn_sched_barrier(0); // keep these loads here, a phase ahead of their use
+            times_t(sQT, oh, ol, [&](int kb, floatx4 d) { sY[(wave * NKT + kb) * 64 + lane] = d * (rows_of(eQT, kb) * eo); });
+            split_at(ra); // of chunk n - 1
+            lds_barrier(); // sY of chunk n, sAT of chunk n - 1 are there; sQT, sZ are free
+            load_at(ra, cid0 + at_or_first(n - 2));
+            __builtin_amdgcn_sched_barrier(0);
+            eo = split_columns<NT>(dO, oh, ol);
+            load_dO(dO, at_or_first(n - 2));
+            __builtin_amdgcn_sched_barrier(0);
+            products_z();
+            split_key(rq, sQT, eQT);
+        }
+        return;
+    }
+
+    // the gradient leaving the segment: d_state_out (one segment), the chained
+    // gradient (pass 3) or 0 (pass 1)
+    // (row terms are wave-uniform offsets in a buffer resource: no registers held across the loop)
+    floatx4 dS[NKT];
+    const float *din = nullptr;
+    if (!LOCAL)
+        din = p.NSEG > 1      ? bp.ws_rseg + ((size_t)bh * p.NSEG + seg) * K * V
+              : bp.d_state_out ? bp.d_state_out + (size_t)bh * K * V
+                               : nullptr;
+    auto state_rsrc = [&](const float *base, int bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), (short)0, bytes, 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t Rin = state_rsrc(din, din ? K * V * 4 : 0); // without a gradient every load reads 0
+#pragma unroll
+    for (int kb = 0; kb < NKT; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            dS[kb][i] = LOCAL ? 0.f
+                              : __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                              Rin, 4 * (4 * lg * V + col), 4 * (16 * kb + i) * V, 0));
+
+    floatx4 rk[CW * NKT], rw[CK * NT], rg;
+    auto load_kd = [&](size_t c) {
+#pragma unroll
+        for (int i = 0; i < CW * NKT; ++i) rk[i] = ld_uni(KD4 + c * OPF4 + wave * CW * NKT * 64, i * 64 + lane);
+    };
+    auto split_kd = [&]() {
+#pragma unroll
+        for (int i = 0; i < CW; ++i) {
+            const int st = wave * CW + i;
+            split_row_tile<NKT>(&rk[i * NKT], &sKd[st * NKT * 64], lane, &eKd[16 * st]);
+        }
+    };
+    halfx8 sh[NKT / 2], sl[NKT / 2]; // dS' and its columns' inverse scales
+    float es = 0.f;
+    if (n1 > n0) {
+        load_kd(cid0 + n1 - 1);
+        load_key(WT4, rw, cid0 + n1 - 1);
+        rg = ld_uni(G4 + (cid0 + n1 - 1) * (K / 4), lane % (K / 4));
+        split_kd();
+        es = split_columns<NKT>(dS, sh, sl);
+        lds_barrier();
+    }
+    for (int n = n1 - 1; n >= n0; --n) {
+        const size_t cid = cid0 + n, cnext = cid0 + max(n - 1, n0);
+        lds_barrier(); // sKd, sZ hold chunk n; every wave is done with sWT, sY (n + 1)
+        load_kd(cnext);
+        if (!LOCAL) { // dL/d(state leaving chunk n)
+            floatx4 *Dsn = reinterpret_cast<floatx4 *>(bp.ws_dsn + cid * K * V) + vt * NKT * 64;
+#pragma unroll
+            for (int kb = 0; kb < NKT; ++kb) Dsn[kb * 64 + lane] = dS[kb];
+        }
+        __builtin_amdgcn_sched_barrier(0); // keep these loads here, a phase ahead of their use
+
+        // 1: dv_new = Kd dS' + A_qk^T dO
+        floatx4 dvn[NT];
+#pragma unroll
+        for (int st = 0; st < NT; ++st) dvn[st] = floatx4{0.f, 0.f, 0.f, 0.f};
+        {
+            halfx8 w[2][NT][2]; // a step's operands are read during the step before it
+            auto fetch = [&](int kp) {
+#pragma unroll
+                for (int st = 0; st < NT; ++st)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) w[kp & 1][st][h] = half8(sKd, st * NKT + 2 * kp + h);
+            };
+            fetch(0);
+#pragma unroll
+            for (int kp = 0; kp < NKT / 2; ++kp) {
+                if (kp + 1 < NKT / 2) fetch(kp + 1);
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+#pragma unroll
+                    for (int st = 0; st < NT; ++st)
+                        dvn[st] = mfma32h(w[kp & 1][st][t == 1], t == 2 ? sl[kp] : sh[kp], dvn[st]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        split_key(rw, sWT, eWT);
+        if (wave == 0 && lane < K / 4) sGam[lane] = rg;
+#pragma unroll
+        for (int st = 0; st < NT; ++st)
+            dvn[st] = sZ[(wave * NT + st) * 64 + lane] + dvn[st] * (rows_of(eKd, st) * es);
+        halfx8 vh[NT / 2], vl[NT / 2];
+        const float ev = split_columns<NT>(dvn, vh, vl);
+        lds_barrier(); // sKd, sZ free; sWT, sY and e^{G_last} of chunk n are there
+        if (!LOCAL) {
+            floatx4 *Dvn = reinterpret_cast<floatx4 *>(bp.ws_dvn + cid * C * V) + vt * NT * 64;
+#pragma unroll
+            for (int st = 0; st < NT; ++st) Dvn[st * 64 + lane] = dvn[st];
+        }
+        load_key(WT4, rw, cnext);
+        rg = ld_uni(G4 + cnext * (K / 4), lane % (K / 4));
+        __builtin_amdgcn_sched_barrier(0);
+
+        // 2: dS' <- e^{G_last} dS' + QG^T dO - W^T dv_new
+        times_t(sWT, vh, vl, [&](int kb, floatx4 d) {
+            const floatx4 g = sGam[4 * kb + lg]; // rows 16 kb + 4 lg .. + 3
+            dS[kb] = (g * dS[kb] + sY[(wave * NKT + kb) * 64 + lane]) - d * (rows_of(eWT, kb) * ev);
+        });
+        split_kd();
+        es = split_columns<NKT>(dS, sh, sl);
+    }
+    // the gradient entering the segment: dS0 (first segment) or R_j (pass 1)
+    float *out = nullptr;
+    if (!LOCAL) {
+        if (seg == 0) out = bp.d_state0 + (size_t)bh * K * V;
+    } else {
+        out = bp.ws_rseg + ((size_t)bh * p.NSEG + seg - 1) * K * V;
+    }
+    if (out) {
+        const __amdgpu_buffer_rsrc_t R = state_rsrc(out, K * V * 4);
+#pragma unroll
+        for (int kb = 0; kb < NKT; ++kb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float val = dS[kb][i]; // through a scalar: a bit_cast of the element lvalue reads element 0
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, val), R, 4 * (4 * lg * V + col),
+                                                      4 * (16 * kb + i) * V, 0);
+            }
     }
 }
 
@@ -1048,16 +1295,21 @@ hipError_t launch_bwd_t(const BwdParams &bp, hipStream_t s) {
     static_assert(V % VSW == 0, "V");
     const int seqs = p.B * p.HV, nch = seqs * p.NC;
     hipError_t e;
+    auto inter = [&](auto mode, int seg, int nseg) {
+        const dim3 grid(seqs * nseg * (V / VSW));
+        if constexpr (K <= 128)
+            hipLaunchKernelGGL((bwd_inter_kernel<K, decltype(mode)::value, NW>), grid, dim3(128 * NW), 0, s, bp, seg, nseg);
+        else
+            hipLaunchKernelGGL((bwd_inter_wide_kernel<K, decltype(mode)::value, NW>), grid, dim3(64 * NW), 0, s, bp, seg,
+                               nseg);
+        return hipGetLastError();
+    };
     if (p.NSEG > 1) {
-        hipLaunchKernelGGL((bwd_inter_kernel<K, kRevLocal, NW>), dim3(seqs * (p.NSEG - 1) * (V / VSW)), dim3(64 * NW),
-                           0, s, bp, 1, p.NSEG - 1);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if ((e = inter(std::integral_constant<int, kRevLocal>{}, 1, p.NSEG - 1)) != hipSuccess) return e;
         hipLaunchKernelGGL((bwd_chain_kernel<K>), dim3(seqs * (V / 16)), dim3(4 * K), 0, s, bp);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((bwd_inter_kernel<K, kRevOut, NW>), dim3(seqs * p.NSEG * (V / VSW)), dim3(64 * NW), 0, s, bp,
-                       0, p.NSEG);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = inter(std::integral_constant<int, kRevOut>{}, 0, p.NSEG)) != hipSuccess) return e;
     hipLaunchKernelGGL((bwd_vprod_kernel<K, V>), dim3(nch), dim3(256), 0, s, bp);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL((bwd_decay_kernel<K, V>), dim3(nch), dim3(K * 4), 0, s, bp);

@@ -143,7 +143,6 @@ __device__ __forceinline__ void quad_swap_pairs(floatx4 &x, bool odd) { // odd =
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef int intx4v __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ floatx4 mfma32h(halfx8 a, halfx8 b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -232,12 +231,6 @@ __device__ __forceinline__ floatx4 ld_uni(const floatx4 *base, unsigned idx) {
 __device__ __forceinline__ void lds_copy4(const floatx4 *src, floatx4 *wave_base) {
     __builtin_amdgcn_global_load_lds(static_cast<const void *>(src),
                                      (__attribute__((address_space(3))) void *)(wave_base), 16, 0, 0);
-}
-// The same copy through a buffer resource (buffer_load_dwordx4 ... lds): the
-// range check zero-fills the lanes whose 16 bytes at byte offset `off` lie
-// past the resource, e.g. the rows past T of a rows_rsrc.
-__device__ __forceinline__ void lds_copy4_rsrc(__amdgpu_buffer_rsrc_t r, int off, floatx4 *wave_base) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)(wave_base), 16, off, 0, 0, 0);
 }
 // Pulls the 128-byte line holding `line` toward this XCD's L2: a 4-byte copy
 // into the calling lane's word of wave_slot (64 floats per wave, never read).

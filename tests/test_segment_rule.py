@@ -117,3 +117,33 @@ def test_forward_scales_with_the_values(gpu, K, V, size):
         big = np.abs(ref).max(axis=(0, 1, 2))  # per value column
         err = np.abs(got - ref).max(axis=(0, 1, 2))
         assert (err <= tol * big).all(), (err / np.maximum(big, 1e-300)).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,V,T", [(32, 64, 130), (64, 64, 64), (64, 96, 700), (128, 128, 65), (128, 192, 1030),
+                                   (256, 128, 70)])
+@pytest.mark.parametrize("size", [1e-12, 1.0, 1e9])
+def test_gradients_scale_with_the_output_gradient(gpu, K, V, T, size):
+    """The reverse walk splits d_out, dS' and dv_new likewise: dv, dw and dS0
+    are linear in a column of (d_out, d_state), so columns of very different
+    sizes, and zero ones, keep their own relative error."""
+    import torch
+
+    import gdn2_amd
+
+    B, H = 1, 2
+    rng = np.random.default_rng(K + V + T)
+    q, k, v, g, b, w = rand_inputs(rng, B, H, H, T, K, V, g_lo=-0.05, g_hi=-0.001)
+    S0 = rng.standard_normal((B, H, K, V)).astype(np.float32)
+    col = np.float32(size) * np.float32(2.0) ** rng.integers(-20, 21, V).astype(np.float32)
+    col[:: 7] = 0.0
+    dO = (rng.standard_normal((B, H, T, V)) * col).astype(np.float32)
+    dST = (rng.standard_normal((B, H, K, V)) * col).astype(np.float32)
+    ref = O.recurrent_bwd_f64(q, k, v, g, b, w, dO, S0=S0, d_ST=dST, scale=0.1)
+    ref = ref if isinstance(ref, dict) else dict(zip(("dq", "dk", "dg", "db", "dv", "dw", "dS0"), ref))
+    d = [torch.from_numpy(x).to(gpu) for x in (q, k, v, g, b, w, S0, dO, dST)]
+    got = gdn2_amd.chunk_wy_backward(*d[:8], 0.1, 64, d_state=d[8])
+    tol = 16 * (64 + K) * EPS  # as above for gradients
+    for n in ("dv", "dw", "dS0"):
+        err = np.abs(got[n].cpu().numpy() - ref[n]).max(axis=(0, 1, 2))
+        assert (err <= tol * np.abs(ref[n]).max(axis=(0, 1, 2))).all(), n
