@@ -1569,9 +1569,7 @@ struct WsLayout {
 // that the output pass runs about one workgroup per compute unit (an MI355X
 // has 256); a segment keeps at least 4 chunks.  The split only binds where
 // the sequences leave most of the chip idle, so the extra passes' work (each
-// segment's transition, the chain) costs little beside the shorter walk: at
-// 4 value heads x 16 chunks (hidden 256, K = V = 64) chunk-inter takes 57 us
-// in 4 segments against 79 us in one.
+// segment's transition, the chain) costs little beside the shorter walk.
 // For K <= 128 a segment keeps 2 chunks where that makes at most 8 segments: a
 // step of a short chain costs less than the chunks it saves.  In all,
 // forward / training pair, 4 against 2 chunks: T = 1024, 4 heads of 64 50.5
@@ -1626,6 +1624,23 @@ Segments inter_segments(int64_t B, int64_t HV, int64_t K, int64_t V, int64_t NC)
     return segments_of(n, NC);
 }
 
+// Workspace of a sequence of NC chunks.  Short segments make their count fall
+// at some longer lengths (8 chunks: four segments, 9 chunks: three), so the
+// size also covers every shorter length whose segments are short: a workspace
+// for the longest sequence serves the shorter ones.  (A segment's P and entering
+// state are at most 1.1 times a chunk's operands, and 8 segments the most:
+// lengths further below than 8 chunks need less.)
+size_t ws_bytes(int64_t seqs, int64_t NC, int64_t K, int64_t V) {
+    size_t most = ws_layout(seqs, NC, K, V, inter_segments(seqs, 1, K, V, NC).nseg).total;
+    const int64_t last = K <= 128 ? std::min(NC - 1, kMinSegmentChunks * kMaxShortSegments - 1) : 0;
+    for (int64_t m = std::max(2 * kMinSegmentChunks, NC - 8); m <= last; ++m)
+        most = std::max(most, ws_layout(seqs, m, K, V, inter_segments(seqs, 1, K, V, m).nseg).total);
+    return most;
+}
+size_t ws_bytes(const gdn2_chunk_args *a) {
+    return ws_bytes(a->batch * a->num_v_heads, (a->seq_len + kChunk - 1) / kChunk, a->head_dim, a->head_v_dim);
+}
+
 WsLayout ws_layout(const gdn2_chunk_args *a) {
     const int64_t seqs = a->batch * a->num_v_heads, NC = (a->seq_len + kChunk - 1) / kChunk;
     return ws_layout(seqs, NC, a->head_dim, a->head_v_dim,
@@ -1639,7 +1654,7 @@ bool aligned16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u
 extern "C" size_t gdn2_chunk_workspace_bytes(const gdn2_chunk_args *a) {
     if (!a || a->batch <= 0 || a->num_v_heads <= 0 || a->seq_len <= 0 || a->head_dim <= 0 || a->head_v_dim <= 0)
         return 0;
-    return ws_layout(a).total;
+    return ws_bytes(a);
 }
 
 namespace gdn2 {
@@ -1692,7 +1707,7 @@ gdn2_status chunk_setup(const gdn2_chunk_args *a, const char *who, bool need_out
     return GDN2_OK;
 }
 
-size_t chunk_fwd_ws_bytes(const gdn2_chunk_args *a) { return ws_layout(a).total; }
+size_t chunk_fwd_ws_bytes(const gdn2_chunk_args *a) { return ws_bytes(a); }
 
 int chunk_segments(int64_t seqs, int64_t K, int64_t V, int64_t NC) { return inter_segments(seqs, 1, K, V, NC).nseg; }
 
