@@ -10,7 +10,7 @@ kernels) over all 8 x 16 x 4096 token-heads, inputs already resident in
 HBM.  The projected operands (q, k, g, b, v, w) come from the layer's own
 project() once, outside the timed region.
 
-Also reported: the whole layer (hipBLASLt Linear layers + kernels) for the
+Also reported: the whole layer (Linear layers + kernels) for the
 same prefill; B = 64 fused decode (short conv + gates + L2 norm + step +
 gated RMSNorm per token), the kernel alone over 256 tokens with 5 rotating
 state buffers (335 MB, larger than the 256 MB MALL; the kernel's time does
@@ -253,6 +253,7 @@ def bench_prefill(torch, G, args, dev):
     tokens = B * T
     intra_gflop = B * H * T * 2 * C * (3 * K + V) / 1e9
     inter_gflop = B * H * T * (6 * K * V + 2 * C * V) / 1e9
+    # (chunk-inter's f32 products run as three f16 ones each: its fraction of the f32 peak may pass 1)
     kernels = {
         "chunk_intra": {"ms": intra_ms, "ms_median": _median(intra_all), "gflop": intra_gflop,
                         "tflops": intra_gflop / intra_ms, "frac_f32_mfma": intra_gflop / intra_ms / PEAK_F32_TFLOPS},

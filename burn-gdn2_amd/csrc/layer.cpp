@@ -1,7 +1,8 @@
 // The GDN-2 layer on the device: Gdn2Config checks, parameter initialisation,
 // GatedDeltaNet2::{project, forward, forward_train} and Gdn2State
-// (src/config.rs, src/module.rs), driving rocBLAS for the Linear layers and
-// the HIP kernels of this library for everything else.
+// (src/config.rs, src/module.rs), with the Linear layers through Gemm (blas.hpp:
+// split products on the f16 matrix cores, hipBLASLt for small shapes) and the
+// HIP kernels of this library for everything else.
 //
 // Data flow of one call over M = B * T tokens (all buffers row-major):
 //   Y [M, ld_in] = x W_in            W_in = [q | k | b | v | w | f0 | g0] (one GEMM)
