@@ -173,7 +173,7 @@ GDN2_API gdn2_status gdn2_chunk_inter_f32(const gdn2_chunk_args *args, gdn2_stre
  * the compute units: pass 1 runs every segment but the last from a zero state
  * (its transition and offset), pass 2 chains the segments' entering states,
  * pass 3 re-runs every segment from its entering state and writes out and the
- * final state.  Where those segments are long (16 chunks and more), one more
+ * final state.  Where those segments are long (6 chunks and more), one more
  * segment is cut and segment 0, whose entering state is S0, is walked once
  * with the output during pass 1 (on a second stream the library forks from
  * and joins back to `stream`); passes 2 and 3 then cover the rest.  With one
