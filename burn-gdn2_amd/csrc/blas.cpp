@@ -42,19 +42,6 @@ bool split_pays(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, bool b_kept)
 }
 }
 
-gdn2_status Gemm::ensure_ws(size_t bytes) {
-    if (bytes <= ws_bytes_) return GDN2_OK;
-    if (ws_) {
-        GDN2_HIP_CHECK(hipDeviceSynchronize());
-        GDN2_HIP_CHECK(hipFree(ws_));
-        ws_ = nullptr;
-        ws_bytes_ = 0;
-    }
-    GDN2_HIP_CHECK(hipMalloc(&ws_, bytes));
-    ws_bytes_ = bytes;
-    return GDN2_OK;
-}
-
 gdn2_status Gemm::init() {
     if (hipblasLtCreate(&lt_) != HIPBLAS_STATUS_SUCCESS) return fail(GDN2_EHIP, "hipblasLtCreate failed");
     if (rocblas_create_handle(&rb_) != rocblas_status_success) return fail(GDN2_EHIP, "rocblas_create_handle failed");
@@ -70,12 +57,8 @@ void Gemm::destroy() {
         hipblasLtMatmulDescDestroy(p.desc);
     }
     plans_.clear();
-    if (ws_) (void)hipFree(ws_);
-    ws_ = nullptr;
-    ws_bytes_ = 0;
-    if (sws_) (void)hipFree(sws_);
-    sws_ = nullptr;
-    sws_bytes_ = 0;
+    ws_.destroy();
+    sws_.destroy();
     if (lt_) hipblasLtDestroy(lt_);
     lt_ = nullptr;
     if (rb_) rocblas_destroy_handle(rb_);
@@ -124,15 +107,13 @@ gdn2_status Gemm::plan(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const
     if (hs == HIPBLAS_STATUS_SUCCESS)
         for (int i = 0; i < n && best < 0; ++i)
             if (res[i].state == HIPBLAS_STATUS_SUCCESS && res[i].workspaceSize <= kMaxWorkspace) best = i;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (best >= 0 && n > 1 && hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+    if (best >= 0 && n > 1 && !recording_) {
         // time the candidates on these operands, writing a scratch output
         size_t wsmax = 0;
         for (int i = 0; i < n; ++i)
             if (res[i].state == HIPBLAS_STATUS_SUCCESS && res[i].workspaceSize <= kMaxWorkspace)
                 wsmax = std::max(wsmax, res[i].workspaceSize);
-        gdn2_status st = ensure_ws(wsmax);
-        if (st != GDN2_OK) return st;
+        GDN2_HIP_CHECK(ws_.ensure(wsmax, false));
         float *scratch = nullptr, *flush = nullptr;
         hipEvent_t e0 = nullptr, e1 = nullptr;
         if (M <= kColdTimingMaxM && hipMalloc(&flush, kFlushBytes) != hipSuccess) flush = nullptr;
@@ -149,7 +130,7 @@ gdn2_status Gemm::plan(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const
                     if (flush) ok = launch_cache_sweep(flush, nflush, flush, s) == hipSuccess;
                     if (r > 0) ok = ok && hipEventRecord(e0, s) == hipSuccess;
                     ok = ok && hipblasLtMatmul(lt_, p.desc, &alpha, B, p.la, A, p.lb, &beta, scratch, p.lc, scratch,
-                                               p.lc, &res[i].algo, res[i].workspaceSize ? ws_ : nullptr,
+                                               p.lc, &res[i].algo, res[i].workspaceSize ? ws_.ptr() : nullptr,
                                                res[i].workspaceSize, s) == HIPBLAS_STATUS_SUCCESS;
                     if (r > 0) {
                         float ms = 0.0f;
@@ -200,23 +181,10 @@ bool Gemm::run_split(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const f
     const size_t fa = split_frag_bytes(M, Kd), sa = split_stat_bytes(M);
     const size_t fb = split_frag_bytes(N, Kd), sb = split_stat_bytes(N);
     const size_t need = part + fa + sa + (w ? 0 : fb + sb);
-    const auto capturing = [&] {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
-    };
-    const auto grow = [](void **ptr, size_t bytes) {
-        if (hipMalloc(ptr, bytes) == hipSuccess) return true;
-        *ptr = nullptr;
+    if (recording_ && need > sws_.bytes()) return false;
+    if (sws_.ensure(need, recording_) != hipSuccess) {
         (void)hipGetLastError();
         return false;
-    };
-    if (need > sws_bytes_) {
-        if (capturing()) return false;
-        void *bigger = nullptr;
-        if (!grow(&bigger, need)) return false;
-        if (sws_ && (hipDeviceSynchronize() != hipSuccess || hipFree(sws_) != hipSuccess)) (void)hipGetLastError();
-        sws_ = bigger;
-        sws_bytes_ = need;
     }
     const auto check = [&](hipError_t e) {
         if (e != hipSuccess) *st = fail(GDN2_EHIP, std::string("split product: ") + hipGetErrorString(e));
@@ -224,14 +192,16 @@ bool Gemm::run_split(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const f
     };
     *st = GDN2_OK;
     if (w && !w->frags) {
-        if (capturing()) return false;
         void *buf = nullptr;
-        if (!grow(&buf, fb + sb)) return false;
+        if (recording_ || hipMalloc(&buf, fb + sb) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
         w->frags = buf;
         w->stat = reinterpret_cast<SplitStat *>(static_cast<char *>(buf) + fb);
         if (!check(w->refresh(s))) return true;
     }
-    char *base = static_cast<char *>(sws_);
+    char *base = static_cast<char *>(sws_.ptr());
     p.part = reinterpret_cast<float *>(base);
     void *fra = base + part;
     SplitStat *sta = reinterpret_cast<SplitStat *>(base + part + fa);
@@ -262,9 +232,9 @@ gdn2_status Gemm::run(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const 
     st = plan(ta, tb, M, N, Kd, A, lda, B, ldb, ldc, s, &p);
     if (st != GDN2_OK) return st;
     if (p->ok) {
-        if ((st = ensure_ws(p->ws)) != GDN2_OK) return st;
+        GDN2_HIP_CHECK(ws_.ensure(p->ws, recording_));
         const hipblasStatus_t hs = hipblasLtMatmul(lt_, p->desc, &alpha, B, p->la, A, p->lb, &beta, C, p->lc, C,
-                                                   p->lc, &p->algo, p->ws ? ws_ : nullptr, p->ws, s);
+                                                   p->lc, &p->algo, p->ws ? ws_.ptr() : nullptr, p->ws, s);
         if (hs != HIPBLAS_STATUS_SUCCESS)
             return fail(GDN2_EHIP, "hipblasLtMatmul failed with status " + std::to_string((int)hs));
         return GDN2_OK;

@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "grow_block.hpp"
 #include "split_gemm.hpp"
 
 namespace gdn2 {
@@ -43,6 +44,8 @@ class Gemm {
   public:
     gdn2_status init();
     void destroy();
+    // Whether the products that follow are being captured (said once per layer call).
+    void set_recording(bool r) { recording_ = r; }
     // op(A) [M, Kd]: A stored [M, Kd] (ta = false) or [Kd, M] (ta = true), row stride lda;
     // op(B) [Kd, N]: B stored [Kd, N] (tb = false) or [N, Kd] (tb = true), row stride ldb.
     // w: op(B) as a weight that may keep its split copy (its src and ld are B and ldb).
@@ -63,14 +66,12 @@ class Gemm {
     };
     gdn2_status plan(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const float *A, int64_t lda, const float *B,
                      int64_t ldb, int64_t ldc, hipStream_t s, const Plan **out);
-    gdn2_status ensure_ws(size_t bytes);
     hipblasLtHandle_t lt_ = nullptr;
     rocblas_handle rb_ = nullptr;
     std::vector<Plan> plans_;
-    void *ws_ = nullptr;
-    size_t ws_bytes_ = 0;
-    void *sws_ = nullptr; // split operands and partial sums of one product
-    size_t sws_bytes_ = 0;
+    bool recording_ = false;
+    GrowBlock ws_;  // the library algorithms' workspace
+    GrowBlock sws_; // split operands and partial sums of one product
 };
 
 }  // namespace gdn2

@@ -261,10 +261,8 @@ struct gdn2_layer {
     // Split copies of the Linear weights (blas.hpp), allocated by the first
     // product large enough to use them: W of y = x W, and W^T of dx = dy W^T.
     SplitWeight sw_in, sw_in_t, sw_o, sw_o_t, sw_f1, sw_g1;
-    void *ws = nullptr;
-    size_t ws_bytes = 0;
-    void *bws = nullptr;  // backward workspace, grown on demand
-    size_t bws_bytes = 0;
+    GrowBlock ws;  // workspaces of a call: forward, backward
+    GrowBlock bws;
     mutable HostStage stage; // pinned buffers of the parameter and gradient copies
 
     int64_t col_offset(int id) const {
@@ -343,7 +341,7 @@ gdn2_chunk_args chunk_args_for(const gdn2_layer &L, int64_t B, int64_t T, const 
 }
 
 // Carve the workspace for M = B * T tokens, growing it when needed.
-gdn2_status workspace(gdn2_layer &L, int64_t B, int64_t T, bool need_s0, Work *wk) {
+gdn2_status workspace(gdn2_layer &L, int64_t B, int64_t T, bool need_s0, Work *wk, hipStream_t s) {
     const Dims &d = L.d;
     const int64_t M = B * T;
     Work tmp{};
@@ -354,20 +352,13 @@ gdn2_status workspace(gdn2_layer &L, int64_t B, int64_t T, bool need_s0, Work *w
                      f * M * d.kd, f * M * d.vd, f * M * d.vd, f * M * d.vd,
                      need_s0 ? f * B * d.HV * d.K * d.V : 0};
     size_t total = 0;
-    for (size_t s : sz) total += align256(s);
+    for (size_t n : sz) total += align256(n);
     total += carve_expanded(d, M, nullptr, wk);
     total += align256(chunk_bytes);
-    if (total > L.ws_bytes) {
-        if (L.ws) {
-            GDN2_HIP_CHECK(hipDeviceSynchronize());
-            GDN2_HIP_CHECK(hipFree(L.ws));
-            L.ws = nullptr;
-            L.ws_bytes = 0;
-        }
-        GDN2_HIP_CHECK(hipMalloc(&L.ws, total));
-        L.ws_bytes = total;
-    }
-    char *base = static_cast<char *>(L.ws);
+    const bool recording = stream_recording(s);
+    L.mm.set_recording(recording);
+    GDN2_HIP_CHECK(L.ws.ensure(total, recording));
+    char *base = static_cast<char *>(L.ws.ptr());
     float **dst[10] = {&wk->Y, &wk->F, &wk->G, &wk->q, &wk->k, &wk->g, &wk->b, &wk->v, &wk->w, &wk->O};
     for (int i = 0; i < 10; ++i) {
         *dst[i] = reinterpret_cast<float *>(base);
@@ -590,8 +581,8 @@ extern "C" void gdn2_layer_destroy(gdn2_layer *L) {
     for (SplitWeight *w : {&L->sw_in, &L->sw_in_t, &L->sw_o, &L->sw_o_t, &L->sw_f1, &L->sw_g1}) w->destroy();
     (void)hipFree(L->w_in);
     for (float *p : L->p) (void)hipFree(p);
-    (void)hipFree(L->ws);
-    (void)hipFree(L->bws);
+    L->ws.destroy();
+    L->bws.destroy();
     L->stage.destroy();
     if (prev >= 0) (void)hipSetDevice(prev);
     delete L;
@@ -706,7 +697,7 @@ extern "C" gdn2_status gdn2_layer_forward_train_f32(gdn2_layer *L, const float *
     if (st != GDN2_OK || T == 0) return st;
     hipStream_t s = (hipStream_t)stream;
     Work wk{};
-    if ((st = workspace(*L, B, T, true, &wk)) != GDN2_OK) return st;
+    if ((st = workspace(*L, B, T, true, &wk, s)) != GDN2_OK) return st;
     const int64_t M = B * T;
     if ((st = input_gemms(*L, x, M, wk, s)) != GDN2_OK) return st;
     if ((st = project_epilogue(*L, B, T, nullptr, wk, s)) != GDN2_OK) return st;
@@ -728,7 +719,7 @@ extern "C" gdn2_status gdn2_layer_forward_f32(gdn2_layer *L, const float *x, int
     const Dims &d = L->d;
     const bool sc = L->cfg.use_short_conv != 0;
     Work wk{};
-    if ((st = workspace(*L, B, T, false, &wk)) != GDN2_OK) return st;
+    if ((st = workspace(*L, B, T, false, &wk, s)) != GDN2_OK) return st;
     const int64_t M = B * T;
     // Option::None: S = 0; Gdn2State::zeros caches when the conv does not replace them
     if (!S->some) {
@@ -802,7 +793,7 @@ extern "C" gdn2_status gdn2_layer_project_f32(gdn2_layer *L, const float *x, int
     hipStream_t s = (hipStream_t)stream;
     const Dims &d = L->d;
     Work wk{};
-    if ((st = workspace(*L, B, T, false, &wk)) != GDN2_OK) return st;
+    if ((st = workspace(*L, B, T, false, &wk, s)) != GDN2_OK) return st;
     const int64_t M = B * T;
     if ((st = input_gemms(*L, x, M, wk, s, true)) != GDN2_OK) return st;  // gate out with its bias
     const float *conv_in[3] = {};
@@ -1176,7 +1167,7 @@ struct BwdWork {
     float *part;                  // column-sum partials
 };
 
-gdn2_status bwd_workspace(gdn2_layer &L, int64_t B, int64_t T, bool recompute, BwdWork *bw) {
+gdn2_status bwd_workspace(gdn2_layer &L, int64_t B, int64_t T, bool recompute, BwdWork *bw, hipStream_t s) {
     const Dims &d = L.d;
     const int64_t M = B * T;
     const bool sc = L.cfg.use_short_conv != 0, md = L.cfg.has_min_decay != 0;
@@ -1212,17 +1203,10 @@ gdn2_status bwd_workspace(gdn2_layer &L, int64_t B, int64_t T, bool recompute, B
     };
     size_t total = align256(chunk_bytes);
     for (const Slot &sl : slots) total += align256(sl.bytes);
-    if (total > L.bws_bytes) {
-        if (L.bws) {
-            GDN2_HIP_CHECK(hipDeviceSynchronize());
-            GDN2_HIP_CHECK(hipFree(L.bws));
-            L.bws = nullptr;
-            L.bws_bytes = 0;
-        }
-        GDN2_HIP_CHECK(hipMalloc(&L.bws, total));
-        L.bws_bytes = total;
-    }
-    char *base = static_cast<char *>(L.bws);
+    const bool recording = stream_recording(s);
+    L.mm.set_recording(recording);
+    GDN2_HIP_CHECK(L.bws.ensure(total, recording));
+    char *base = static_cast<char *>(L.bws.ptr());
     bw->fw.chunk = base;
     bw->fw.chunk_bytes = chunk_bytes;
     base += align256(chunk_bytes);
@@ -1309,7 +1293,7 @@ extern "C" gdn2_status gdn2_layer_forward_train_saved_f32(gdn2_layer *L, const f
     }
     hipStream_t s = (hipStream_t)stream;
     Work wk{};
-    if ((st = workspace(*L, B, T, true, &wk)) != GDN2_OK) return st;
+    if ((st = workspace(*L, B, T, true, &wk, s)) != GDN2_OK) return st;
     Work sv = A->fw;
     sv.chunk = wk.chunk;
     sv.chunk_bytes = wk.chunk_bytes;
@@ -1451,7 +1435,7 @@ extern "C" gdn2_status gdn2_layer_backward_f32(gdn2_layer *L, const float *x, in
     }
 
     BwdWork bw{};
-    if ((st = bwd_workspace(*L, B, T, saved == nullptr, &bw)) != GDN2_OK) return st;
+    if ((st = bwd_workspace(*L, B, T, saved == nullptr, &bw, s)) != GDN2_OK) return st;
     if (saved) {  // the forward's buffers come from forward_train_saved
         void *chunk = bw.fw.chunk;
         const size_t chunk_bytes = bw.fw.chunk_bytes;

@@ -20,7 +20,8 @@
  * errors return GDN2_EINVAL with the reference's panic message.  The layer
  * owns its parameters and a workspace in device memory (allocated on the
  * device current at gdn2_layer_create; the workspace grows on the first
- * call at a larger batch x tokens).  x and out are caller-owned device
+ * call at a larger batch x tokens, and a block that a captured graph was
+ * recorded with is kept until gdn2_layer_destroy).  x and out are caller-owned device
  * buffers [B, T, hidden_size], contiguous f32.  Calls are asynchronous on
  * `stream`; calls on one layer must not overlap (they share the workspace).
  */
