@@ -34,8 +34,9 @@
 // MFMA mapping (v_mfma_f32_16x16x4_f32, see common.hpp): an accumulator tile
 // holds rows 4*(lane/16)+i, column lane%16; with the contraction label
 // k = 4*(lane/16) + step inside a 16-wide block it is directly the B operand
-// of the next product.  The solve, A_qk [W|U] and, in the inter kernel, the
-// state S and v_new therefore never leave registers.
+// of the next product.  The solve and A_qk [W|U] therefore never leave
+// registers, nor do, in the inter kernel, the state S and v_new (its output
+// waves get copies in LDS).
 #include "chunk_common.hpp"
 
 #include <algorithm>
@@ -692,24 +693,21 @@ __global__ __launch_bounds__(512, K > 128 ? 2 : 4) void chunk_intra_kernel(Chunk
 //   B: v_new = U - X1
 //   C: S = exp(G_last) S + Kd^T v_new         (reads sKd)
 //   D: out = X2 + A_qk v_new                  (reads sA; independent of C)
-// The products run on the f16 matrix cores, two f16 terms per f32 operand
-// (chunk_common.hpp): as f32 products they took 13.6k of a chunk's 17.2k
-// cycles (K = 128, one wave a SIMD).  Each wave loads its share of W, q exp(G),
-// Kd^T and A_qk as f32 row tiles, half a chunk ahead of their use, finds the
-// rows' scales in registers and writes the terms into LDS, where a chunk of
-// every operand has one buffer: W, q exp(G)(n + 1) while C(n), D(n) run,
-// Kd^T, A_qk(n) while A(n) runs.  S and v_new are split in registers, with a
-// scale per column.
-// What bounds it now: at one wave a SIMD a chunk's 5k cycles of vector
-// instructions (half of them splitting), 2.6k of matrix instructions and 5k of
-// LDS reads ran one after the other, 15k in all; with a state and an output
-// wave per column tile (inter_roles) they overlap, 12k, of which LDS is busy
-// half.  Measured, before -> now: B = 8, T = 4096, 16 heads, K = V = 128 478
-// -> 429 us under the profiler, with chunk-intra 1007 -> 887 us a pass; B = 1,
-// T = 32768 pass 1 (two waves a SIMD) 562 -> 279 us beside the walk, pass 3
-// 529 -> 339 us.
-// Error against f64 (2-norm, outputs and state): unchanged to two digits
-// (2.6e-7).
+// W and q exp(G) of chunk n + 1 come into LDS while C(n), D(n) run, Kd^T and
+// A_qk of chunk n while A(n) runs: one buffer each, with the HBM latency off the
+// sequential path.
+// With the output the products are f32 instructions, and they bound the kernel:
+// 13.6k cycles of a chunk at K = 128, at the 1.8 GHz that the card keeps under
+// them 7.5 of the 7.6 us that a chunk takes.  (Two f16 terms per operand under a
+// scale per row or column took 6.7, but a scale is not causal: a later token
+// 2^24 larger cost the tokens before it their digits.  Three bf16 terms need no
+// scale, but LDS holds f32 operands only, and splitting them in every wave took
+// 9.2 us.)  Measured, one wave per column tile -> a state and an output wave: B =
+// 8, T = 4096, 16 heads, K = V = 128 495 -> 486 us; K = 64, V = 96, training, B =
+// 8, T = 1999, 4 heads 75 -> 54.
+// Pass 1 (below) has no output, and LDS room for its operands' bf16 terms
+// (chunk_common.hpp), split once for 128 columns: B = 1, T = 32768, 16 heads 481
+// -> 342 us beside the split's walk of segment 0.
 //
 // Segmented form (NSEG > 1, few long sequences).  Over one segment the
 // recurrence is affine in its entering state:
@@ -751,11 +749,10 @@ __device__ __forceinline__ size_t seg_slot(const ChunkParams &p, int bh, int j) 
     return (size_t)bh * p.NSLOT + (j - p.SLOT0);
 }
 
-// Waves of a workgroup.  With the output (and K <= 128) each column tile has
-// two: a state wave (A's X1, B, C) and an output wave (A's X2, D, the stores),
-// so that one's matrix instructions, LDS reads and splitting cover the
-// other's waits; the state wave hands S and v_new over in LDS, already as f16
-// terms.  K = 256 has no LDS left for that.
+// Waves of a workgroup (K <= 128).  With the output each column tile has two: a
+// state wave (A's X1, B, C) and an output wave (A's X2, D, the stores), whose
+// products cover each other's LDS reads and waits; the state wave hands S and
+// v_new over in LDS.  Without it there is one.
 constexpr bool inter_roles(int K, int MODE) {
     return (MODE == kInterOut || MODE == kInterOutStates || MODE == kInterOutTrain) && K <= 128;
 }
@@ -768,32 +765,18 @@ __global__ __launch_bounds__(inter_threads(K, MODE, NWV), 1) void chunk_inter_ke
     constexpr bool LOCAL = MODE == kInterLocal;
     constexpr bool STATES = MODE == kInterStates || MODE == kInterOutStates || MODE == kInterOutTrain;
     constexpr bool FRAG = MODE == kInterStates || MODE == kInterOutTrain; // the backward's layouts
-    constexpr bool ROLES = inter_roles(K, MODE);
-    constexpr int VSW = 16 * NWV; // value columns per workgroup
+    constexpr int NTH = inter_threads(K, MODE, NWV), NWS = NTH / 64; // threads and waves per workgroup
+    constexpr int VSW = 16 * NWV;                                    // value columns per workgroup
     constexpr int NKT = K / 16;
-    constexpr int FR = NKT * NT;   // 16x16 fragments per operand per chunk
-    constexpr int OPF4 = FR * 64;  // float4 per operand per chunk
-    static_assert(K % VSW == 0, "K");
-    constexpr int AF4 = NT * NT * 64; // float4 of A_qk per chunk
-    // K = 256: W and Kd^T take 64 KiB each, so scale q exp(G), which feeds only
-    // the output (off the sequential chain), is read from L2 into registers in
-    // phase A instead of through a third LDS buffer, and its product is an f32
-    // one.
-    constexpr bool QLDS = ROLES;
-    // A_qk by pairs of tiles on or below the diagonal: row tiles 0 and 1 hold one, 2 and 3 two
-    constexpr int AFR = 12;
-    __shared__ floatx4 sW[OPF4], sKd[OPF4];
-    __shared__ floatx4 sQ[QLDS ? OPF4 : 1], sA[OUT ? AFR * 64 : 1];
-    __shared__ floatx4 sS[ROLES ? NWV * NKT * 64 : 1], sV[ROLES ? NWV * NT * 64 : 1]; // S, v_new of the column tiles
-    __shared__ float eS[ROLES ? NWV * 16 : 1], eV[ROLES ? NWV * 16 : 1];              // and their columns' inverse scales
-    __shared__ floatx4 sGam[K / 4]; // exp(G_last) of the chunk
-    // inverse scales of the rows of W, q exp(G), Kd^T and A_qk (split_row_tile)
-    __shared__ __align__(16) float eW[C], eQ[QLDS ? C : 4], eK[K], eA[OUT ? C : 4];
-    // A chunk's operands are loaded and split by row tiles: CW row tiles of W,
-    // q exp(G) and A_qk a wave (with eight waves the first four take one each),
-    // CK of Kd^T.
-    constexpr int CW = NWV <= NT ? NT / NWV : 1, CK = NKT / NWV;
-    static_assert(NKT % NWV == 0, "row tiles of Kd^T per wave");
+    constexpr int OPF4 = NKT * NT * 64; // float4 per operand per chunk
+    constexpr int AF4 = NT * NT * 64;   // float4 of A_qk per chunk
+    constexpr int NAT = NT * (NT + 1) / 2; // its tiles on or below the diagonal, (mt, qt) at mt (mt + 1) / 2 + qt
+    constexpr int PAIRS = OPF4 / 128;      // pairs of operand tiles
+    static_assert(OPF4 % NTH == 0 && PAIRS % NWV == 0 && K % VSW == 0, "K");
+    __shared__ floatx4 sW[LOCAL ? 3 * PAIRS * 64 : OPF4], sKd[LOCAL ? 3 * PAIRS * 64 : OPF4]; // terms, or f32
+    __shared__ floatx4 sQ[OUT ? OPF4 : 1], sA[OUT ? NAT * 64 : 1];
+    __shared__ floatx4 sS[OUT ? NWV * NKT * 64 : 1], sV[OUT ? NWV * NT * 64 : 1]; // S, v_new of the column tiles
+    __shared__ floatx4 sGam[K / 4];                                               // exp(G_last) of the chunk
 
     const int V = p.V;
     const int nvv = V / VSW;                    // value slices
@@ -805,10 +788,9 @@ __global__ __launch_bounds__(inter_threads(K, MODE, NWV), 1) void chunk_inter_ke
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6); // wave-uniform (scalar)
     const int wave = wid % NWV;                               // this wave's column tile
-    const bool out_role = ROLES && wid >= NWV;
     const int lr = lane & 15, lg = lane >> 4;
-    const bool pcol = LOCAL && vs >= nvv;          // a slice of P (wave-uniform)
-    const int vt = (pcol ? vs - nvv : vs) * NWV + wave; // this wave's 16-column tile
+    const bool pcol = LOCAL && vs >= nvv;        // a slice of P (wave-uniform)
+    const int vt = (pcol ? vs - nvv : vs) * NWV + wave; // ... in the whole matrix
     const int col = 16 * vt + lr;
     int n0, n1;
     seg_range(p, seg, &n0, &n1);
@@ -822,89 +804,47 @@ __global__ __launch_bounds__(inter_threads(K, MODE, NWV), 1) void chunk_inter_ke
     const size_t cid0 = (size_t)bh * p.NC;
     const size_t uvf4 = (size_t)C * V / 4;
 
-    // This wave's row tiles of the operands, on their way from HBM to LDS: W and
-    // q exp(G) of chunk n + 1 are requested at the start of A(n) (K = 256: of
-    // C(n), for registers) and split into sW, sQ during C(n); Kd^T, A_qk,
-    // exp(G_last) and U of chunk n + 1 at the start of C(n) (K = 256: Kd^T of
-    // chunk n at the start of A(n)), and split into sKd, sA during A(n + 1).
-    // Past the last chunk the current one is taken again.
-    constexpr bool LATE = K > 128;
-    const bool owns_w = NWV <= NT || wave < NT; // (wave-uniform)
-    auto load_rows = [&](const floatx4 *src, floatx4 *r, size_t c) { // W or q exp(G)
+    // W, q exp(G) of chunk n + 1 come into LDS during B-D(n), Kd^T, A_qk and
+    // exp(G_last) of chunk n during A(n).  f32 operands go there straight from
+    // global memory (lds_copy4), all waves taking part.
+    const int wv = 64 * wid;
+    auto copy_wq = [&](size_t c) {
 #pragma unroll
-        for (int i = 0; i < CW * NKT; ++i) r[i] = ld_uni(src + c * OPF4 + (owns_w ? wave : 0) * CW * NKT * 64, i * 64 + lane);
-    };
-    auto split_rows = [&](const floatx4 *r, floatx4 *s, float *e) {
-        if (!owns_w) return;
-#pragma unroll
-        for (int i = 0; i < CW; ++i) {
-            const int mt = wave * CW + i;
-            split_row_tile<NKT>(&r[i * NKT], &s[mt * NKT * 64], lane, &e[16 * mt]);
+        for (int i = 0; i < OPF4 / NTH; ++i) {
+            lds_copy4(&W4[c * OPF4 + i * NTH + tid], &sW[i * NTH + wv]);
+            if (OUT) lds_copy4(&Q4[c * OPF4 + i * NTH + tid], &sQ[i * NTH + wv]);
         }
     };
-    auto load_a = [&](floatx4 *r, size_t c) { // A_qk is lower block-triangular: tiles (mt, qt <= mt) only
+    auto copy_ka = [&](size_t c) {
 #pragma unroll
-        for (int i = 0; i < CW * NT; ++i) {
-            const int mt = wave * CW + i / NT, qt = i % NT;
-            r[i] = qt <= mt ? ld_uni(A4 + c * AF4 + mt * NT * 64, qt * 64 + lane) : floatx4{0.f, 0.f, 0.f, 0.f};
-        }
+        for (int i = 0; i < OPF4 / NTH; ++i) lds_copy4(&K4[c * OPF4 + i * NTH + tid], &sKd[i * NTH + wv]);
+#pragma unroll
+        for (int mt = 0; mt < NT; ++mt)
+#pragma unroll
+            for (int qt = 0; qt <= mt; ++qt) {
+                const int t = mt * (mt + 1) / 2 + qt;
+                if (OUT && t % NWS == wid) lds_copy4(&A4[c * AF4 + (mt * NT + qt) * 64 + lane], &sA[t * 64]);
+            }
+        if (wid == 0 && lane < K / 4) lds_copy4(&G4[c * (K / 4) + lane], sGam);
     };
-    const auto a_first = [](int mt) { return mt < 2 ? 2 * mt : 4 * (mt - 1); }; // row tile mt's first fragment in sA
-    auto split_a = [&](const floatx4 *r) {
+    // Pass 1's operands pass through registers, half a chunk ahead, each wave
+    // splitting PAIRS / NWV pairs of tiles.  Past the last chunk the current
+    // one is loaded again.
+    constexpr int PW = PAIRS / NWV;
+    auto load_op = [&](const floatx4 *src, floatx4 *r, size_t c) {
 #pragma unroll
-        for (int i = 0; i < CW; ++i) {
-            const int mt = wave * CW + i;
-            floatx4 *d = &sA[a_first(mt) * 64];
-            if (mt < 2)
-                split_row_tile<2>(&r[i * NT], d, lane, &eA[16 * mt]);
-            else
-                split_row_tile<4>(&r[i * NT], d, lane, &eA[16 * mt]);
-        }
+        for (int i = 0; i < 2 * PW; ++i) r[i] = ld_uni(src + c * OPF4 + wave * PW * 128, i * 64 + lane);
     };
-    auto rows_of = [&](const float *e, int tile) { return *reinterpret_cast<const floatx4 *>(&e[16 * tile + 4 * lg]); };
-    auto half8 = [&](const floatx4 *s, int f) { return __builtin_bit_cast(halfx8, s[f * 64 + lane]); };
-    // X (+)= T S' for the NT row tiles of a chunk operand in LDS (W or q exp(G))
-    auto times_s = [&](const floatx4 *s, const halfx8 *hi, const halfx8 *lo, floatx4 *X) {
+    auto split_op = [&](const floatx4 *r, floatx4 *s) {
 #pragma unroll
-        for (int mt = 0; mt < NT; ++mt) X[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-        halfx8 w[2][NT][2]; // a step's operands are read during the step before it
-        auto fetch = [&](int kp) {
-#pragma unroll
-            for (int mt = 0; mt < NT; ++mt)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) w[kp & 1][mt][h] = half8(s, mt * NKT + 2 * kp + h);
-        };
-        fetch(0);
-#pragma unroll
-        for (int kp = 0; kp < NKT / 2; ++kp) {
-            if (kp + 1 < NKT / 2) fetch(kp + 1);
-#pragma unroll
-            for (int t = 0; t < 3; ++t) // hi hi, lo hi, hi lo: four independent chains
-#pragma unroll
-                for (int mt = 0; mt < NT; ++mt)
-                    X[mt] = mfma32h(w[kp & 1][mt][t == 1], t == 2 ? lo[kp] : hi[kp], X[mt]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    // y = A_qk v_new
-    auto times_v = [&](const halfx8 *vh, const halfx8 *vl, floatx4 *y) {
-#pragma unroll
-        for (int mt = 0; mt < NT; ++mt) y[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int tp = 0; tp < NT / 2; ++tp)
-#pragma unroll
-            for (int t = 0; t < 3; ++t)
-#pragma unroll
-                for (int mt = 2 * tp; mt < NT; ++mt)
-                    y[mt] = mfma32h(half8(sA, a_first(mt) + 2 * tp + (t == 1)), t == 2 ? vl[tp] : vh[tp], y[mt]);
+        for (int i = 0; i < PW; ++i) put_terms(r[2 * i], r[2 * i + 1], s, wave * PW + i, lane);
     };
 
-    // chunk nn's output rows from X2 through a buffer resource over its valid
-    // rows: rows past T fall outside its range and the hardware drops those
-    // stores, and each store's offset is a per-lane term (row 4 lg of each
-    // 16-row tile, column col) plus a wave-uniform row term, both 32-bit, in
-    // place of 64-bit row addresses.  Needs sot >= V and 63 sot + V < 2^29
-    // (checked on the host).
+    // chunk nn's output rows through a buffer resource over its valid rows:
+    // rows past T fall outside its range and the hardware drops those stores,
+    // and each store's offset is a per-lane term (row 4 lg of each 16-row tile,
+    // column col) plus a wave-uniform row term, both 32-bit, in place of 64-bit
+    // row addresses.  Needs sot >= V and 63 sot + V < 2^29 (checked on the host).
     float *obh = p.out + (int64_t)bi * p.sob + (int64_t)hv * p.soh;
     const int sot = (int)p.sot, olane = 4 * (4 * lg * sot + col);
     auto store_out = [&](const floatx4 *o, int nn) {
@@ -917,45 +857,43 @@ __global__ __launch_bounds__(inter_threads(K, MODE, NWV), 1) void chunk_inter_ke
                 __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, val), R, olane, 4 * (16 * mt + i) * sot, 0);
             }
     };
+    if (!LOCAL && n1 > n0) copy_wq(cid0 + n0);
 
-    if (ROLES && out_role) { // the output wave of a column tile (every barrier below has its twin in the state wave)
+    if (OUT && wid >= NWV) { // the output wave (every barrier below has its twin in the state wave)
         if (n1 <= n0) return;
-        floatx4 rq[QLDS ? CW * NKT : 1], ra[CW * NT], X2[NT];
-        load_rows(Q4, rq, cid0 + n0);
-        load_a(ra, cid0 + n0);
-        split_rows(rq, sQ, eQ);
+        floatx4 X2[NT];
         for (int n = n0; n < n1; ++n) {
-            const size_t cnext = cid0 + (n + 1 < n1 ? n + 1 : n);
-            lds_barrier(); // sQ and S's terms of chunk n are there; the state wave is done with sKd (n-1)
-            load_rows(Q4, rq, cnext);
+            const size_t cid = cid0 + n;
+            vm_wait0();
+            lds_barrier(); // sW, sQ and sS hold chunk n; every wave is done with sKd, sA, sV (n-1)
+            copy_ka(cid);
             if (n > n0) store_out(X2, n - 1);
-            __builtin_amdgcn_sched_barrier(0); // keep these loads here, a phase ahead of their use
-            halfx8 hi[NKT / 2], lo[NKT / 2];
+            floatx4 S[NKT];
 #pragma unroll
-            for (int kp = 0; kp < NKT / 2; ++kp) {
-                hi[kp] = half8(sS, wave * NKT + 2 * kp);
-                lo[kp] = half8(sS, wave * NKT + 2 * kp + 1);
+            for (int kb = 0; kb < NKT; ++kb) S[kb] = sS[(wave * NKT + kb) * 64 + lane];
+            // A: X2 = scale (q exp(G)) S
+#pragma unroll
+            for (int mt = 0; mt < NT; ++mt) X2[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+            products_f32<NT, NKT>(sQ, lane, S, X2);
+            vm_wait0();
+            lds_barrier(); // sQ, sS free; sKd, sA and sV hold chunk n
+            if (n + 1 < n1) copy_wq(cid + 1);
+            // D: out = X2 + A_qk v_new, 16 tokens at a time and on or below the
+            // diagonal: an output row meets no token of a later 16-row tile, and
+            // those after it in its own with exact zeros
+            floatx4 v[NT];
+#pragma unroll
+            for (int qt = 0; qt < NT; ++qt) v[qt] = sV[(wave * NT + qt) * 64 + lane];
+#pragma unroll
+            for (int qt = 0; qt < NT; ++qt) {
+                floatx4 a[NT];
+#pragma unroll
+                for (int mt = qt; mt < NT; ++mt) a[mt] = sA[(mt * (mt + 1) / 2 + qt) * 64 + lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int mt = qt; mt < NT; ++mt) X2[mt] = mfma16(a[mt][i], v[qt][i], X2[mt]);
             }
-            times_s(sQ, hi, lo, X2); // X2 = scale (q exp(G)) S
-            const float es = eS[wave * 16 + lr];
-#pragma unroll
-            for (int mt = 0; mt < NT; ++mt) X2[mt] = X2[mt] * (rows_of(eQ, mt) * es);
-            split_a(ra);
-            lds_barrier(); // sQ free; sA and v_new's terms of chunk n are there
-            load_a(ra, cnext);
-            __builtin_amdgcn_sched_barrier(0);
-            halfx8 vh[NT / 2], vl[NT / 2];
-#pragma unroll
-            for (int tp = 0; tp < NT / 2; ++tp) {
-                vh[tp] = half8(sV, wave * NT + 2 * tp);
-                vl[tp] = half8(sV, wave * NT + 2 * tp + 1);
-            }
-            floatx4 y[NT];
-            times_v(vh, vl, y); // D: out = X2 + A_qk v_new
-            const float ev = eV[wave * 16 + lr];
-#pragma unroll
-            for (int mt = 0; mt < NT; ++mt) X2[mt] += y[mt] * (rows_of(eA, mt) * ev);
-            split_rows(rq, sQ, eQ);
         }
         store_out(X2, n1 - 1);
         return;
@@ -985,58 +923,37 @@ __global__ __launch_bounds__(inter_threads(K, MODE, NWV), 1) void chunk_inter_ke
                              : __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
                                                              Rin, 4 * (4 * lg * V + col), 4 * (16 * kb + i) * V, 0));
         }
-
-    floatx4 rw[CW * NKT], rk[CK * NT], ra[OUT && !ROLES ? CW * NT : 1], rg, u_cur[NT];
-    auto load_k = [&](size_t c) {
+    Terms st[LOCAL ? NKT / 2 : 1]; // S as the second operand of phase A
+    auto pass_s = [&]() {
+        if (OUT)
 #pragma unroll
-        for (int i = 0; i < CK * NT; ++i) rk[i] = ld_uni(K4 + c * OPF4 + wave * CK * NT * 64, i * 64 + lane);
+            for (int kb = 0; kb < NKT; ++kb) sS[(wave * NKT + kb) * 64 + lane] = S[kb];
+        if (LOCAL) split_tiles<NKT>(S, st);
     };
+    floatx4 rw[LOCAL ? 2 * PW : 1], rk[LOCAL ? 2 * PW : 1], rg, u[NT];
     auto load_gu = [&](size_t c) {
-        if (OUT && !ROLES) load_a(ra, c);
-        rg = ld_uni(G4 + c * (K / 4), lane % (K / 4));
+        if (LOCAL) rg = ld_uni(G4 + c * (K / 4), lane % (K / 4));
 #pragma unroll
         for (int mt = 0; mt < NT; ++mt) // (the P slices of pass 1 have no U)
-            u_cur[mt] = pcol ? floatx4{0.f, 0.f, 0.f, 0.f} : ld_uni(U4 + c * uvf4 + (size_t)vt * NT * 64, mt * 64 + lane);
-    };
-    auto split_k = [&]() {
-#pragma unroll
-        for (int i = 0; i < CK; ++i) {
-            const int kb = wave * CK + i;
-            split_row_tile<NT>(&rk[i * NT], &sKd[kb * NT * 64], lane, &eK[16 * kb]);
-        }
-        if (OUT && !ROLES) split_a(ra);
-        if (wave == 0 && lane < K / 4) sGam[lane] = rg;
-    };
-    halfx8 sh[NKT / 2], sl[NKT / 2]; // S as the second operand of phase A, and its columns' inverse scales
-    float es = 0.f;
-    auto split_s = [&]() {
-        es = split_columns<NKT>(S, sh, sl);
-        if (ROLES) {
-#pragma unroll
-            for (int kp = 0; kp < NKT / 2; ++kp) {
-                sS[(wave * NKT + 2 * kp) * 64 + lane] = __builtin_bit_cast(floatx4, sh[kp]);
-                sS[(wave * NKT + 2 * kp + 1) * 64 + lane] = __builtin_bit_cast(floatx4, sl[kp]);
-            }
-            if (lane < 16) eS[wave * 16 + lane] = es;
-        }
+            u[mt] = pcol ? floatx4{0.f, 0.f, 0.f, 0.f} : ld_uni(U4 + c * uvf4 + (size_t)vt * NT * 64, mt * 64 + lane);
     };
     if (n1 > n0) {
-        load_rows(W4, rw, cid0 + n0);
-        if (!LATE) load_k(cid0 + n0);
+        if (LOCAL) {
+            load_op(W4, rw, cid0 + n0);
+            load_op(K4, rk, cid0 + n0);
+            split_op(rw, sW);
+        }
         load_gu(cid0 + n0);
-        split_rows(rw, sW, eW);
-        split_s();
+        pass_s();
     }
-    floatx4 X1[NT], X2[NT]; // chunk n's v_new; its output (K = 256), stored in iteration n + 1
     for (int n = n0; n < n1; ++n) {
-        const size_t cid = cid0 + n;
-        const size_t cnext = n + 1 < n1 ? cid + 1 : cid;
-        lds_barrier(); // sW holds chunk n's terms; every wave is done with sKd, sA (n-1)
-        if (LATE)
-            load_k(cid);
+        const size_t cid = cid0 + n, cnext = n + 1 < n1 ? cid + 1 : cid;
+        if (!LOCAL) vm_wait0();
+        lds_barrier(); // sW (sQ, sS) hold chunk n; every wave is done with sKd (sA, sV) (n-1)
+        if (LOCAL)
+            load_op(W4, rw, cnext);
         else
-            load_rows(W4, rw, cnext);
-        if (OUT && !ROLES && n > n0) store_out(X2, n - 1);
+            copy_ka(cid);
         if (STATES) { // the state entering chunk n
             size_t slot = cid;
             bool keep = true;
@@ -1063,43 +980,34 @@ __global__ __launch_bounds__(inter_threads(K, MODE, NWV), 1) void chunk_inter_ke
             }
         }
         __builtin_amdgcn_sched_barrier(0); // keep these loads here, a phase ahead of their use
-
-        // A: X1 = W S (K = 256: and X2 = scale (q exp(G)) S, in f32 from L2)
-        times_s(sW, sh, sl, X1);
-        if (OUT && !ROLES) {
-            floatx4 ma[2][NT];
-            auto load_m = [&](int kb, int bf) {
+        // A: X1 = W S
+        floatx4 X1[NT];
+        if (LOCAL) {
+            products<NT, NKT / 2>(sW, W4 + cid * OPF4, lane, S, st, X1);
+            split_op(rk, sKd);
+            if (wave == 0 && lane < K / 4) sGam[lane] = rg;
+        } else {
 #pragma unroll
-                for (int mt = 0; mt < NT; ++mt) ma[bf][mt] = ld_uni(Q4 + cid * OPF4, (mt * NKT + kb) * 64 + lane);
-            };
-            load_m(0, 0);
-#pragma unroll
-            for (int mt = 0; mt < NT; ++mt) X2[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kb = 0; kb < NKT; ++kb) {
-                if (kb + 1 < NKT) load_m(kb + 1, (kb & 1) ^ 1);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int st = 0; st < 4; ++st)
-#pragma unroll
-                    for (int mt = 0; mt < NT; ++mt) X2[mt] = mfma16(ma[kb & 1][mt][st], S[kb][st], X2[mt]);
-            }
+            for (int mt = 0; mt < NT; ++mt) X1[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+            products_f32<NT, NKT>(sW, lane, S, X1);
         }
-        split_k();
         // B: v_new = U - X1 (kept in X1)
+        Terms vterms[LOCAL ? NT / 2 : 1];
 #pragma unroll
-        for (int mt = 0; mt < NT; ++mt) X1[mt] = u_cur[mt] - X1[mt] * (rows_of(eW, mt) * es);
-        halfx8 vh[NT / 2], vl[NT / 2];
-        const float ev = split_columns<NT>(X1, vh, vl);
-        if (ROLES) {
-#pragma unroll
-            for (int tp = 0; tp < NT / 2; ++tp) {
-                sV[(wave * NT + 2 * tp) * 64 + lane] = __builtin_bit_cast(floatx4, vh[tp]);
-                sV[(wave * NT + 2 * tp + 1) * 64 + lane] = __builtin_bit_cast(floatx4, vl[tp]);
-            }
-            if (lane < 16) eV[wave * 16 + lane] = ev;
+        for (int mt = 0; mt < NT; ++mt) {
+            X1[mt] = u[mt] - X1[mt];
+            if (OUT) sV[(wave * NT + mt) * 64 + lane] = X1[mt];
         }
-        lds_barrier(); // A done everywhere (sW, sQ free); sKd(n), sA(n) hold their terms
+        if (LOCAL)
+            split_tiles<NT>(X1, vterms);
+        else
+            vm_wait0();
+        lds_barrier(); // A done everywhere (sW, sQ, sS free); sKd (sA, sV) and exp(G_last) hold chunk n
+        if (LOCAL)
+            load_op(K4, rk, cnext);
+        else if (n + 1 < n1)
+            copy_wq(cid + 1);
+        load_gu(cnext);
         if (STATES) {
             // row-major rows through a buffer resource over the chunk's rows:
             // token rows [B * HV, T, V] (the resource ends at row T, so rows past T
@@ -1116,53 +1024,27 @@ __global__ __launch_bounds__(inter_threads(K, MODE, NWV), 1) void chunk_inter_ke
                                                               4 * (16 * mt + i) * V, 0);
                     }
             } else { // tile (value tile, time tile)
-                float *Vn = p.ws_vn + cid * C * V;
+                floatx4 *Vn = reinterpret_cast<floatx4 *>(p.ws_vn + cid * C * V);
 #pragma unroll
-                for (int mt = 0; mt < NT; ++mt) reinterpret_cast<floatx4 *>(Vn)[(vt * NT + mt) * 64 + lane] = X1[mt];
+                for (int mt = 0; mt < NT; ++mt) Vn[(vt * NT + mt) * 64 + lane] = X1[mt];
             }
         }
-        if (LATE)
-            load_rows(W4, rw, cnext);
-        else
-            load_k(cnext);
-        load_gu(cnext);
         __builtin_amdgcn_sched_barrier(0);
 
-        // C: S = exp(G_last) S + Kd^T v_new, four chains at a time
+        // C: S = exp(G_last) S + Kd^T v_new
+        if (LOCAL) {
+            floatx4 d[NKT];
+            products<NKT, NT / 2>(sKd, K4 + cid * OPF4, lane, X1, vterms, d);
 #pragma unroll
-        for (int k4 = 0; k4 < NKT; k4 += 4) {
-            constexpr int KC = NKT < 4 ? NKT : 4;
-            floatx4 d[KC];
-            halfx8 k[KC][NT / 2][2];
+            for (int kb = 0; kb < NKT; ++kb) S[kb] = sGam[4 * kb + lg] * S[kb] + d[kb]; // rows 16 kb + 4 lg .. + 3
+            split_op(rw, sW);
+        } else {
 #pragma unroll
-            for (int i = 0; i < KC; ++i) {
-                d[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int f = 0; f < NT; ++f) k[i][f / 2][f & 1] = half8(sKd, (k4 + i) * NT + f);
-            }
-#pragma unroll
-            for (int tp = 0; tp < NT / 2; ++tp)
-#pragma unroll
-                for (int t = 0; t < 3; ++t)
-#pragma unroll
-                    for (int i = 0; i < KC; ++i) d[i] = mfma32h(k[i][tp][t == 1], t == 2 ? vl[tp] : vh[tp], d[i]);
-#pragma unroll
-            for (int i = 0; i < KC; ++i) {
-                const floatx4 g = sGam[4 * (k4 + i) + lg]; // rows 16 kb + 4 lg .. + 3
-                S[k4 + i] = g * S[k4 + i] + d[i] * (rows_of(eK, k4 + i) * ev);
-            }
-            __builtin_amdgcn_sched_barrier(0); // one group's fragments at a time in registers
+            for (int kb = 0; kb < NKT; ++kb) S[kb] *= sGam[4 * kb + lg];
+            products_f32<NKT, NT>(sKd, lane, X1, S);
         }
-        if (OUT && !ROLES) { // D: out = X2 + A_qk v_new
-            floatx4 y[NT];
-            times_v(vh, vl, y);
-#pragma unroll
-            for (int mt = 0; mt < NT; ++mt) X2[mt] += y[mt] * (rows_of(eA, mt) * ev);
-        }
-        split_rows(rw, sW, eW);
-        split_s();
+        pass_s();
     }
-    if (OUT && !ROLES && n1 > n0) store_out(X2, n1 - 1);
 
     // leaving state: the final state (last segment), the state entering
     // segment 1 (the split's segment 0), Q_j or P_j (pass 1)
@@ -1190,6 +1072,352 @@ __global__ __launch_bounds__(inter_threads(K, MODE, NWV), 1) void chunk_inter_ke
                                                       4 * (16 * kb + i) * ld, 0);
             }
     }
+}
+
+// K = 256: W and Kd^T take 64 KiB of LDS each, which leaves none for q exp(G)
+// and for what a second wave would be handed.  f32 products, one wave per
+// column tile; scale q exp(G), which feeds only the output (off the sequential
+// chain), is read from L2 into registers in phase A.  D(n) runs at the top of
+// iteration n + 1, before the wait for chunk n + 1's copies, whose latency its
+// products cover.
+template <int K, int MODE, int NWV>
+__global__ __launch_bounds__(64 * NWV, 1) void chunk_inter_wide_kernel(ChunkParams p, int nseg_launch, int seg_base) {
+    constexpr bool OUT = MODE == kInterOut || MODE == kInterOutStates || MODE == kInterOutTrain;
+    constexpr bool LOCAL = MODE == kInterLocal;
+    constexpr bool STATES = MODE == kInterStates || MODE == kInterOutStates || MODE == kInterOutTrain;
+    constexpr bool FRAG = MODE == kInterStates || MODE == kInterOutTrain; // the backward's layouts
+    constexpr int NTH = 64 * NWV;  // threads per workgroup
+    constexpr int VSW = 16 * NWV;  // value columns per workgroup
+    constexpr int NKT = K / 16;
+    constexpr int FR = NKT * NT;   // 16x16 fragments per operand per chunk
+    constexpr int OPF4 = FR * 64;  // float4 per operand per chunk
+    constexpr int PFO = OPF4 / NTH; // float4 per lane per operand
+    static_assert(OPF4 % NTH == 0 && K % VSW == 0, "K");
+    constexpr int AF4 = NT * NT * 64; // float4 of A_qk per chunk
+    constexpr int APF = AF4 / NTH;
+    __shared__ floatx4 sW[OPF4], sKd[OPF4];
+    __shared__ floatx4 sA[OUT ? AF4 : 1];
+    __shared__ float sPf[NTH]; // destination of the L2 touches, never read
+    // exp(G_last) of the chunk, copied with Kd^T: read just before phase C, so
+    // that it holds no registers through phases A and D
+    __shared__ floatx4 sGam[K / 4];
+
+    const int V = p.V;
+    const int nvv = V / VSW;                    // value slices
+    const int nvs = LOCAL ? nvv + K / VSW : nvv; // pass 1 adds the slices of P
+    int sq, vs;
+    inter_block(blockIdx.x, p.B * p.HV * nseg_launch, nvs, &sq, &vs);
+    const int bh = sq / nseg_launch, seg = seg_base + sq % nseg_launch;
+    const int bi = bh / p.HV, hv = bh % p.HV;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6); // wave-uniform (scalar)
+    const int lr = lane & 15, lg = lane >> 4;
+    const bool pcol = LOCAL && vs >= nvv;          // a slice of P (wave-uniform)
+    const int vt = (pcol ? vs - nvv : vs) * NWV + wave; // this wave's 16-column tile
+    const int col = 16 * vt + lr;
+    int n0, n1;
+    seg_range(p, seg, &n0, &n1);
+
+    // entering state: S0 (one segment, or the split's segment 0), the chained
+    // state (pass 3; in uniform runs slot 0 is a copy of S0, so that no
+    // workgroup reads the state that the last segment overwrites), 0 (pass 1
+    // value columns) or the identity (pass 1, P columns)
+    const float *Sin = nullptr;
+    if (!LOCAL)
+        Sin = p.NSEG == 1 || (p.SLOT0 && seg == 0) ? p.state + (size_t)bh * K * V
+                                                   : p.ws_qseg + seg_slot(p, bh, seg) * K * V;
+    floatx4 S[NKT];
+#pragma unroll
+    for (int kb = 0; kb < NKT; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = 16 * kb + 4 * lg + i;
+            S[kb][i] = !LOCAL ? Sin[(size_t)row * V + col] : (pcol && row == col ? 1.f : 0.f);
+        }
+
+    const floatx4 *__restrict__ W4 = reinterpret_cast<const floatx4 *>(p.ws_w);
+    const floatx4 *__restrict__ Q4 = reinterpret_cast<const floatx4 *>(p.ws_qg);
+    const floatx4 *__restrict__ K4 = reinterpret_cast<const floatx4 *>(p.ws_kdt);
+    const floatx4 *__restrict__ U4 = reinterpret_cast<const floatx4 *>(p.ws_u);
+    const floatx4 *__restrict__ A4 = reinterpret_cast<const floatx4 *>(p.ws_aqk);
+    const floatx4 *__restrict__ G4 = reinterpret_cast<const floatx4 *>(p.ws_gam);
+    const size_t cid0 = (size_t)bh * p.NC;
+    const size_t uvf4 = (size_t)C * V / 4;
+
+    // the operands go from global memory straight into LDS (lds_copy4):
+    // thread tid's float4 i lands at index i * NTH + tid, as a wave's 64 lanes.
+    // (The buffer-resource form of these copies, buffer_load_dwordx4 ... lds
+    // with 32-bit offsets, needs fewer registers but measured 1.8 % slower.)
+    const int wv = 64 * wave;
+    // Each chunk's operands are also pulled toward L2 one phase before their
+    // LDS copy (l2_touch, one 128-byte line per thread): W, q exp(G) of chunk
+    // n + 1 during A(n), Kd^T, A_qk, U of chunk n + 1 during B-D(n).  Every
+    // wave issues the same count (2, then 3) last before the vmcnt waits, which
+    // leave them in flight; past the last chunk the current one is touched.
+    float *pf_slot = &sPf[wv];
+    constexpr int LOP = OPF4 / 8, LA = AF4 / 8, LU = NWV * NT * 64 / 8; // lines per operand block
+    const int vsu = pcol ? 0 : vs; // the P slices of pass 1 read no U
+    auto touch_wq = [&](size_t c) { // 2 per wave
+        l2_touch(reinterpret_cast<const char *>(W4 + c * OPF4) + 128 * (tid % LOP), pf_slot);
+        l2_touch(reinterpret_cast<const char *>((OUT ? Q4 : K4) + c * OPF4) + 128 * (tid % LOP), pf_slot);
+    };
+    auto touch_kau = [&](size_t c) { // 3 per wave
+        l2_touch(reinterpret_cast<const char *>(K4 + c * OPF4) + 128 * (tid % LOP), pf_slot);
+        if (OUT)
+            l2_touch(reinterpret_cast<const char *>(A4 + c * AF4) + 128 * (tid % LA), pf_slot);
+        else
+            l2_touch(reinterpret_cast<const char *>(W4 + c * OPF4) + 128 * (tid % LOP), pf_slot);
+        l2_touch(reinterpret_cast<const char *>(U4 + c * uvf4 + (size_t)vsu * NWV * NT * 64) + 128 * (tid % LU), pf_slot);
+    };
+    if (n1 > n0) {
+#pragma unroll
+        for (int i = 0; i < PFO; ++i) lds_copy4(&W4[(cid0 + n0) * OPF4 + i * NTH + tid], &sW[i * NTH + wv]);
+        __builtin_amdgcn_sched_barrier(0);
+        touch_kau(cid0 + n0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // S and the first copies have landed: nothing from before the loop is
+    // left in flight for the compiler's own vmcnt waits inside it
+    vm_wait0();
+
+    // chunk nn's output rows from X2 through a buffer resource over its valid
+    // rows: rows past T fall outside its range and the hardware drops those
+    // stores, and each store's offset is a per-lane term (row 4 lg of each
+    // 16-row tile, column col) plus a wave-uniform row term, both 32-bit, in
+    // place of 64-bit row addresses.  Needs sot >= V and 63 sot + V < 2^29
+    // (checked on the host).
+    float *obh = p.out + (int64_t)bi * p.sob + (int64_t)hv * p.soh;
+    const int sot = (int)p.sot, olane = 4 * (4 * lg * sot + col);
+    auto store_out = [&](const floatx4 *o, int nn) {
+        const __amdgpu_buffer_rsrc_t R = rows_rsrc(obh + (int64_t)nn * C * p.sot, sot, min(C, p.T - nn * C), V);
+#pragma unroll
+        for (int mt = 0; mt < NT; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float val = o[mt][i]; // through a scalar: a bit_cast of the element lvalue reads element 0
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, val), R, olane, 4 * (16 * mt + i) * sot, 0);
+            }
+    };
+    floatx4 X1[NT], X2[NT]; // chunk n's v_new and output, both read again in iteration n + 1
+    // D: out = X2 + A_qk v_new (A_qk is lower block-triangular; the chains of
+    // the four time tiles interleave).  D(n) runs at the top of iteration
+    // n + 1, where its MFMAs cover this wave's wait for the next copies.  Its
+    // A_qk tiles are read from sA during the last time tile of C(n), so that
+    // D waits on no LDS read.
+    floatx4 aq[NT][NT]; // A_qk tiles (mt, qt), mt >= qt
+    auto load_aq = [&]() {
+#pragma unroll
+        for (int qt = 0; qt < NT; ++qt)
+#pragma unroll
+            for (int mt = qt; mt < NT; ++mt) aq[mt][qt] = sA[(mt * NT + qt) * 64 + lane];
+    };
+    auto phase_d = [&]() {
+#pragma unroll
+        for (int qt = 0; qt < NT; ++qt)
+#pragma unroll
+            for (int st = 0; st < 4; ++st)
+#pragma unroll
+                for (int mt = qt; mt < NT; ++mt) X2[mt] = mfma16(aq[mt][qt][st], X1[qt][st], X2[mt]);
+    };
+    for (int n = n0; n < n1; ++n) {
+        const size_t cid = cid0 + n;
+        const size_t cnext = n + 1 < n1 ? cid + 1 : cid;
+        if (OUT && n > n0) phase_d(); // D(n - 1)
+        vm_wait<3>();  // this wave's copies of chunk n's W, q exp(G) have landed (not the 3 touches after them)
+        lds_barrier(); // sW, sQ hold chunk n; every wave is done with sKd, sA (n-1)
+#pragma unroll
+        for (int i = 0; i < PFO; ++i) lds_copy4(&K4[cid * OPF4 + i * NTH + tid], &sKd[i * NTH + wv]);
+        if (OUT) {
+            // A_qk is lower block-triangular: copy i of wave w brings tile
+            // f = NWV i + w = (f / NT, f % NT), copied only on or below the
+            // diagonal (10 of the 16 tiles)
+#pragma unroll
+            for (int i = 0; i < APF; ++i) {
+                const int f = NWV * i + wave;
+                if (f % NT <= f / NT) lds_copy4(&A4[cid * AF4 + i * NTH + tid], &sA[i * NTH + wv]);
+            }
+            if (n > n0) store_out(X2, n - 1);
+        }
+        if (wave == 0 && lane < K / 4) lds_copy4(&G4[cid * (K / 4) + lane], sGam);
+        floatx4 u_cur[NT];
+#pragma unroll
+        for (int mt = 0; mt < NT; ++mt)
+            u_cur[mt] = pcol ? floatx4{0.f, 0.f, 0.f, 0.f} : U4[cid * uvf4 + (size_t)(vt * NT + mt) * 64 + lane];
+        if (STATES) { // the state entering chunk n
+            size_t slot = cid;
+            bool keep = true;
+            if (p.st_cc) { // the first caller chunk starting inside chunk n (wave-uniform)
+                const int j0 = (n * C + p.st_cc - 1) / p.st_cc;
+                keep = j0 < p.st_chunks;
+                slot = (size_t)bh * p.st_chunks + j0;
+            }
+            float *Sn = p.ws_sn + slot * K * V;
+            if (keep) {
+                // row-major: 32-bit offsets in a buffer resource over the slot
+                const __amdgpu_buffer_rsrc_t R = __builtin_amdgcn_make_buffer_rsrc(Sn, (short)0, K * V * 4, 0x00020000);
+#pragma unroll
+                for (int kb = 0; kb < NKT; ++kb)
+                    if (FRAG) // the backward's fragment layout: tile (value tile, key tile)
+                        reinterpret_cast<floatx4 *>(Sn)[(vt * NKT + kb) * 64 + lane] = S[kb];
+                    else
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float val = S[kb][i]; // (through a scalar, see store_out)
+                            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, val), R, 4 * (4 * lg * V + col),
+                                                                  4 * (16 * kb + i) * V, 0);
+                        }
+            }
+        }
+        // keep these loads here, a whole phase ahead of their use and of the
+        // vmcnt wait before the next barrier, and the touches last
+        __builtin_amdgcn_sched_barrier(0);
+        touch_wq(cnext);
+        __builtin_amdgcn_sched_barrier(0);
+
+        // A: X1 = W S, X2 = scale (q exp(G)) S
+#pragma unroll
+        for (int mt = 0; mt < NT; ++mt) X1[mt] = X2[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        floatx4 wa[2][NT], ma[2][NT];
+        auto load_a = [&](int kb, int bf) {
+#pragma unroll
+            for (int mt = 0; mt < NT; ++mt) {
+                wa[bf][mt] = sW[(mt * NKT + kb) * 64 + lane];
+                if (OUT) ma[bf][mt] = Q4[cid * OPF4 + (mt * NKT + kb) * 64 + lane];
+            }
+        };
+        load_a(0, 0);
+#pragma unroll
+        for (int kb = 0; kb < NKT; ++kb) {
+            const int cb = kb & 1;
+            // eight (pass 1: four) independent accumulator chains per k-step;
+            // the next step's operands are requested after the first quarter
+#pragma unroll
+            for (int st = 0; st < 4; ++st) {
+#pragma unroll
+                for (int mt = 0; mt < NT; ++mt) {
+                    X1[mt] = mfma16(wa[cb][mt][st], S[kb][st], X1[mt]);
+                    if (OUT) X2[mt] = mfma16(ma[cb][mt][st], S[kb][st], X2[mt]);
+                }
+                if (st == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (kb + 1 < NKT) load_a(kb + 1, cb ^ 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        vm_wait<2>();  // this wave's copies of chunk n's Kd, A_qk, exp(G_last) and its U have landed (not the 2 touches)
+        lds_barrier(); // A done everywhere (sW, sQ free); sKd(n), sA(n) visible
+        // exp(G_last) and phase C's first Kd^T tile, requested before the
+        // copies below so that their latency is spent on the copies' issue
+        floatx4 gk[NKT], ka[2][NKT];
+        auto load_c = [&](int tt, int bf) {
+#pragma unroll
+            for (int kb = 0; kb < NKT; ++kb) ka[bf][kb] = sKd[(kb * NT + tt) * 64 + lane];
+        };
+#pragma unroll
+        for (int kb = 0; kb < NKT; ++kb) gk[kb] = sGam[4 * kb + lg]; // rows 16 kb + 4 lg .. + 3
+        load_c(0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+
+        // B: v_new = U - X1 (kept in X1)
+#pragma unroll
+        for (int mt = 0; mt < NT; ++mt) X1[mt] = u_cur[mt] - X1[mt];
+        if (STATES) {
+            // row-major rows through a buffer resource over the chunk's rows:
+            // token rows [B * HV, T, V] (the resource ends at row T, so rows past T
+            // of a ragged last chunk are dropped) or the chunk's [C, V] block
+            if (p.st_cc || !FRAG) {
+                float *Vn = p.st_cc ? p.ws_vn + ((size_t)bh * p.T + (size_t)n * C) * V : p.ws_vn + cid * C * V;
+                const __amdgpu_buffer_rsrc_t R = rows_rsrc(Vn, V, p.st_cc ? min(C, p.T - n * C) : C, V);
+#pragma unroll
+                for (int mt = 0; mt < NT; ++mt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float val = X1[mt][i]; // (through a scalar, see store_out)
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, val), R, 4 * (4 * lg * V + col),
+                                                              4 * (16 * mt + i) * V, 0);
+                    }
+            } else { // tile (value tile, time tile)
+                float *Vn = p.ws_vn + cid * C * V;
+#pragma unroll
+                for (int mt = 0; mt < NT; ++mt) reinterpret_cast<floatx4 *>(Vn)[(vt * NT + mt) * 64 + lane] = X1[mt];
+            }
+        }
+
+        // W, q exp(G) of chunk n+1, then the touches of its Kd^T, A_qk, U
+        __builtin_amdgcn_sched_barrier(0);
+        if (n + 1 < n1) {
+#pragma unroll
+            for (int i = 0; i < PFO; ++i) lds_copy4(&W4[(cid + 1) * OPF4 + i * NTH + tid], &sW[i * NTH + wv]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        touch_kau(cnext);
+        __builtin_amdgcn_sched_barrier(0);
+
+        // C: S = exp(G_last) S + Kd^T v_new
+#pragma unroll
+        for (int kb = 0; kb < NKT; ++kb) {
+            S[kb][0] *= gk[kb][0];
+            S[kb][1] *= gk[kb][1];
+            S[kb][2] *= gk[kb][2];
+            S[kb][3] *= gk[kb][3];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) {
+            const int cb = tt & 1;
+            // NKT independent accumulator chains per k-step; the next time
+            // tile's operands are requested after the first quarter
+#pragma unroll
+            for (int st = 0; st < 4; ++st) {
+#pragma unroll
+                for (int kb = 0; kb < NKT; ++kb) S[kb] = mfma16(ka[cb][kb][st], X1[tt][st], S[kb]);
+                if (st == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (tt + 1 < NT) load_c(tt + 1, cb ^ 1);
+                    else if (OUT) load_aq(); // for D(n), at the top of iteration n + 1
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    vm_wait0(); // the last touches have landed in sPf
+    if (OUT && n1 > n0) {
+        phase_d();
+        store_out(X2, n1 - 1);
+    }
+
+    // leaving state: the final state (last segment), the state entering
+    // segment 1 (the split's segment 0), Q_j or P_j (pass 1)
+    float *Sout = nullptr;
+    int ld = V;
+    if (OUT) {
+        if (seg == p.NSEG - 1)
+            Sout = p.state + (size_t)bh * K * V;
+        else if (MODE == kInterOut && p.SLOT0 && seg == 0)
+            Sout = p.ws_qseg + seg_slot(p, bh, 1) * K * V;
+    } else if (LOCAL && pcol) {
+        Sout = p.ws_pseg + seg_slot(p, bh, seg) * K * K;
+        ld = K;
+    } else if (LOCAL && seg + 1 < p.NSEG) { // (the last segment runs for its P only: training)
+        Sout = p.ws_qseg + seg_slot(p, bh, seg + 1) * K * V;
+    }
+    if (Sout) {
+#pragma unroll
+        for (int kb = 0; kb < NKT; ++kb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) Sout[(size_t)(16 * kb + 4 * lg + i) * ld + col] = S[kb][i];
+    }
+}
+
+// The kernel for a head width, mode and column tiles per workgroup.
+template <int K, int MODE, int NWV> constexpr auto inter_kernel() {
+    if constexpr (K <= 128)
+        return &chunk_inter_kernel<K, MODE, NWV>;
+    else
+        return &chunk_inter_wide_kernel<K, MODE, NWV>;
 }
 
 // Pass 2 of the segmented form.  Per (b, hv), the slot of segment j + 1
@@ -1403,7 +1631,7 @@ template <int K, int MODE, int NW>
 size_t half_cu_pad() {
     static const size_t pad = [] {
         hipFuncAttributes a{};
-        if (hipFuncGetAttributes(&a, reinterpret_cast<const void *>(&chunk_inter_kernel<K, MODE, NW>)) != hipSuccess)
+        if (hipFuncGetAttributes(&a, reinterpret_cast<const void *>(inter_kernel<K, MODE, NW>())) != hipSuccess)
             return size_t(0);
         constexpr size_t half = 80 * 1024 + 256;
         return a.sharedSizeBytes >= half ? size_t(0) : half - a.sharedSizeBytes;
@@ -1416,7 +1644,7 @@ size_t half_cu_pad() {
 template <int K, int V, int MODE>
 void launch_inter(const ChunkParams &p, hipStream_t s, int nseg, int seg_base, size_t lds = 0) {
     constexpr int NWV = inter_nwv(K, V), VSW = 16 * NWV;
-    hipLaunchKernelGGL((chunk_inter_kernel<K, MODE, NWV>), dim3(p.B * p.HV * nseg * (V / VSW)),
+    hipLaunchKernelGGL((inter_kernel<K, MODE, NWV>()), dim3(p.B * p.HV * nseg * (V / VSW)),
                        dim3(inter_threads(K, MODE, NWV)), lds, s, p, nseg, seg_base);
 }
 
@@ -1436,14 +1664,14 @@ hipError_t launch_chunk_t(const ChunkParams &p0, hipStream_t s, int phases) {
     // chunk's W and Kd^T are loaded and split once for twice the columns, and
     // two waves per SIMD still fit its registers.
     constexpr int NWL = (K == 128 && V % 128 == 0) ? 8 : NWV, VSWL = 16 * NWL;
-    const dim3 blk(64 * NWV), blkl(64 * NWL);
+    const dim3 blkl(inter_threads(K, kInterLocal, NWL));
     const int seqs = p0.B * p0.HV;
     const bool infer = (phases & 112) || (phases & 14) == 2;
     ChunkParams ps;
     const bool split = infer && split_segments(p0, &ps);
     const ChunkParams &p = split ? ps : p0;
     auto summaries = [&](int nl) -> hipError_t { // pass 1 over segments 0 .. nl - 1 (uniform)
-        hipLaunchKernelGGL((chunk_inter_kernel<K, kInterLocal, NWL>), dim3(seqs * nl * ((V + K) / VSWL)), blkl, 0, s,
+        hipLaunchKernelGGL((inter_kernel<K, kInterLocal, NWL>()), dim3(seqs * nl * ((V + K) / VSWL)), blkl, 0, s,
                            p, nl, 0);
         return hipGetLastError();
     };
@@ -1453,7 +1681,7 @@ hipError_t launch_chunk_t(const ChunkParams &p0, hipStream_t s, int phases) {
             s, [&](hipStream_t sa) { launch_inter<K, V, kInterOut>(p, sa, 1, 0, half_cu_pad<K, kInterOut, NWV>()); },
             [&](hipStream_t sm) {
                 const size_t lds = half_cu_pad<K, kInterLocal, NWL>();
-                hipLaunchKernelGGL((chunk_inter_kernel<K, kInterLocal, NWL>),
+                hipLaunchKernelGGL((inter_kernel<K, kInterLocal, NWL>()),
                                    dim3(seqs * (p.NSEG - 2) * ((V + K) / VSWL)), blkl, lds, sm, p, p.NSEG - 2, 1);
             });
     };

@@ -70,18 +70,16 @@ __device__ __forceinline__ floatx4 mfma4x(floatx4 a, floatx4 b, floatx4 c) {
 //   1: dv_new = A_qk^T dO + Kd dS'
 //      dS' and dv_new go to the workspace for the per-chunk kernels
 //   2: dS' <- e^{G_last} dS' + QG^T dO - W^T dv_new
-// The products run on the f16 matrix cores, every operand as two f16 terms per
-// row or column scale.  What bounds the walk is one chunk's serial work: loads,
-// splitting, LDS reads and products of a wave one after the other.  So each
-// column tile has two waves: a state wave takes what hangs on dS' (Kd dS',
-// W^T dv_new, the update), and an output-gradient wave computes A_qk^T dO of
-// chunk n - 1 and QG^T dO of chunk n beside it and hands them over in LDS.
-// An operand is split once, by row tiles shared out over the waves of its
-// role, during the phase before its use; its loads are issued a phase earlier
-// still.  B = 4, T = 2048, 16 heads, K = V = 128: 174 us with f32 products in
-// one wave a column tile, 140 now (0.48 GB, 92 us at the card's copy rate);
-// the half of it that pass 1 walks 137 -> 104; K = 64, V = 96, T = 1999 79 -> 48
-// and 70 -> 44.
+// f32 products.  Each column tile has two waves: a state wave takes what hangs
+// on dS' (Kd dS', W^T dv_new, the update), and an output-gradient wave computes
+// A_qk^T dO of chunk n - 1 and QG^T dO of chunk n beside it and hands them over
+// in LDS.  Every operand has one LDS buffer, refilled by direct copies during the
+// phase that does not read it.  The products bound the walk: 13.6k cycles a chunk
+// at K = 128.  (Two f16 terms under a scale per row or column took less, 127 and
+// 91 us below, but a token's gradient must not depend on the size of an earlier
+// token's d_out, and under a shared scale it did.)  One wave per column tile ->
+// two: B = 4, T = 2048, 16 heads, K = V = 128 158 -> 151 us, the half of it that
+// pass 1 walks 122 -> 113; K = 64, V = 96, T = 1999 77 -> 59 and 68 -> 44.
 //
 // Segmented form (NSEG > 1), the mirror of the forward's: over a segment the
 // map from the gradient leaving it to the gradient entering it is affine,
@@ -94,9 +92,9 @@ __device__ __forceinline__ floatx4 mfma4x(floatx4 a, floatx4 b, floatx4 c) {
 // ---------------------------------------------------------------------------
 constexpr int kRevOut = 0, kRevLocal = 1;
 
-// K = 256: no LDS left for a third operand, the terms handed over and a second
-// wave per column tile.  f32 products, one wave per column tile; QG^T, whose
-// product feeds only dS (not the dS -> dv_new chain), is read from L2.  The
+// K = 256: no LDS left for a third operand and for what a second wave would
+// hand over.  One wave per column tile; QG^T, whose product feeds only dS (not
+// the dS -> dv_new chain), is read from L2.  The
 // operands are A-operand fragments written by the training forward; each LDS
 // buffer is refilled by direct copies while the other phase runs, behind
 // fence-free barriers that wait only for those copies.
@@ -343,20 +341,18 @@ __global__ __launch_bounds__(64 * NW, 1) void bwd_inter_wide_kernel(BwdParams bp
     }
 }
 
-// K <= 128 (see above): the terms of all operands in LDS, two waves per column
-// tile.
+// K <= 128 (see above): two waves per column tile.
 template <int K, int MODE, int NW>
 __global__ __launch_bounds__(128 * NW, 1) void bwd_inter_kernel(BwdParams bp, int seg0, int nseg_launch) {
     const ChunkParams &p = bp.f;
     constexpr bool LOCAL = MODE == kRevLocal;
+    constexpr int NTH = 128 * NW, NWS = 2 * NW; // threads, waves per workgroup
     constexpr int NKT = K / 16, OPF4 = NKT * NT * 64, AF4 = NT * NT * 64;
-    static_assert(NT % NW == 0 && NKT % NW == 0, "row tiles per wave");
-    constexpr int CW = NT / NW, CK = NKT / NW; // row tiles a wave loads and splits: of Kd, A_qk^T; of W^T, QG^T
-    __shared__ floatx4 sKd[OPF4], sWT[OPF4], sQT[OPF4];
-    __shared__ floatx4 sAT[12 * 64]; // A_qk^T by pairs of tiles on or above the diagonal
+    constexpr int NAT = NT * (NT + 1) / 2; // tiles of A_qk^T on or above the diagonal, at at_tile(st, rt)
+    static_assert(OPF4 % NTH == 0, "K");
+    __shared__ floatx4 sKd[OPF4], sWT[OPF4], sQT[OPF4], sAT[NAT * 64];
     __shared__ floatx4 sZ[NW * NT * 64], sY[NW * NKT * 64]; // A_qk^T dO, QG^T dO of the column tiles
     __shared__ floatx4 sGam[K / 4];                         // e^{G_last} of the chunk
-    __shared__ __align__(16) float eKd[C], eAT[C], eQT[K], eWT[K]; // inverse scales of the rows (split_row_tile)
 
     const int V = p.V, nvv = V / (16 * NW);
     int sq, vs;
@@ -376,44 +372,35 @@ __global__ __launch_bounds__(128 * NW, 1) void bwd_inter_kernel(BwdParams bp, in
     const floatx4 *__restrict__ WT4 = reinterpret_cast<const floatx4 *>(p.ws_wt);
     const floatx4 *__restrict__ G4 = reinterpret_cast<const floatx4 *>(p.ws_gam);
     const size_t cid0 = (size_t)bh * p.NC;
-    auto rows_of = [&](const float *e, int tile) { return *reinterpret_cast<const floatx4 *>(&e[16 * tile + 4 * lg]); };
-    auto half8 = [&](const floatx4 *s, int f) { return __builtin_bit_cast(halfx8, s[f * 64 + lane]); };
-    // row tiles of a key-row operand (QG^T, W^T) through registers into its terms in LDS
-    auto load_key = [&](const floatx4 *src, floatx4 *r, size_t c) {
+    const int wv = 64 * wid;
+    // The operands go from global memory straight into LDS (lds_copy4), all
+    // waves taking part: Kd, QG^T of chunk n - 1 during phase 2 of chunk n, W^T
+    // and e^{G_last} of chunk n and A_qk^T of chunk n - 1 during its phase 1.
+    auto copy_kq = [&](size_t c) {
 #pragma unroll
-        for (int i = 0; i < CK * NT; ++i) r[i] = ld_uni(src + c * OPF4 + wave * CK * NT * 64, i * 64 + lane);
-    };
-    auto split_key = [&](const floatx4 *r, floatx4 *s, float *e) {
-#pragma unroll
-        for (int i = 0; i < CK; ++i) {
-            const int kb = wave * CK + i;
-            split_row_tile<NT>(&r[i * NT], &s[kb * NT * 64], lane, &e[16 * kb]);
+        for (int i = 0; i < OPF4 / NTH; ++i) {
+            lds_copy4(&KD4[c * OPF4 + i * NTH + tid], &sKd[i * NTH + wv]);
+            lds_copy4(&QT4[c * OPF4 + i * NTH + tid], &sQT[i * NTH + wv]);
         }
     };
-    // rows of a key-row operand times C x 16 terms, four row tiles (chains) at a time; f(kb, product before scales)
-    auto times_t = [&](const floatx4 *s, const halfx8 *hi, const halfx8 *lo, auto f) {
-        constexpr int KC = NKT < 4 ? NKT : 4;
+    auto copy_w = [&](size_t c) {
 #pragma unroll
-        for (int k4 = 0; k4 < NKT; k4 += 4) {
-            floatx4 d[KC];
-            halfx8 k[KC][NT / 2][2];
-#pragma unroll
-            for (int i = 0; i < KC; ++i) {
-                d[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int t = 0; t < NT; ++t) k[i][t / 2][t & 1] = half8(s, (k4 + i) * NT + t);
-            }
-#pragma unroll
-            for (int tp = 0; tp < NT / 2; ++tp)
-#pragma unroll
-                for (int t = 0; t < 3; ++t)
-#pragma unroll
-                    for (int i = 0; i < KC; ++i) d[i] = mfma32h(k[i][tp][t == 1], t == 2 ? lo[tp] : hi[tp], d[i]);
-#pragma unroll
-            for (int i = 0; i < KC; ++i) f(k4 + i, d[i]);
-            __builtin_amdgcn_sched_barrier(0); // one group's fragments at a time in registers
-        }
+        for (int i = 0; i < OPF4 / NTH; ++i) lds_copy4(&WT4[c * OPF4 + i * NTH + tid], &sWT[i * NTH + wv]);
+        if (wid == 0 && lane < K / 4) lds_copy4(&G4[c * (K / 4) + lane], sGam);
     };
+    const auto at_tile = [](int st, int rt) { return st * NT - st * (st - 1) / 2 + rt - st; };
+    auto copy_at = [&](size_t c) {
+#pragma unroll
+        for (int st = 0; st < NT; ++st)
+#pragma unroll
+            for (int rt = st; rt < NT; ++rt)
+                if (at_tile(st, rt) % NWS == wid)
+                    lds_copy4(&AT4[c * AF4 + (st * NT + rt) * 64 + lane], &sAT[at_tile(st, rt) * 64]);
+    };
+    if (n1 > n0) {
+        copy_at(cid0 + n1 - 1);
+        copy_kq(cid0 + n1 - 1);
+    }
 
     if (wid >= NW) { // the output-gradient wave of a column tile (every barrier has its twin below)
         if (n1 <= n0) return;
@@ -428,68 +415,50 @@ __global__ __launch_bounds__(128 * NW, 1) void bwd_inter_kernel(BwdParams bp, in
 #pragma unroll
                 for (int i = 0; i < 4; ++i) dO[mt][i] = bld1(R, dol + (16 * mt + i) * ro);
         };
-        const auto at_first = [](int st) { return st < 2 ? 4 * st : 4 + 2 * st; }; // row tile st's first fragment in sAT
-        auto load_at = [&](floatx4 *r, size_t c) { // upper block-triangular: tiles (st, rt >= st) only
-#pragma unroll
-            for (int i = 0; i < CW * NT; ++i) {
-                const int st = wave * CW + i / NT, rt = i % NT;
-                r[i] = rt >= st ? ld_uni(AT4 + c * AF4 + st * NT * 64, rt * 64 + lane) : floatx4{0.f, 0.f, 0.f, 0.f};
-            }
-        };
-        auto split_at = [&](const floatx4 *r) {
-#pragma unroll
-            for (int i = 0; i < CW; ++i) {
-                const int st = wave * CW + i;
-                floatx4 *d = &sAT[at_first(st) * 64];
-                if (st < 2)
-                    split_row_tile<4>(&r[i * NT], d, lane, &eAT[16 * st]);
-                else
-                    split_row_tile<2>(&r[i * NT + 2], d, lane, &eAT[16 * st]);
-            }
-        };
-        halfx8 oh[NT / 2], ol[NT / 2]; // dO of a chunk and its columns' inverse scale
-        float eo = 0.f;
-        auto products_z = [&]() {
+        floatx4 dO[NT], next[NT];
+        auto products_z = [&](const floatx4 *o) {
             floatx4 z[NT];
 #pragma unroll
             for (int st = 0; st < NT; ++st) z[st] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int tp = 0; tp < NT / 2; ++tp)
+            for (int rt = 0; rt < NT; ++rt) {
+                floatx4 a[NT];
 #pragma unroll
-                for (int t = 0; t < 3; ++t)
+                for (int st = 0; st <= rt; ++st) a[st] = sAT[at_tile(st, rt) * 64 + lane];
 #pragma unroll
-                    for (int st = 0; st < 2 * tp + 2; ++st) // (row tiles 2, 3 hold the second pair only)
-                        z[st] = mfma32h(half8(sAT, at_first(st) + (st < 2 ? 2 * tp : 0) + (t == 1)), t == 2 ? ol[tp] : oh[tp],
-                                        z[st]);
+                for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int st = 0; st < NT; ++st) sZ[(wave * NT + st) * 64 + lane] = z[st] * (rows_of(eAT, st) * eo);
+                    for (int st = 0; st <= rt; ++st) z[st] = mfma16(a[st][i], o[rt][i], z[st]);
+            }
+#pragma unroll
+            for (int st = 0; st < NT; ++st) sZ[(wave * NT + st) * 64 + lane] = z[st];
         };
-        floatx4 rq[CK * NT], ra[CW * NT], dO[NT];
-        auto at_or_first = [&](int n) { return max(n, n0); };
-        load_at(ra, cid0 + n1 - 1);
-        load_key(QT4, rq, cid0 + n1 - 1);
         load_dO(dO, n1 - 1);
-        split_at(ra);
-        load_at(ra, cid0 + at_or_first(n1 - 2));
-        split_key(rq, sQT, eQT);
-        eo = split_columns<NT>(dO, oh, ol);
-        load_dO(dO, at_or_first(n1 - 2));
-        lds_barrier(); // sAT holds the last chunk's terms
-        products_z();
+        vm_wait0();
+        lds_barrier(); // sAT holds the last chunk
+        products_z(dO);
         for (int n = n1 - 1; n >= n0; --n) {
-            lds_barrier(); // sQT and sZ of chunk n are there
-            load_key(QT4, rq, cid0 + at_or_first(n - 1));
+            const size_t cid = cid0 + n;
+            vm_wait0();
+            lds_barrier(); // sKd, sQT and sZ hold chunk n; every wave is done with sWT, sY (n + 1), sAT (n)
+            copy_w(cid);
+            if (n > n0) copy_at(cid - 1);
+            load_dO(next, max(n - 1, n0));
             __builtin_amdgcn_sched_barrier(0); // keep these loads here, a phase ahead of their use
-            times_t(sQT, oh, ol, [&](int kb, floatx4 d) { sY[(wave * NKT + kb) * 64 + lane] = d * (rows_of(eQT, kb) * eo); });
-            split_at(ra); // of chunk n - 1
-            lds_barrier(); // sY of chunk n, sAT of chunk n - 1 are there; sQT, sZ are free
-            load_at(ra, cid0 + at_or_first(n - 2));
-            __builtin_amdgcn_sched_barrier(0);
-            eo = split_columns<NT>(dO, oh, ol);
-            load_dO(dO, at_or_first(n - 2));
-            __builtin_amdgcn_sched_barrier(0);
-            products_z();
-            split_key(rq, sQT, eQT);
+            floatx4 y[NKT];
+#pragma unroll
+            for (int kb = 0; kb < NKT; ++kb) y[kb] = floatx4{0.f, 0.f, 0.f, 0.f};
+            products_f32<NKT, NT>(sQT, lane, dO, y);
+#pragma unroll
+            for (int kb = 0; kb < NKT; ++kb) sY[(wave * NKT + kb) * 64 + lane] = y[kb];
+#pragma unroll
+            for (int mt = 0; mt < NT; ++mt) dO[mt] = next[mt];
+            vm_wait0();
+            lds_barrier(); // sKd, sQT, sZ free; sWT, sY of chunk n, sAT of chunk n - 1 are there
+            if (n > n0) {
+                copy_kq(cid - 1);
+                products_z(dO);
+            }
         }
         return;
     }
@@ -514,88 +483,45 @@ __global__ __launch_bounds__(128 * NW, 1) void bwd_inter_kernel(BwdParams bp, in
             dS[kb][i] = LOCAL ? 0.f
                               : __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
                                                               Rin, 4 * (4 * lg * V + col), 4 * (16 * kb + i) * V, 0));
-
-    floatx4 rk[CW * NKT], rw[CK * NT], rg;
-    auto load_kd = [&](size_t c) {
-#pragma unroll
-        for (int i = 0; i < CW * NKT; ++i) rk[i] = ld_uni(KD4 + c * OPF4 + wave * CW * NKT * 64, i * 64 + lane);
-    };
-    auto split_kd = [&]() {
-#pragma unroll
-        for (int i = 0; i < CW; ++i) {
-            const int st = wave * CW + i;
-            split_row_tile<NKT>(&rk[i * NKT], &sKd[st * NKT * 64], lane, &eKd[16 * st]);
-        }
-    };
-    halfx8 sh[NKT / 2], sl[NKT / 2]; // dS' and its columns' inverse scales
-    float es = 0.f;
     if (n1 > n0) {
-        load_kd(cid0 + n1 - 1);
-        load_key(WT4, rw, cid0 + n1 - 1);
-        rg = ld_uni(G4 + (cid0 + n1 - 1) * (K / 4), lane % (K / 4));
-        split_kd();
-        es = split_columns<NKT>(dS, sh, sl);
+        vm_wait0();
         lds_barrier();
     }
     for (int n = n1 - 1; n >= n0; --n) {
-        const size_t cid = cid0 + n, cnext = cid0 + max(n - 1, n0);
-        lds_barrier(); // sKd, sZ hold chunk n; every wave is done with sWT, sY (n + 1)
-        load_kd(cnext);
+        const size_t cid = cid0 + n;
+        vm_wait0();
+        lds_barrier(); // sKd, sQT and sZ hold chunk n; every wave is done with sWT, sY (n + 1), sAT (n)
+        copy_w(cid);
+        if (n > n0) copy_at(cid - 1);
         if (!LOCAL) { // dL/d(state leaving chunk n)
             floatx4 *Dsn = reinterpret_cast<floatx4 *>(bp.ws_dsn + cid * K * V) + vt * NKT * 64;
 #pragma unroll
             for (int kb = 0; kb < NKT; ++kb) Dsn[kb * 64 + lane] = dS[kb];
         }
-        __builtin_amdgcn_sched_barrier(0); // keep these loads here, a phase ahead of their use
+        __builtin_amdgcn_sched_barrier(0);
 
-        // 1: dv_new = Kd dS' + A_qk^T dO
+        // 1: dv_new = A_qk^T dO + Kd dS'
         floatx4 dvn[NT];
 #pragma unroll
-        for (int st = 0; st < NT; ++st) dvn[st] = floatx4{0.f, 0.f, 0.f, 0.f};
-        {
-            halfx8 w[2][NT][2]; // a step's operands are read during the step before it
-            auto fetch = [&](int kp) {
-#pragma unroll
-                for (int st = 0; st < NT; ++st)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) w[kp & 1][st][h] = half8(sKd, st * NKT + 2 * kp + h);
-            };
-            fetch(0);
-#pragma unroll
-            for (int kp = 0; kp < NKT / 2; ++kp) {
-                if (kp + 1 < NKT / 2) fetch(kp + 1);
-#pragma unroll
-                for (int t = 0; t < 3; ++t)
-#pragma unroll
-                    for (int st = 0; st < NT; ++st)
-                        dvn[st] = mfma32h(w[kp & 1][st][t == 1], t == 2 ? sl[kp] : sh[kp], dvn[st]);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        split_key(rw, sWT, eWT);
-        if (wave == 0 && lane < K / 4) sGam[lane] = rg;
-#pragma unroll
-        for (int st = 0; st < NT; ++st)
-            dvn[st] = sZ[(wave * NT + st) * 64 + lane] + dvn[st] * (rows_of(eKd, st) * es);
-        halfx8 vh[NT / 2], vl[NT / 2];
-        const float ev = split_columns<NT>(dvn, vh, vl);
-        lds_barrier(); // sKd, sZ free; sWT, sY and e^{G_last} of chunk n are there
+        for (int st = 0; st < NT; ++st) dvn[st] = sZ[(wave * NT + st) * 64 + lane];
+        products_f32<NT, NKT>(sKd, lane, dS, dvn);
+        vm_wait0();
+        lds_barrier(); // sKd, sQT, sZ free; sWT, sY of chunk n, sAT of chunk n - 1 are there
+        if (n > n0) copy_kq(cid - 1);
         if (!LOCAL) {
             floatx4 *Dvn = reinterpret_cast<floatx4 *>(bp.ws_dvn + cid * C * V) + vt * NT * 64;
 #pragma unroll
             for (int st = 0; st < NT; ++st) Dvn[st * 64 + lane] = dvn[st];
         }
-        load_key(WT4, rw, cnext);
-        rg = ld_uni(G4 + cnext * (K / 4), lane % (K / 4));
         __builtin_amdgcn_sched_barrier(0);
 
         // 2: dS' <- e^{G_last} dS' + QG^T dO - W^T dv_new
-        times_t(sWT, vh, vl, [&](int kb, floatx4 d) {
-            const floatx4 g = sGam[4 * kb + lg]; // rows 16 kb + 4 lg .. + 3
-            dS[kb] = (g * dS[kb] + sY[(wave * NKT + kb) * 64 + lane]) - d * (rows_of(eWT, kb) * ev);
-        });
-        split_kd();
-        es = split_columns<NKT>(dS, sh, sl);
+#pragma unroll
+        for (int kb = 0; kb < NKT; ++kb) // rows 16 kb + 4 lg .. + 3
+            dS[kb] = sGam[4 * kb + lg] * dS[kb] + sY[(wave * NKT + kb) * 64 + lane];
+#pragma unroll
+        for (int st = 0; st < NT; ++st) dvn[st] = -dvn[st];
+        products_f32<NKT, NT>(sWT, lane, dvn, dS);
     }
     // the gradient entering the segment: dS0 (first segment) or R_j (pass 1)
     float *out = nullptr;

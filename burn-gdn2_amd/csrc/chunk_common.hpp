@@ -127,95 +127,131 @@ __device__ __forceinline__ void quad_swap_pairs(floatx4 &x, bool odd) { // odd =
 }
 
 // ---------------------------------------------------------------------------
-// f32 products on the f16 matrix cores, for the sequential kernels: an operand
-// x is taken as two f16 terms of x 2^s,
-//   hi = f16(x 2^s),  lo = f16(x 2^s - hi),
-// and hi hi + hi lo + lo hi accumulated in f32 (the remaining lo lo is below
-// 2^-22 of a product).  s is one exponent per row of the first operand and per
-// column of the second, chosen so that their largest magnitude lies in
-// [2^14, 2^15): 23 bits of every element down to 2^-17 of the largest, and an
-// absolute error of 2^-40 of it below.  A 16x16x32 step takes the fragments
-// of two neighbouring 16x16 tiles of the contraction, k = 4 group + step in
-// each, so that two f32 accumulator tiles are one f16 second operand.  Three
-// such steps (16 cycles each) stand for the eight 16x16x4 f32 steps (32 cycles
-// each) of the same contraction.
+// f32 products on the bf16 matrix cores, for the segment summaries: an operand
+// x is taken as three bf16 terms,
+//   h = bf16(x),  m = bf16(x - h),  l = bf16(x - h - m),
+// whose sum is x exactly (8 significant bits each, and the signs of the
+// remainders, cover f32's 24), whatever its neighbours in the row are, and
+// hh + hm + mh + mm + hl + lh are accumulated in f32: what is left out is below
+// 2^-25 of a product, less than its rounding in f32.  bf16 has f32's exponents,
+// so there is no scale; only remainders below 2^-133 are lost.  A 16x16x32
+// step takes the fragments of two neighbouring 16x16 tiles of the contraction,
+// k = 4 group + step in each, so that two f32 accumulator tiles are one second
+// operand.  Six such steps (16 cycles each) stand for the eight 16x16x4 f32
+// steps (32 cycles each) of the same contraction; splitting costs 5.5 vector
+// instructions an element, so it pays where a workgroup splits an operand once
+// for many columns.
+//
+// Infinities (h infinite, x - h not a number) and values that round to one do
+// not split.  They show as an output that is not finite; such outputs are
+// formed again from the f32 operands by f32 instructions (products).
 // ---------------------------------------------------------------------------
-typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
-typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ floatx4 mfma32h(halfx8 a, halfx8 b, floatx4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-// The scale 2^s for a largest magnitude mx (1 where it is 0 or not finite;
-// s at most 100, so that the inverse and its product with another stay normal).
-__device__ __forceinline__ float f16_scale(float mx) {
-    const bool ok = mx > 0.f && mx < __builtin_inff();
-    return __builtin_ldexpf(1.f, ok ? min(100, 15 - __builtin_amdgcn_frexp_expf(mx)) : 0);
-}
-// 1 / scale, exactly
-__device__ __forceinline__ float inv_scale(float scale) {
-    return __builtin_bit_cast(float, 0x7F000000u - __builtin_bit_cast(unsigned, scale));
-}
-__device__ __forceinline__ float max4(float m, floatx4 x) {
-    m = fmaxf(fmaxf(m, fabsf(x[0])), fabsf(x[1]));
-    return fmaxf(fmaxf(m, fabsf(x[2])), fabsf(x[3]));
-}
-// Largest over the four lanes l % 16, in all of them.  (The swaps' results go
-// through scalars: a bit_cast of a vector's element reads element 0.)
-__device__ __forceinline__ float max_groups(float m) {
-    const unsigned u = __builtin_bit_cast(unsigned, m);
-    const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    const unsigned a0 = a[0], a1 = a[1];
-    m = fmaxf(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
-    const unsigned v = __builtin_bit_cast(unsigned, m);
-    const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    const unsigned b0 = b[0], b1 = b[1];
-    return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
-}
-// Two tiles' four elements each as the two terms of one 32-deep operand: the
-// scaled values rounded in pairs, then their exact remainders rounded by one
-// mixed-precision multiply-add each (v_fma_mixlo/hi_f16).
-__device__ __forceinline__ void split_pair(floatx4 a, floatx4 b, float scale, halfx8 *hi, halfx8 *lo) {
+struct Terms {
+    bf16x8 t[3]; // h, m, l
+};
+// Two tiles' four elements each as one 32-deep operand.
+__device__ __forceinline__ Terms split_pair(floatx4 a, floatx4 b) {
+    Terms r;
 #pragma unroll
     for (int j = 0; j < 8; j += 2) {
-        const float x = j < 4 ? a[j & 3] : b[j & 3], y = j < 4 ? a[(j & 3) + 1] : b[(j & 3) + 1];
-        const halfx2 h = __builtin_convertvector(floatx2{x * scale, y * scale}, halfx2);
-        (*hi)[j] = h[0];
-        (*hi)[j + 1] = h[1];
-        (*lo)[j] = (_Float16)__builtin_fmaf(x, scale, -(float)h[0]);
-        (*lo)[j + 1] = (_Float16)__builtin_fmaf(y, scale, -(float)h[1]);
+        float x = j < 4 ? a[j & 3] : b[j & 3], y = j < 4 ? a[(j & 3) + 1] : b[(j & 3) + 1];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const bf16x2 q = __builtin_convertvector(floatx2{x, y}, bf16x2);
+            r.t[t][j] = q[0];
+            r.t[t][j + 1] = q[1];
+            x -= (float)q[0];
+            y -= (float)q[1];
+        }
+    }
+    return r;
+}
+// T accumulator tiles of a column block as T / 2 second operands.
+template <int T> __device__ __forceinline__ void split_tiles(const floatx4 *x, Terms *r) {
+#pragma unroll
+    for (int t = 0; t < T; t += 2) r[t / 2] = split_pair(x[t], x[t + 1]);
+}
+
+// A first operand's terms in LDS: pair i of neighbouring tiles (f32 fragments
+// 2 i and 2 i + 1 of it) lies at s[3 i], as h, m and l of 64 lanes each.
+__device__ __forceinline__ void put_terms(floatx4 a, floatx4 b, floatx4 *s, int pair, int lane) {
+    const Terms r = split_pair(a, b);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) s[(pair * 3 + t) * 64 + lane] = __builtin_bit_cast(floatx4, r.t[t]);
+}
+
+// x (+)= A b with f32 instructions, A of R row tiles x T tiles in f32 fragments
+// in (row tile, tile) order from s (tile columns K0 .. K1 - 1 of it).  A tile
+// column's fragments are read during the products of the one before it.
+template <int R, int T, int K0 = 0, int K1 = T>
+__device__ __forceinline__ void products_f32(const floatx4 *s, int lane, const floatx4 *b, floatx4 *x) {
+    floatx4 a[2][R];
+    auto read = [&](int k) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) a[k & 1][r] = s[(r * T + k) * 64 + lane];
+    };
+    read(K0);
+#pragma unroll
+    for (int k = K0; k < K1; ++k) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) x[r] = mfma16(a[k & 1][r][i], b[k][i], x[r]);
+            if (i == 0) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (k + 1 < K1) read(k + 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
-// One row tile of a first operand, NF fragments v along the contraction, into
-// LDS as its two terms: of fragments 2 p and 2 p + 1 (64 float4 each from s),
-// the first becomes hi and the second lo of the pair.  Every lane of the wave
-// takes part; ex[l % 16] receives the rows' 2^-s.
-template <int NF> __device__ __forceinline__ void split_row_tile(const floatx4 *v, floatx4 *s, int lane, float *ex) {
-    static_assert(NF % 2 == 0, "pairs of tiles");
-    float mx = 0.f;
+
+// x = A b for A of R row tiles x P pairs of tiles whose terms lie in LDS from s,
+// and a column block b (f32 tiles, and their terms t); src: A's f32 fragments.
+template <int R, int P>
+__device__ __forceinline__ void products(const floatx4 *s, const floatx4 *src, int lane, const floatx4 *b, const Terms *t,
+                                         floatx4 *x) {
+    constexpr int RB = R < 4 ? R : 4; // row tiles (independent chains) at a time
+    constexpr int ta[6] = {2, 0, 1, 1, 0, 0}, tb[6] = {0, 2, 1, 0, 1, 0};
+    constexpr int F = R / RB * P;
+    bf16x8 a[2][RB][3]; // a step's operands are read during the step before it
+    auto read = [&](int f) {
 #pragma unroll
-    for (int f = 0; f < NF; ++f) mx = max4(mx, v[f]);
-    const float scale = f16_scale(max_groups(mx));
+        for (int r = 0; r < RB; ++r)
 #pragma unroll
-    for (int f = 0; f < NF; f += 2) {
-        halfx8 hi, lo;
-        split_pair(v[f], v[f + 1], scale, &hi, &lo);
-        s[f * 64 + lane] = __builtin_bit_cast(floatx4, hi);
-        s[(f + 1) * 64 + lane] = __builtin_bit_cast(floatx4, lo);
+            for (int j = 0; j < 3; ++j)
+                a[f & 1][r][j] = __builtin_bit_cast(bf16x8, s[(((f / P * RB + r) * P + f % P) * 3 + j) * 64 + lane]);
+    };
+    read(0);
+#pragma unroll
+    for (int r = 0; r < R; ++r) x[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        if (f + 1 < F) read(f + 1);
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+#pragma unroll
+            for (int r = 0; r < RB; ++r) {
+                floatx4 &y = x[f / P * RB + r];
+                y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[f & 1][r][ta[i]], t[f % P].t[tb[i]], y, 0, 0, 0);
+            }
+        __builtin_amdgcn_sched_barrier(0);
     }
-    if (lane < 16) ex[lane] = inv_scale(scale);
-}
-// An accumulator column block as the second operand: T tiles of 16 rows.
-// Returns the column's 2^-s.
-template <int T> __device__ __forceinline__ float split_columns(const floatx4 *x, halfx8 *hi, halfx8 *lo) {
     float mx = 0.f;
 #pragma unroll
-    for (int t = 0; t < T; ++t) mx = max4(mx, x[t]);
-    const float scale = f16_scale(max_groups(mx));
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int t = 0; t < T; t += 2) split_pair(x[t], x[t + 1], scale, &hi[t / 2], &lo[t / 2]);
-    return inv_scale(scale);
+        for (int i = 0; i < 4; ++i) mx = __builtin_elementwise_maximum(mx, __builtin_fabsf(x[r][i]));
+    if (__builtin_expect(__any(!(mx < __builtin_inff())), 0)) { // (maximum() keeps a NaN)
+#pragma unroll
+        for (int r = 0; r < R; ++r) x[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+        products_f32<R, 2 * P>(src, lane, b, x);
+    }
 }
 
 // Element idx of a wave-uniform array: one scalar base and a 32-bit offset per
