@@ -34,8 +34,9 @@ constexpr size_t kFlushBytes = size_t(64) << 20;
 // 8192 x 2048 x 128 50 and 43 us; 148 x 2048 x 2048 23 and 39 us,
 // 8192 x 128 x 2048 41 and 61 us and 1024 x 1408 x 256 22 and 28 us stay.
 // Below 128 rows a product is bound by reading its weights, not by the cores.
+// (Beyond 2^20 elements of a contraction a row's record could overflow.)
 bool split_pays(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, bool b_kept) {
-    if (M < 128 || N < 128 || Kd < 64) return false;
+    if (M < 128 || N < 128 || Kd < 64 || Kd > (int64_t(1) << 20)) return false;
     const double gain = 2.0 * (double)M * (double)N * (double)Kd * (1 / 145e12 - 1 / 400e12);
     const auto cost = [](double n, bool trans) { return trans ? 20e-6 + n * 12 / 4.5e12 : 14e-6 + n * 8 / 4.5e12; };
     return gain > cost((double)M * (double)Kd, ta) + (b_kept ? 0.0 : cost((double)N * (double)Kd, !tb));
@@ -177,7 +178,10 @@ bool Gemm::run_split(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const f
     p.A = A; p.B = B; p.C = C; p.lda = lda; p.ldb = ldb; p.ldc = ldc; p.M = M; p.N = N; p.Kd = Kd;
     p.beta = beta; p.ta = ta; p.tb = tb;
     p.vec_c = reinterpret_cast<uintptr_t>(C) % 16 == 0 && ldc % 4 == 0;
-    const size_t part = (plan_split_gemm(&p) + 255) & ~(size_t)255;
+    const size_t sums = (plan_split_gemm(&p) + 255) & ~(size_t)255;
+    size_t flags, failed;
+    split_redo_bytes(p, &flags, &failed);
+    const size_t part = sums + flags + failed;
     const size_t fa = split_frag_bytes(M, Kd), sa = split_stat_bytes(M);
     const size_t fb = split_frag_bytes(N, Kd), sb = split_stat_bytes(N);
     const size_t need = part + fa + sa + (w ? 0 : fb + sb);
@@ -203,6 +207,8 @@ bool Gemm::run_split(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const f
     }
     char *base = static_cast<char *>(sws_.ptr());
     p.part = reinterpret_cast<float *>(base);
+    p.redo = reinterpret_cast<unsigned char *>(base + sums);
+    p.failed = reinterpret_cast<unsigned short *>(base + sums + flags);
     void *fra = base + part;
     SplitStat *sta = reinterpret_cast<SplitStat *>(base + part + fa);
     if (!check(launch_split(A, lda, ta, M, Kd, fra, sta, s))) return true;

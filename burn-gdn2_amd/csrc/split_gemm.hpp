@@ -7,8 +7,10 @@
 
 namespace gdn2 {
 
+// What a row of a split operand records about its elements.
 struct SplitStat {
-    unsigned amax, small, nonzero;
+    unsigned amax; // bits of the largest magnitude (NaN > infinity > every finite value)
+    unsigned lost; // sum of what its small elements lose, in units of 2^-36 of its scale
 };
 
 struct SplitGemmParams {
@@ -21,6 +23,10 @@ struct SplitGemmParams {
     const void *fa, *fb;   // the split operands: rows of op(A), columns of op(B)
     const SplitStat *sa, *sb;
     float *part;           // partial sums of the tiles cut along the contraction
+    // the 32 x 32 parts whose outputs are formed again by redo_kernel, eight bytes
+    // of flags a tile, and which outputs of them (16 bits a lane)
+    unsigned char *redo;
+    unsigned short *failed;
     // plan_split_gemm:
     int tile, KT;
     unsigned ntm, ntn, split, whole;
@@ -36,6 +42,7 @@ hipError_t launch_split(const float *src, int64_t ld, bool trans, int64_t rows, 
                         hipStream_t s);
 // Fills the plan of p from M, N, Kd; returns the bytes of `part`.
 size_t plan_split_gemm(SplitGemmParams *p);
+void split_redo_bytes(const SplitGemmParams &p, size_t *flags, size_t *failed);
 hipError_t launch_split_gemm(const SplitGemmParams &p, hipStream_t s);
 
 }  // namespace gdn2

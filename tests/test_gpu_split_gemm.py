@@ -155,3 +155,74 @@ def test_backward_products_match_oracle(gpu):
         # the layer tests' bound, max |error| <= 1e-4 max |reference|, on the sum of both calls
         assert maxabs(twice.get(n), 2 * ref.params[n]) <= 2e-4 * scale + 1e-7, n
     assert maxabs(dx.cpu().numpy(), ref.dx) <= 1e-4 * float(np.abs(ref.dx).max()) + 1e-7
+
+
+def _folded(torch, gpu, D, rows, large, p, seed, zero=False):
+    """A layer and an input whose `large` channels are 2^p larger, read by
+    weights that fold that back (or are zero there)."""
+    _, layer = _layer(D)
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(seed)
+    x = torch.randn((1, rows, D), generator=gen, device=gpu)
+    big = torch.rand(D, generator=gen, device=gpu) < large
+    x[:, :, big] *= 2.0 ** p
+    for n in ("b_proj", "w_proj"):
+        W = layer.param(n)
+        W[big.cpu().numpy()] *= 0.0 if zero else np.float32(2.0 ** -p)
+        layer.set_param(n, W)
+    return layer, x
+
+
+@pytest.mark.parametrize("zero", [False, True], ids=["folded", "unread"])
+@pytest.mark.parametrize("large", [0.02, 0.5, 0.56, 0.98])
+@pytest.mark.parametrize("p", [12, 18, 21, 30, 41, 70])
+def test_channels_of_very_different_sizes(gpu, p, large, zero):
+    """Each output keeps the product's bound whatever share of its row is large:
+    what small elements lose of their row's largest is at most 2^-21 of the
+    output, or the output is formed in f32."""
+    import torch
+
+    layer, x = _folded(torch, gpu, 1040, 1500, large, p, p, zero)
+    _check_products(torch, layer, x, layer.project(x))
+
+
+@pytest.mark.parametrize("T", [700, 9000])
+@pytest.mark.parametrize("last", [1, 64])
+def test_gradients_that_decay_over_the_tokens(gpu, T, last):
+    """A loss on the last tokens only: the gradients of the projected columns
+    fall off exponentially over the tokens that dW = x^T dY contracts."""
+    import torch
+
+    import gdn2_amd as G
+
+    B, D = 1, 1040
+    cfg, layer = _layer(D)
+    layer.set_param("a_log", np.full(4, 1.0, np.float32))
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(T + last)
+    x = torch.randn((B, T, D), generator=gen, device=gpu)
+    d = torch.zeros_like(x)
+    d[:, -last:] = torch.randn((B, last, D), generator=gen, device=gpu)
+    dx, grads, _ = layer.backward(x, d)
+    if T < 1000:
+        ref = O.layer_backward_f64(cfg, layer.params(), x.cpu().numpy(), d.cpu().numpy(), None, None)
+        for n in ("q_proj", "k_proj", "b_proj", "v_proj", "w_proj", "f_proj_0", "g_proj_0", "o_proj"):
+            scale = float(np.abs(ref.params[n]).max())
+            assert maxabs(grads.get(n), ref.params[n]) <= 1e-4 * scale + 1e-12, n
+        assert maxabs(dx.cpu().numpy(), ref.dx) <= 1e-4 * float(np.abs(ref.dx).max())
+    # linear in d.  (Not bit for bit: the tails underflow at other tokens.)  Each side
+    # is off by at most 2^-20 of the sum of its terms' magnitudes, which is below
+    # the largest output's times the 2^7 tokens or fewer that matter
+    again = layer.backward(x, d * 2.0 ** -20)[1]
+    for n in ("k_proj", "b_proj", "w_proj"):
+        a, b = again.get(n) * np.float32(2.0 ** 20), grads.get(n)
+        assert maxabs(a, b) <= 2.0 ** -12 * float(np.abs(b).max()), n
+
+
+def test_products_are_reproducible(gpu):
+    import torch
+
+    layer, x = _folded(torch, gpu, 1040, 1500, 0.5, 19, 3)
+    first = layer.project(x)["b"].clone()
+    for _ in range(3):
+        assert torch.equal(layer.project(x)["b"], first)
