@@ -195,15 +195,10 @@ bool Gemm::run_split(bool ta, bool tb, int64_t M, int64_t N, int64_t Kd, const f
         return e == hipSuccess;
     };
     *st = GDN2_OK;
-    if (w && !w->frags) {
-        void *buf = nullptr;
-        if (recording_ || hipMalloc(&buf, fb + sb) != hipSuccess) {
-            (void)hipGetLastError();
-            return false;
-        }
-        w->frags = buf;
-        w->stat = reinterpret_cast<SplitStat *>(static_cast<char *>(buf) + fb);
-        if (!check(w->refresh(s))) return true;
+    if (w) {
+        hipError_t e = hipSuccess;
+        if (!w->ready(s, recording_, &e)) return false;
+        if (!check(e)) return true;
     }
     char *base = static_cast<char *>(sws_.ptr());
     p.part = reinterpret_cast<float *>(base);

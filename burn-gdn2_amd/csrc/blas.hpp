@@ -21,25 +21,6 @@
 
 namespace gdn2 {
 
-// A weight matrix as the second operand of split products, split once: the
-// owner calls refresh() whenever the weight's values change, so that captured
-// graphs, which read the split copy, keep seeing the current values.
-struct SplitWeight {
-    const float *src = nullptr; // [rows of the stored matrix, cols], row stride ld
-    int64_t ld = 0, rows = 0, Kd = 0; // rows of the operand (N of the product) and its contraction
-    bool trans = false;         // the operand's rows are src's columns
-    void *frags = nullptr;      // allocated by the first product that uses it
-    SplitStat *stat = nullptr;
-    hipError_t refresh(hipStream_t s) const {
-        return frags ? launch_split(src, ld, trans, rows, Kd, frags, stat, s) : hipSuccess;
-    }
-    void destroy() {
-        if (frags) (void)hipFree(frags);
-        frags = nullptr;
-        stat = nullptr;
-    }
-};
-
 class Gemm {
   public:
     gdn2_status init();

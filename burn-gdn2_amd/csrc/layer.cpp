@@ -602,13 +602,13 @@ extern "C" gdn2_status gdn2_layer_set_param(gdn2_layer *L, const char *name, con
     const OnDevice on(L->device);
     GDN2_HIP_CHECK(off >= 0 ? L->stage.copy(L->w_in + off, L->ld_in, const_cast<float *>(host), rows, cols, false)
                             : L->stage.copy(L->p[id], cols, const_cast<float *>(host), rows, cols, false));
-    // the split copies that products (and captured graphs) already read
     const float *changed = off >= 0 ? L->w_in : L->p[id];
     bool any = false;
     for (SplitWeight *w : {&L->sw_in, &L->sw_in_t, &L->sw_o, &L->sw_o_t, &L->sw_f1, &L->sw_g1})
-        if (w->frags && w->src == changed) {
-            GDN2_HIP_CHECK(w->refresh(nullptr));
-            any = true;
+        if (w->src == changed) {
+            hipError_t e = hipSuccess;
+            any |= w->changed(&e);
+            GDN2_HIP_CHECK(e);
         }
     if (any) GDN2_HIP_CHECK(hipStreamSynchronize(nullptr));
     return GDN2_OK;

@@ -31,6 +31,8 @@
 // times more roundings of the running sum).
 #include "split_gemm.hpp"
 
+#include "common.hpp"
+
 namespace gdn2 {
 namespace {
 

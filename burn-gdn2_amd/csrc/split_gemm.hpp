@@ -1,9 +1,11 @@
 // f32 matrix products on the f16 matrix cores (split_gemm.hip).
 #pragma once
 
-#include <algorithm>
+#include <hip/hip_runtime_api.h>
 
-#include "common.hpp"
+#include <algorithm>
+#include <cstddef>
+#include <cstdint>
 
 namespace gdn2 {
 
@@ -44,5 +46,57 @@ hipError_t launch_split(const float *src, int64_t ld, bool trans, int64_t rows, 
 size_t plan_split_gemm(SplitGemmParams *p);
 void split_redo_bytes(const SplitGemmParams &p, size_t *flags, size_t *failed);
 hipError_t launch_split_gemm(const SplitGemmParams &p, hipStream_t s);
+
+// A weight matrix as the second operand of split products, whose terms are kept
+// between them.  Its owner says when the values change; the next product then
+// splits it again, or, once a captured graph reads the terms, changed() does.
+struct SplitWeight {
+    const float *src = nullptr;       // [rows of the stored matrix, cols], row stride ld
+    int64_t ld = 0, rows = 0, Kd = 0; // rows of the operand (N of the product) and its contraction
+    bool trans = false;               // the operand's rows are src's columns
+    void *frags = nullptr;            // allocated by the first product that uses it
+    SplitStat *stat = nullptr;
+
+    // The terms of the present values, for work on s; false: no memory for them
+    // (a call that is being recorded allocates none).
+    bool ready(hipStream_t s, bool recording, hipError_t *e) {
+        *e = hipSuccess;
+        if (!frags) {
+            const size_t fb = split_frag_bytes(rows, Kd);
+            void *buf = nullptr;
+            if (recording || hipMalloc(&buf, fb + split_stat_bytes(rows)) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
+            frags = buf;
+            stat = reinterpret_cast<SplitStat *>(static_cast<char *>(buf) + fb);
+        }
+        if (!fresh_) {
+            *e = launch_split(src, ld, trans, rows, Kd, frags, stat, s);
+            fresh_ = *e == hipSuccess && !recording; // (what is recorded runs with each replay)
+        }
+        recorded_ = recorded_ || recording;
+        return true;
+    }
+    // The values have changed: returns whether a split was queued (on the null stream).
+    bool changed(hipError_t *e) {
+        *e = hipSuccess;
+        fresh_ = false;
+        if (!recorded_) return false;
+        *e = launch_split(src, ld, trans, rows, Kd, frags, stat, nullptr);
+        fresh_ = *e == hipSuccess;
+        return true;
+    }
+    void destroy() {
+        if (frags) (void)hipFree(frags);
+        frags = nullptr;
+        stat = nullptr;
+        fresh_ = recorded_ = false;
+    }
+
+  private:
+    bool fresh_ = false;    // the terms are those of the present values
+    bool recorded_ = false; // a captured graph reads them
+};
 
 }  // namespace gdn2

@@ -21,7 +21,12 @@
  * owns its parameters and a workspace in device memory (allocated on the
  * device current at gdn2_layer_create; the workspace grows on the first
  * call at a larger batch x tokens, and a block that a captured graph was
- * recorded with is kept until gdn2_layer_destroy).  x and out are caller-owned device
+ * recorded with is kept until gdn2_layer_destroy).  Beside them it keeps, for
+ * its large matrix products, from the first one on: f16 copies of the Linear
+ * weights as large as these (forward only; twice that with the backward), a
+ * workspace of 4 bytes per element of a product's activations (default layer:
+ * 0.3 GB for a forward and 1.6 GB for a backward of 32768 tokens, 0.5 GB for a
+ * backward of 8192), and 8 MB of pinned host memory for parameter copies.  x and out are caller-owned device
  * buffers [B, T, hidden_size], contiguous f32.  Calls are asynchronous on
  * `stream`; calls on one layer must not overlap (they share the workspace).
  */
