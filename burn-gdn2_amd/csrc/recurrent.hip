@@ -201,6 +201,106 @@ __global__ __launch_bounds__(64 * NW) void scan_kernel(ScanParams p) {
                 make_float2(S[j][i][0], S[j][i][1]);
 }
 
+// The same for a few tokens, where reading and writing S counts: K rows x VS
+// columns per workgroup of 256 lanes, lane t with the 4 contiguous columns 4 (t
+// % (VS / 4)) of rows t / (VS / 4) + i RPP, so that a state row is read and
+// written in runs of 256 bytes (of 64 by scan_kernel), but a token takes three
+// barriers.
+template <int K, int VS>
+__global__ __launch_bounds__(256) void scan_few_kernel(ScanParams p) {
+    constexpr int TPR = VS / 4;    // lanes per state row
+    constexpr int RPP = 256 / TPR; // rows covered by one pass of the workgroup
+    constexpr int NP = K / RPP;    // float4 registers of S per lane
+    static_assert(VS % 4 == 0 && TPR <= 64 && 64 % TPR == 0, "VS");
+    static_assert(K % RPP == 0, "K");
+
+    const int nvs = p.V / VS;
+    const int bh = blockIdx.x / nvs, vsl = blockIdx.x % nvs;
+    const int bi = bh / p.HV, hv = bh % p.HV, hk = hv / p.rep;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int cg = tid % TPR, r0 = tid / TPR;
+
+    __shared__ float s_eg[2][K], s_a1[2][K], s_a2[2][K], s_k[2][K];
+    __shared__ float s_red[2][4][VS];
+    __shared__ float s_vn[VS];
+    __shared__ float s_kq[4];
+
+    const size_t sbase = (size_t)bh * K * p.V + (size_t)vsl * VS + cg * 4;
+    float4 S[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+        S[i] = *reinterpret_cast<const float4 *>(p.state_in + sbase + (size_t)(r0 + i * RPP) * p.V);
+
+    const int64_t koff = (int64_t)bi * p.sqb + (int64_t)hk * p.sqh;
+    const int64_t voff = (int64_t)bi * p.svb + (int64_t)hv * p.svh;
+    const int64_t ooff = (int64_t)bi * p.sob + (int64_t)hv * p.soh;
+
+    for (int t = 0; t < p.T; ++t) {
+        const int buf = t & 1;
+        float kq = 0.0f;
+        for (int r = tid; r < K; r += 256) {
+            const int64_t o = koff + (int64_t)t * p.sqt + r;
+            const float qq = p.q[o], kk = p.k[o], gg = p.g[o], bb = p.b[o];
+            const float eg = expf(gg);
+            s_eg[buf][r] = eg;
+            s_a1[buf][r] = eg * (bb * kk);
+            s_a2[buf][r] = eg * qq;
+            s_k[buf][r] = kk;
+            kq += kk * qq;
+        }
+        kq = wave_sum(kq);
+        if (lane == 0) s_kq[wave] = kq;
+        __syncthreads();
+
+        float e1[4] = {0.f, 0.f, 0.f, 0.f}, e2[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const int r = r0 + i * RPP;
+            const float a1 = s_a1[buf][r], a2 = s_a2[buf][r];
+            e1[0] += S[i].x * a1; e1[1] += S[i].y * a1; e1[2] += S[i].z * a1; e1[3] += S[i].w * a1;
+            e2[0] += S[i].x * a2; e2[1] += S[i].y * a2; e2[2] += S[i].z * a2; e2[3] += S[i].w * a2;
+        }
+#pragma unroll
+        for (int off = TPR; off < 64; off <<= 1)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                e1[j] += __shfl_xor(e1[j], off, 64);
+                e2[j] += __shfl_xor(e2[j], off, 64);
+            }
+        if (lane < TPR)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                s_red[0][wave][cg * 4 + j] = e1[j];
+                s_red[1][wave][cg * 4 + j] = e2[j];
+            }
+        __syncthreads();
+        if (tid < VS) {
+            const float E1 = s_red[0][0][tid] + s_red[0][1][tid] + s_red[0][2][tid] + s_red[0][3][tid];
+            const float E2 = s_red[1][0][tid] + s_red[1][1][tid] + s_red[1][2][tid] + s_red[1][3][tid];
+            const float kqs = s_kq[0] + s_kq[1] + s_kq[2] + s_kq[3];
+            const int col = vsl * VS + tid;
+            const int64_t vo = voff + (int64_t)t * p.svt + col;
+            const float vn = p.w[vo] * p.v[vo] - E1;
+            p.out[ooff + (int64_t)t * p.sot + col] = p.scale * (E2 + vn * kqs);
+            s_vn[tid] = vn;
+        }
+        __syncthreads();
+        const float4 vn = *reinterpret_cast<const float4 *>(&s_vn[cg * 4]);
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const int r = r0 + i * RPP;
+            const float eg = s_eg[buf][r], kk = s_k[buf][r];
+            S[i].x = S[i].x * eg + kk * vn.x;
+            S[i].y = S[i].y * eg + kk * vn.y;
+            S[i].z = S[i].z * eg + kk * vn.z;
+            S[i].w = S[i].w * eg + kk * vn.w;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+        *reinterpret_cast<float4 *>(p.state_out + sbase + (size_t)(r0 + i * RPP) * p.V) = S[i];
+}
+
 // Any K, V (<= 1024): one workgroup per (b, hv), the state is updated in
 // place in state_out (copied from state_in first), each column owned by one
 // lane for the whole launch.  Used for shapes the register kernel does not
@@ -702,17 +802,31 @@ __global__ __launch_bounds__(256) void decode_fused_generic_kernel(DecodeParams 
     }
 }
 
-// Up to two workgroups a unit a token is a chain of LDS reads, sums and
-// exchanges, and reading ahead (178 registers at K = 128) shortens it: 4
-// sequences of 37 tokens at 16 heads 25 against 34 us.  Beyond, four waves a
-// SIMD (127 registers) hide it better: 32 sequences of 48 tokens 75 against 82.
+// A few tokens: scan_few_kernel, whose 256-byte state rows outweigh its barriers.
+// scan / few kernel, us, at K x V and 16 heads of 64 sequences: 64 x 256 one token
+// 31 / 23, three 31 / 30, four 32 / 35; 64 x 96 three 19 / 22; 128 x 256 two 72 / 51,
+// four 81 / 69, six 82 / 85; 128 x 128 four 35 / 33, five 35 / 37; 256 x 256 one
+// 136 / 105, six 155 / 154, eight 166 / 179; no difference at few sequences.
+constexpr int few_tokens(int K) { return K <= 64 ? 2 : K <= 128 ? 4 : 6; }
+// Reading ahead shortens a token's chain of LDS reads, sums and exchanges, and
+// holds more registers: it pays until they keep a second (K = 256: the first)
+// workgroup of four waves off a unit.  On / off, us, 37 tokens: K = 128 64
+// workgroups 25 / 33, 512 37 / 39, 640 54 / 46; K = 256 256 46 / 49, 384 83 / 59;
+// K = 64 512 23 / 23, 2048 57 / 59; two waves K = 128 512 33 / 33, 2048 85 / 89,
+// K = 256 1024 96 / 107.
+constexpr int ahead_grid(int K, int NW) { return NW < 4 || K <= 64 ? 0x7fffffff : K <= 128 ? 512 : 256; }
 template <int K, int NW>
 hipError_t launch_scan_t(const ScanParams &p, hipStream_t s) {
     const int grid = p.B * p.HV * (p.V / (16 * NW));
-    if (grid <= 512)
+    constexpr int kAhead = ahead_grid(K, NW);
+    if (p.T <= few_tokens(K)) {
+        hipLaunchKernelGGL((scan_few_kernel<K, 16 * NW>), dim3(grid), dim3(256), 0, s, p);
+    } else if (grid <= kAhead) {
         hipLaunchKernelGGL((scan_kernel<K, NW, true>), dim3(grid), dim3(64 * NW), 0, s, p);
-    else
-        hipLaunchKernelGGL((scan_kernel<K, NW, false>), dim3(grid), dim3(64 * NW), 0, s, p);
+    } else {
+        if constexpr (kAhead != 0x7fffffff)
+            hipLaunchKernelGGL((scan_kernel<K, NW, false>), dim3(grid), dim3(64 * NW), 0, s, p);
+    }
     return hipGetLastError();
 }
 

@@ -26,9 +26,10 @@
  * weights as large as these (forward only; twice that with the backward), a
  * workspace of 4 bytes per element of a product's activations (default layer:
  * 0.3 GB for a forward and 1.6 GB for a backward of 32768 tokens, 0.5 GB for a
- * backward of 8192), and 8 MB of pinned host memory for parameter copies.  x and out are caller-owned device
- * buffers [B, T, hidden_size], contiguous f32.  Calls are asynchronous on
- * `stream`; calls on one layer must not overlap (they share the workspace).
+ * backward of 8192), and 8 MB of pinned host memory for parameter copies.
+ * x and out are caller-owned device buffers [B, T, hidden_size], contiguous
+ * f32.  Calls are asynchronous on `stream`; calls on one layer must not
+ * overlap (they share the workspace).
  */
 #ifndef GDN2_LAYER_H_
 #define GDN2_LAYER_H_
