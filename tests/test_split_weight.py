@@ -93,19 +93,18 @@ def test_weights_set_before_and_after_a_capture(gpu):
         layer.forward_train(x)
     torch.cuda.synchronize()
     layer.load_params(other.params())  # between the eager call and the capture
-    want = other.forward_train(x)
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
         out = layer.forward_train(x)
     rng = np.random.default_rng(1)
     for step in range(3):
+        out.zero_()
         g.replay()
         torch.cuda.synchronize()
-        assert torch.equal(out, want), step
-        assert torch.equal(layer.forward_train(x), want), step
+        want = other.forward_train(x)  # (its library products may sum in another order: 2^-24 times their terms)
+        assert float((out - want).abs().max()) <= D * 2.0 ** -24 * float(want.abs().max()), step
+        assert torch.equal(layer.forward_train(x), out), step
         for n in ("q_proj", "b_proj", "o_proj", "f_proj_1"):
             W = (layer.param(n) * rng.uniform(0.5, 1.5, layer.param(n).shape)).astype(np.float32)
             layer.set_param(n, W)
             other.set_param(n, W)
-        want = other.forward_train(x)
-        out.zero_()
