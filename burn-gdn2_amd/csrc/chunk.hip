@@ -1805,8 +1805,12 @@ struct WsLayout {
 // 103, B = 4, T = 512, 4 heads of 128 76 against 65 / 225 against 187; with
 // more segments B = 2, T = 2048, 2 heads, V = 96 (16) 56.0 against 58.0, T =
 // 4096, 4 heads of 128 (32) 112 against 138; K = 256 (T = 1024, 8 heads) 166
-// against 184; below 8 chunks (T = 300) one segment, 36.8 against 42.4.  Not where the workspace would then outgrow the no-allocation entry's
-// scratch, so that that entry's range does not depend on this rule.
+// against 184; below 8 chunks (T = 300) one segment, 36.8 against 42.4.  Not
+// where the workspace would then outgrow the no-allocation entry's scratch, so
+// that that entry's range does not depend on this rule; and not where the
+// caller's workspace holds only the segments of 4 chunks (shorten = false), since
+// the short ones need more at some sizes than at larger ones (64 sequences of 8
+// chunks, K = V = 64, more than 66): whatever held a call before this rule does.
 constexpr int64_t kInterWorkgroups = 256;
 constexpr int64_t kMinSegmentChunks = 4, kMinShortSegmentChunks = 2, kMaxShortSegments = 8;
 
@@ -1839,40 +1843,39 @@ WsLayout ws_layout(int64_t seqs, int64_t NC, int64_t K, int64_t V, int64_t nseg)
     return L;
 }
 
-Segments inter_segments(int64_t B, int64_t HV, int64_t K, int64_t V, int64_t NC) {
-    const int64_t w = (K > 0 && V > 0) ? B * HV * (V / (16 * inter_nwv((int)K, (int)V))) : 0;
+Segments inter_segments(int64_t seqs, int64_t K, int64_t V, int64_t NC, bool shorten) {
+    const int64_t w = (K > 0 && V > 0) ? seqs * (V / (16 * inter_nwv((int)K, (int)V))) : 0;
     if (w <= 0 || NC <= 0) return {1, (int)NC}; // (K, V) outside the chunk kernels, or no tokens
     const int64_t fill = kInterWorkgroups / w;
     const int64_t n = std::min(fill, NC / kMinSegmentChunks);
     const int64_t ns = std::min({fill, NC / kMinShortSegmentChunks, kMaxShortSegments});
-    if (K <= 128 && NC >= 2 * kMinSegmentChunks && ns > n) {
+    if (shorten && K <= 128 && NC >= 2 * kMinSegmentChunks && ns > n) {
         const Segments sg = segments_of(ns, NC);
-        if (ws_layout(B * HV, NC, K, V, sg.nseg).total <= kNoallocScratchBytes) return sg;
+        if (ws_layout(seqs, NC, K, V, sg.nseg).total <= kNoallocScratchBytes) return sg;
     }
     return segments_of(n, NC);
 }
 
-// Workspace of a sequence of NC chunks.  Short segments make their count fall
-// at some longer lengths (8 chunks: four segments, 9 chunks: three), so the
-// size also covers every shorter length whose segments are short: a workspace
-// for the longest sequence serves the shorter ones.  (A segment's P and entering
-// state are at most 1.1 times a chunk's operands, and 8 segments the most:
-// lengths further below than 8 chunks need less.)
-size_t ws_bytes(int64_t seqs, int64_t NC, int64_t K, int64_t V) {
-    size_t most = ws_layout(seqs, NC, K, V, inter_segments(seqs, 1, K, V, NC).nseg).total;
-    const int64_t last = K <= 128 ? std::min(NC - 1, kMinSegmentChunks * kMaxShortSegments - 1) : 0;
-    for (int64_t m = std::max(2 * kMinSegmentChunks, NC - 8); m <= last; ++m)
-        most = std::max(most, ws_layout(seqs, m, K, V, inter_segments(seqs, 1, K, V, m).nseg).total);
-    return most;
-}
-size_t ws_bytes(const gdn2_chunk_args *a) {
-    return ws_bytes(a->batch * a->num_v_heads, (a->seq_len + kChunk - 1) / kChunk, a->head_dim, a->head_v_dim);
-}
-
-WsLayout ws_layout(const gdn2_chunk_args *a) {
+WsLayout ws_layout(const gdn2_chunk_args *a, bool shorten) {
     const int64_t seqs = a->batch * a->num_v_heads, NC = (a->seq_len + kChunk - 1) / kChunk;
     return ws_layout(seqs, NC, a->head_dim, a->head_v_dim,
-                     inter_segments(seqs, 1, a->head_dim, a->head_v_dim, NC).nseg);
+                     inter_segments(seqs, a->head_dim, a->head_v_dim, NC, shorten).nseg);
+}
+
+// Workspace that a call asks for.  Short segments make their count fall at some
+// longer lengths (8 chunks: four segments, 9 chunks: three); up to 31 chunks the
+// size also covers the shorter lengths whose segments are short, so that a
+// workspace for the longest sequence serves the shorter ones in the same
+// segments.  (Elsewhere a shorter sequence may find room for the segments of 4
+// chunks only.)
+size_t ws_bytes(const gdn2_chunk_args *a) {
+    const int64_t seqs = a->batch * a->num_v_heads, NC = (a->seq_len + kChunk - 1) / kChunk, K = a->head_dim,
+                  V = a->head_v_dim;
+    size_t most = ws_layout(a, true).total;
+    const int64_t last = K <= 128 ? std::min(NC - 1, kMinSegmentChunks * kMaxShortSegments - 1) : 0;
+    for (int64_t m = std::max(2 * kMinSegmentChunks, NC - 8); m <= last; ++m)
+        most = std::max(most, ws_layout(seqs, m, K, V, inter_segments(seqs, K, V, m, true).nseg).total);
+    return most;
 }
 
 bool aligned16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
@@ -1927,20 +1930,24 @@ gdn2_status chunk_setup(const gdn2_chunk_args *a, const char *who, bool need_out
     p->svb = a->stride_vw_b; p->svh = a->stride_vw_h; p->svt = a->stride_vw_t;
     p->sob = a->stride_o_b; p->soh = a->stride_o_h; p->sot = a->stride_o_t;
     p->scale = (float)a->scale;
-    const Segments sg = inter_segments(p->B * p->HV, 1, p->K, p->V, p->NC);
+    return GDN2_OK;
+}
+
+size_t chunk_fwd_ws_bytes(const gdn2_chunk_args *a, bool shorten) {
+    return shorten ? ws_bytes(a) : ws_layout(a, false).total;
+}
+
+int chunk_segments(int64_t seqs, int64_t K, int64_t V, int64_t NC, bool shorten) {
+    return inter_segments(seqs, K, V, NC, shorten).nseg;
+}
+
+void chunk_bind_ws(const gdn2_chunk_args *a, char *ws, bool shorten, ChunkParams *p) {
+    const Segments sg = inter_segments(p->B * p->HV, p->K, p->V, p->NC, shorten);
     p->NSEG = sg.nseg;
     p->SEGL = sg.segl;
     p->NSLOT = sg.nseg; // uniform runs; the inference split keeps these slots
     p->SEG0 = p->SLOT0 = 0;
-    return GDN2_OK;
-}
-
-size_t chunk_fwd_ws_bytes(const gdn2_chunk_args *a) { return ws_bytes(a); }
-
-int chunk_segments(int64_t seqs, int64_t K, int64_t V, int64_t NC) { return inter_segments(seqs, 1, K, V, NC).nseg; }
-
-void chunk_bind_ws(const gdn2_chunk_args *a, char *ws, ChunkParams *p) {
-    const WsLayout L = ws_layout(a);
+    const WsLayout L = ws_layout(a, shorten);
     p->ws_w = reinterpret_cast<float *>(ws + L.w);
     p->ws_qg = reinterpret_cast<float *>(ws + L.qg);
     p->ws_u = reinterpret_cast<float *>(ws + L.u);
@@ -1962,9 +1969,11 @@ static gdn2_status chunk_call(const gdn2_chunk_args *a, gdn2_stream_t stream, in
     const gdn2_status st = chunk_setup(a, who, true, &p);
     if (st != GDN2_OK) return st;
     if (a->seq_len == 0) return GDN2_OK;
-    if (!a->workspace || a->workspace_bytes < chunk_fwd_ws_bytes(a) || (reinterpret_cast<uintptr_t>(a->workspace) & 255u))
+    const bool shorten = a->workspace_bytes >= ws_layout(a, true).total;
+    if (!a->workspace || (!shorten && a->workspace_bytes < chunk_fwd_ws_bytes(a, false)) ||
+        (reinterpret_cast<uintptr_t>(a->workspace) & 255u))
         return fail(GDN2_EINVAL, std::string(who) + ": workspace missing, too small or not 256-byte aligned");
-    chunk_bind_ws(a, static_cast<char *>(a->workspace), &p);
+    chunk_bind_ws(a, static_cast<char *>(a->workspace), shorten, &p);
     p.ws_vn = v_new;
     p.ws_sn = states;
     if (st_cc) {
@@ -1991,7 +2000,8 @@ extern "C" gdn2_status gdn2_chunk_inter_f32(const gdn2_chunk_args *a, gdn2_strea
 extern "C" int64_t gdn2_chunk_segments(const gdn2_chunk_args *a) {
     if (!a || a->batch <= 0 || a->num_v_heads <= 0 || a->seq_len <= 0 || a->head_dim <= 0 || a->head_v_dim <= 0)
         return 0;
-    return chunk_segments(a->batch * a->num_v_heads, a->head_dim, a->head_v_dim, (a->seq_len + kChunk - 1) / kChunk);
+    return chunk_segments(a->batch * a->num_v_heads, a->head_dim, a->head_v_dim, (a->seq_len + kChunk - 1) / kChunk,
+                          !a->workspace || a->workspace_bytes >= ws_layout(a, true).total);
 }
 
 extern "C" gdn2_status gdn2_chunk_inter_pass_f32(const gdn2_chunk_args *a, int pass, gdn2_stream_t stream) {

@@ -1274,11 +1274,11 @@ struct BwdLayout {
     size_t fwd, wt, qgt, kd, aqkt, akk, sn, vn, dsn, dvn, dqg, rseg, dkd, daqk, dgam, drk, dakk, kgrad, total;
 };
 
-BwdLayout bwd_layout(const gdn2_chunk_args *a) {
+BwdLayout bwd_layout(const gdn2_chunk_args *a, bool shorten) { // (chunk_fwd_ws_bytes)
     BwdLayout L;
     const size_t nch = (size_t)a->batch * a->num_v_heads * ((a->seq_len + kChunk - 1) / kChunk);
     const size_t K = a->head_dim, V = a->head_v_dim, Cs = kChunk, f = sizeof(float);
-    size_t off = align256(chunk_fwd_ws_bytes(a));
+    size_t off = align256(chunk_fwd_ws_bytes(a, shorten));
     L.fwd = 0;
     auto take = [&](size_t elems) { const size_t o = off; off = align256(off + f * nch * elems); return o; };
     L.wt = take(Cs * K);
@@ -1299,7 +1299,7 @@ BwdLayout bwd_layout(const gdn2_chunk_args *a) {
     L.kgrad = take(a->num_v_heads != a->num_heads ? 4 * Cs * K : 0);
     { // segment buffers of the reverse recurrence, per sequence (not per chunk)
         const size_t seqs = (size_t)a->batch * a->num_v_heads, NC = (a->seq_len + kChunk - 1) / kChunk;
-        const size_t nseg = (size_t)chunk_segments(seqs, K, V, NC);
+        const size_t nseg = (size_t)chunk_segments(seqs, K, V, NC, shorten);
         const size_t ns = nseg > 1 ? seqs * nseg : 0;
         L.rseg = off; off = align256(off + f * ns * K * V);
     }
@@ -1318,7 +1318,7 @@ extern "C" size_t gdn2_chunk_bwd_workspace_bytes(const gdn2_chunk_bwd_args *a) {
     if (!a || a->fwd.batch <= 0 || a->fwd.num_v_heads <= 0 || a->fwd.seq_len <= 0 || a->fwd.head_dim <= 0 ||
         a->fwd.head_v_dim <= 0)
         return 0;
-    return bwd_layout(&a->fwd).total;
+    return bwd_layout(&a->fwd, true).total;
 }
 
 namespace {
@@ -1350,11 +1350,14 @@ gdn2_status chunk_bwd_call(const gdn2_chunk_bwd_args *a, gdn2_stream_t stream, i
             GDN2_HIP_CHECK(launch_fill_rows(a->d_state0, 0, a->d_state_out, 1, (int64_t)(sbytes / sizeof(float)), s));
         return GDN2_OK;
     }
-    const BwdLayout L = bwd_layout(&f);
+    // (the training forward and its backward get the same workspace_bytes)
+    BwdLayout L = bwd_layout(&f, true);
+    const bool shorten = a->workspace_bytes >= L.total;
+    if (!shorten) L = bwd_layout(&f, false);
     if (!a->workspace || a->workspace_bytes < L.total || (reinterpret_cast<uintptr_t>(a->workspace) & 255u))
         return fail(GDN2_EINVAL, w + "workspace missing, too small or not 256-byte aligned");
     char *ws = static_cast<char *>(a->workspace);
-    chunk_bind_ws(&f, ws, &bp.f);
+    chunk_bind_ws(&f, ws, shorten, &bp.f);
     ChunkParams &p = bp.f;
     p.ws_wt = reinterpret_cast<float *>(ws + L.wt);
     p.ws_qgt = reinterpret_cast<float *>(ws + L.qgt);

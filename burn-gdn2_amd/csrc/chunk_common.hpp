@@ -361,9 +361,11 @@ __device__ __forceinline__ void chain_walk(floatx4 x, int nsteps, int V, int col
 
 // Host side of the chunked forward, shared with the backward (chunk.hip).
 gdn2_status chunk_setup(const gdn2_chunk_args *a, const char *who, bool need_out, ChunkParams *p);
-size_t chunk_fwd_ws_bytes(const gdn2_chunk_args *a);
+// shorten: with the short segments (inter_segments), as gdn2_chunk_workspace_bytes
+// sizes it; without them, the least a call takes.
+size_t chunk_fwd_ws_bytes(const gdn2_chunk_args *a, bool shorten);
 // Segments per sequence of the sequential kernels (1 = unsegmented).
-int chunk_segments(int64_t seqs, int64_t K, int64_t V, int64_t NC);
-void chunk_bind_ws(const gdn2_chunk_args *a, char *ws, ChunkParams *p);
+int chunk_segments(int64_t seqs, int64_t K, int64_t V, int64_t NC, bool shorten);
+void chunk_bind_ws(const gdn2_chunk_args *a, char *ws, bool shorten, ChunkParams *p);
 
 }  // namespace gdn2

@@ -131,7 +131,9 @@ GDN2_API gdn2_status gdn2_recurrent_fwd_f32(const gdn2_recurrent_args *args, gdn
  * 64-token chunks of four 16-row tiles; any chunk_size > 0 is accepted, since
  * the result does not depend on it beyond rounding, as in the reference.
  * workspace: device memory of at least gdn2_chunk_workspace_bytes(args)
- * bytes, 256-byte aligned.
+ * bytes, 256-byte aligned (one that was sized for more sequences or longer ones
+ * may be a little smaller than that: the call then cuts its sequences into
+ * fewer segments).
  * Limits (else GDN2_NOT_APPLICABLE): (K, V) with K = 32 and V in {32, 64},
  * K = 64 and V in {64, 96, 128, 256}, K = 128 and V in {64, 128, 192, 256},
  * or K = 256 and V in {128, 256} (the reference takes K, V <= 256; these are
@@ -301,7 +303,7 @@ GDN2_API gdn2_status gdn2_chunk_bwd_f32(const gdn2_chunk_bwd_args *args, gdn2_st
  *       the state entering every chunk and v_new.  The gradient pointers are
  *       not read.
  *   gdn2_chunk_bwd_saved_f32  gdn2_chunk_bwd_f32 on that workspace, untouched
- *       since, for the same q, k, g, b, v, w, shapes and strides: the forward's
+ *       since and given with the same workspace_bytes, for the same q, k, g, b, v, w, shapes and strides: the forward's
  *       quantities are read instead of recomputed (args->fwd.state is not read).
  *       The gradients are bit-identical to gdn2_chunk_bwd_f32's.
  * Limits: those of gdn2_chunk_bwd_f32. */
