@@ -253,7 +253,6 @@ def bench_prefill(torch, G, args, dev):
     tokens = B * T
     intra_gflop = B * H * T * 2 * C * (3 * K + V) / 1e9
     inter_gflop = B * H * T * (6 * K * V + 2 * C * V) / 1e9
-    # (chunk-inter's f32 products run as three f16 ones each: its fraction of the f32 peak may pass 1)
     kernels = {
         "chunk_intra": {"ms": intra_ms, "ms_median": _median(intra_all), "gflop": intra_gflop,
                         "tflops": intra_gflop / intra_ms, "frac_f32_mfma": intra_gflop / intra_ms / PEAK_F32_TFLOPS},

@@ -1534,11 +1534,12 @@ __global__ __launch_bounds__(256) void chunk_states_kernel(ChunkParams p) {
 // segment 0's walk takes one value slice per sequence beside pass 1's.
 // Segment 0 gets L0 = r NC / (n + r) chunks and the others L = ceil((NC - L0)
 // / n), so that its walk and pass 1 end together: r = 0.7 (B = 1, T = 32768, 16
-// heads, K = V = 128: 1209 us in all, 1228 at 0.85, 1253 at 1.0, 1291 at 1.2;
-// B = 8, T = 4096, 4 heads, K = 64, V = 96: 242, 244, 247, 249).  Only where
+// heads, K = V = 128: 1321 us in all, 1329 at 0.55, 1350 at 0.85, 1388 at 1.0,
+// 1455 at 1.2; B = 8, T = 4096, 4 heads, K = 64, V = 96: 250, 258, 241, 244, 247;
+// B = 2, T = 4096, 8 heads, K = 64, V = 128: 130, 130, 159, 162, 161).  Only where
 // every segment keeps at least kMinSplitChunks chunks; else the uniform run
-// (16 against 6 chunks: B = 4, T = 2048, 16 heads, K = V = 128 334 against 307
-// us in all, B = 2, T = 3001 with 16 value heads of 256 370 against 329).
+// (16 against 6 chunks: B = 4, T = 2048, 16 heads, K = V = 128 365 against 333
+// us in all, B = 2, T = 3001 with 16 value heads of 256 452 against 393).
 constexpr int kMinSplitChunks = 6;
 
 bool split_segments(const ChunkParams &p, ChunkParams *q) {
@@ -1800,12 +1801,14 @@ struct WsLayout {
 // segment's transition, the chain) costs little beside the shorter walk.
 // For K <= 128 a segment keeps 2 chunks where that makes at most 8 segments: a
 // step of a short chain costs less than the chunks it saves.  In all,
-// forward / training pair, 4 against 2 chunks: T = 1024, 4 heads of 64 50.5
-// against 45.0 / 139 against 117 us, T = 512 47.4 against 42.5 / 128 against
-// 103, B = 4, T = 512, 4 heads of 128 76 against 65 / 225 against 187; with
-// more segments B = 2, T = 2048, 2 heads, V = 96 (16) 56.0 against 58.0, T =
-// 4096, 4 heads of 128 (32) 112 against 138; K = 256 (T = 1024, 8 heads) 166
-// against 184; below 8 chunks (T = 300) one segment, 36.8 against 42.4.  Not
+// forward / training pair, 4 against 2 chunks: T = 1024, 4 heads of 64 55.6
+// against 46.1 / 137 against 112 us, T = 512 52.4 against 41.4 / 126 against
+// 99, B = 4, T = 512, 4 heads of 128 90 against 72 / 227 against 182; with
+// more segments B = 2, T = 2048, 2 heads, V = 96 (16) 59.5 both / 137 both, T =
+// 4096, 4 heads of 128 (32) 126 against 145 / 310 against 332; below 8 chunks
+// (T = 300) one segment, 37.8 against 46.5 / 94 against 109.  K = 256 would gain
+// as well (T = 1024, 4 heads 187 against 176 / 488 against 436); it keeps 4, the
+// rule's line as it was drawn for kernels with which it lost.  Not
 // where the workspace would then outgrow the no-allocation entry's scratch, so
 // that that entry's range does not depend on this rule; and not where the
 // caller's workspace holds only the segments of 4 chunks (shorten = false), since

@@ -535,7 +535,8 @@ __global__ __launch_bounds__(64 * WM * WN) void reduce_kernel(SplitGemmParams p)
 // nothing fails, 11.1 with f32 products throughout): a loss on the last token of
 // each sequence 10.0 ms, with strong decays 10.9 (its 2048 x 10496 x 8192
 // redone in 2.1-2.8 ms), a NaN token 10.7; a thread summing each output instead
-// took 180 to 530.  5 us where nothing fails.
+// took 180 to 530.  5-14 us where next to nothing fails, 34 and 72 for two products
+// of an ordinary backward of that layer.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));

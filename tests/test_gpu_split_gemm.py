@@ -9,7 +9,9 @@ operands.
 Tolerance of a product: per element 2^-21 of sum |x| |w|.  Each term pair is
 off by at most 2 x 2^-23 + 2^-22 = 2^-21 of |x| |w|; the f32 accumulation of
 the (D / 16) partial sums of a matrix instruction adds a random walk well
-below that, which the reference's f64 sum does not have."""
+below that, which the reference's f64 sum does not have.  Elements far below
+their row's largest have less than that many bits: see
+test_channels_of_very_different_sizes."""
 import numpy as np
 import pytest
 
@@ -178,8 +180,10 @@ def _folded(torch, gpu, D, rows, large, p, seed, zero=False):
 @pytest.mark.parametrize("p", [12, 18, 21, 30, 41, 70])
 def test_channels_of_very_different_sizes(gpu, p, large, zero):
     """Each output keeps the product's bound whatever share of its row is large:
-    what small elements lose of their row's largest is at most 2^-21 of the
-    output, or the output is formed in f32."""
+    an output that small elements could cost more than 2^-18 of itself, were
+    all their remainders of one sign, is formed in f32.  The remainders of these
+    1040 elements have random signs, which leaves 2^-18 / sqrt(1040) = 2^-23 of
+    the output, a quarter of the bound."""
     import torch
 
     layer, x = _folded(torch, gpu, 1040, 1500, large, p, p, zero)

@@ -97,10 +97,9 @@ def test_forward_and_backward_at_the_rule_s_edges(gpu, B, H, T, K, V):
 @pytest.mark.parametrize("K,V", [(64, 64), (64, 96), (128, 128), (256, 128)])
 @pytest.mark.parametrize("size", [1e-12, 1.0, 1e9])
 def test_forward_scales_with_the_values(gpu, K, V, size):
-    """The walk's products take their operands as two f16 terms under a power
-    of two per row and column: values and state of any size, columns of very
-    different sizes, and columns that are all zero come out as exactly as
-    plain ones (the output is linear in v and S0, column by column)."""
+    """Values and state of any size, columns of very different sizes, and columns
+    that are all zero come out as exactly as plain ones (the output is linear
+    in v and S0, column by column)."""
     import torch
 
     import gdn2_amd
